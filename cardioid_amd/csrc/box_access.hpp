@@ -30,6 +30,21 @@ __device__ __forceinline__ double box_load(__amdgpu_buffer_rsrc_t r, uint32_t vo
    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
 
+// the same at agent scope (cache policy SC1, as a relaxed atomic load there
+// has it), for Vm that other wavefronts store while the kernel runs
+constexpr int kSC1 = 16;
+__device__ __forceinline__ double box_load_agent(__amdgpu_buffer_rsrc_t r, uint32_t voff,
+                                                 uint32_t soff)
+{
+   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kSC1));
+}
+__device__ __forceinline__ void box_store_agent(double v, __amdgpu_buffer_rsrc_t r, uint32_t voff,
+                                                uint32_t soff)
+{
+   typedef unsigned int u32x2 __attribute__((__vector_size__(2 * sizeof(unsigned int))));
+   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, kSC1);
+}
+
 // a raw buffer over a wave-uniform base address (offsets below 2^32 bytes)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_rsrc(const void *base)
 {

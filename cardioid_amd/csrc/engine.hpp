@@ -238,10 +238,15 @@ __device__ __forceinline__ int engine_tile_group(const EngineArgs &a)
 // the FP64 engine's reaction arithmetic (engine_f64.hip)
 enum EngineKind : int { kFits = 0, kFitsFma = 1, kExact = 2 };
 
+struct ResidentArgs;           // engine_resident.hpp
+
 // kernels (engine_f64.hip, engine_mixed.hip); WAVES = target waves per SIMD
 template <int WAVES, int KIND>
 __global__ void k_engine_f64(EngineArgs a);
 template <int WAVES>
 __global__ void k_engine_mixed(EngineArgs a);
+template <int KIND, int WAVES>
+__global__ void k_resident_f64(EngineArgs a, ResidentArgs r);
+__global__ void k_resident_mixed(EngineArgs a, ResidentArgs r);
 
 }  // namespace cdh

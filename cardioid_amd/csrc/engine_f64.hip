@@ -15,6 +15,7 @@
 #pragma clang fp contract(off)
 
 #include "engine.hpp"
+#include "engine_resident.hpp"
 #include "tt06_exact.hpp"
 
 namespace cdh {
@@ -80,7 +81,7 @@ __device__ __forceinline__ void cell_f64(const EngineArgs &a, const SlabDev &S, 
    double dVR = 0.0;
    if constexpr (KIND == kExact) {
       if (a.gate_mask & (1u << 12))
-         dVR = nongate_core64(*a.K, P, ExactVoltageFns{a.E, a.K}, a.dt, V, st);
+         dVR = nongate_core64(*a.K, P, exact_voltage_fns(a.E, a.K), a.dt, V, st);
       if (!((meta >> 8) & kFlagGatesFixed))
          gates_exact64(*a.E, P.s_switch, a.dt, V, st, a.gate_mask);
    } else {
@@ -149,5 +150,94 @@ template __global__ void k_engine_f64<2, kFitsFma>(EngineArgs);
 template __global__ void k_engine_f64<3, kFitsFma>(EngineArgs);
 template __global__ void k_engine_f64<2, kExact>(EngineArgs);
 template __global__ void k_engine_f64<3, kExact>(EngineArgs);
+
+// ---- resident form (engine_resident.hpp)
+
+namespace {
+
+// The 18 weights wait in LDS between the steps' stencils, the states in
+// registers.
+template <int KIND>
+struct ResidentF64 {
+   struct Shared {
+      float w[18][kBlk];
+   };
+   double st[N_STATE];
+   Shared *sh;
+   __amdgpu_buffer_rsrc_t RS;
+   uint32_t lc, rw;
+
+   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t, Shared *shared)
+   {
+      sh = shared;
+      const float *wp = a.Aw + (int64_t)t.blk * (18 * kBlk) + t.lane;
+#pragma unroll
+      for (int k = 0; k < 18; k++) sh->w[k][t.lane] = wp[kBlk * k];
+      rw = t.rw;
+      lc = t.lc;
+      RS = stream_rsrc(a.state + t.run_cell * N_STATE);
+#pragma unroll
+      for (int s = 0; s + 1 < N_STATE; s += 2)
+         stream_load_f64x2(RS, 16u * lc, 8u * rw * s, st[s], st[s + 1]);
+      st[N_STATE - 1] = stream_load_f64(RS, 8u * lc, 8u * rw * (N_STATE - 1));
+   }
+   __device__ __forceinline__ void store()
+   {
+#pragma unroll
+      for (int s = 0; s + 1 < N_STATE; s += 2)
+         stream_store_f64x2(st[s], st[s + 1], RS, 16u * lc, 8u * rw * s);
+      stream_store_f64(st[N_STATE - 1], RS, 8u * lc, 8u * rw * (N_STATE - 1));
+   }
+   __device__ __forceinline__ double react(const EngineArgs &a, const ModelTables &T,
+                                           const ParamSet &P, uint32_t meta, double V)
+   {
+      double dVR = 0.0;
+      if constexpr (KIND == kExact) {
+         if (a.gate_mask & (1u << 12))
+            dVR = nongate_core64<true>(*T.K, P, exact_voltage_fns(T.E, T.K), a.dt, V, st);
+         if (!((meta >> 8) & kFlagGatesFixed))
+            gates_exact64(*T.E, P.s_switch, a.dt, V, st, a.gate_mask);
+      } else {
+         constexpr bool FMA = KIND == kFitsFma;
+         if (a.gate_mask & (1u << 12)) dVR = nongate64<FMA, true>(*T.K, P, T.coef, a.dt, V, st);
+         gates64<FMA>(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(meta >> 8), V, st, a.gate_mask);
+      }
+      return dVR;
+   }
+   // the sums of cell_f64, in its order
+   __device__ __forceinline__ double diffuse(const ResidentTile &t, __amdgpu_buffer_rsrc_t R, double V,
+                                             double scale)
+   {
+      double nb[18];
+#pragma unroll
+      for (int k = 0; k < 18; k++) nb[k] = t.neighbour(R, k + 1);
+      __builtin_amdgcn_sched_barrier(0);   // all loads in flight before the first sum
+      double A0 = 0.0;
+#pragma unroll
+      for (int k = 0; k < 18; k++) A0 -= sh->w[k][t.lane];
+      double tmp = A0 * V;
+#pragma unroll
+      for (int k = 1; k < 19; k++) tmp += (double)sh->w[k - 1][t.lane] * nb[k - 1];
+      return tmp * scale;
+   }
+   __device__ __forceinline__ void finish(const EngineArgs &, const ModelTables &, double, double)
+   {
+   }
+};
+
+}  // namespace
+
+template <int KIND, int WAVES>
+__global__ __launch_bounds__(64, WAVES) void k_resident_f64(EngineArgs a, ResidentArgs r)
+{
+   __shared__ typename ResidentF64<KIND>::Shared sh;
+   resident_run<ResidentF64<KIND>>(a, r, &sh);
+}
+
+template __global__ void k_resident_f64<kFits, 3>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_f64<kFits, 4>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_f64<kFitsFma, 3>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_f64<kFitsFma, 4>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_f64<kExact, 3>(EngineArgs, ResidentArgs);
 
 }  // namespace cdh

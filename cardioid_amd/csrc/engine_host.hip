@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "engine_resident.hpp"
 #include "setup.hpp"
 #include "setup_device.hpp"
 
@@ -80,6 +81,92 @@ __global__ __launch_bounds__(256) void k_halo(int64_t n, const uint32_t *pairs, 
 {
    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
    if (i < n) box[pairs[2 * i]] = box[pairs[2 * i + 1]];
+}
+
+// The tiles that can hold neighbours of a tile's cells, for the resident
+// kernels: three ranges (the planes one step back in x, level, and one step
+// on), each {first, last + 1}.  A slab's cells are in box order, so the tiles
+// with cells in a range of box points are a range too, found by the tiles'
+// first box points; a range may hold a tile too many at its start.  Flags of
+// the live tiles start at `base`.
+__global__ __launch_bounds__(64) void k_tile_links(EngineArgs a, uint32_t *links, uint32_t *flags,
+                                                   uint32_t base)
+{
+   const int q = blockIdx.x * 64 + threadIdx.x;
+   const int j = q / 3, part = q % 3;
+   if (j >= a.ntile) return;
+   const int blk = a.tiles ? (int)a.tiles[j] : a.tile_base + j;
+   if (part == 0) flags[kFlagStride * j] = base;
+   uint32_t lo = 0, hi = 0;
+   const int sl = a.blk_slab[blk];
+   if (sl != kNoSlab) {
+      const SlabDev &S = a.slabs[sl];
+      int last = kBlk - 1;
+      while (last > 0 && (a.meta[(int64_t)blk * kBlk + last] & kMetaPad)) --last;
+      const int64_t plane = (int64_t)(S.soff[3] / 8) - kBoxShift;    // x + 1
+      const int64_t row = (int64_t)(S.soff[4] / 8) - kBoxShift;      // y + 1
+      const int64_t reach = part == 1 ? row + 1 : row;
+      const int64_t from = (int64_t)a.bi[(int64_t)blk * kBlk] + (part - 1) * plane - reach;
+      const int64_t to = (int64_t)a.bi[(int64_t)blk * kBlk + last] + (part - 1) * plane + reach;
+      // the number of the slab's tiles whose first box point is at most x
+      auto upto = [&](int64_t x) {
+         int n0 = 0, n1 = S.ntile;
+         while (n0 < n1) {
+            const int m = (n0 + n1) / 2;
+            if ((int64_t)a.bi[((int64_t)S.first_blk + m) * kBlk] <= x) n0 = m + 1;
+            else n1 = m;
+         }
+         return n0;
+      };
+      const int e = upto(to);
+      const int f = upto(from);
+      if (e > 0) {
+         // a slab's tiles stand together in the list
+         const int j0 = j - (blk - S.first_blk);
+         lo = (uint32_t)(j0 + (f > 0 ? f - 1 : 0));
+         hi = (uint32_t)(j0 + e);
+      }
+   }
+   links[6 * j + 2 * part] = lo;
+   links[6 * j + 2 * part + 1] = hi;
+}
+
+// The slabs' clocks after `nsteps` resident steps from parity p, as
+// slab_advance moves them step by step.
+__global__ __launch_bounds__(64) void k_slab_clock(SlabDev *slabs, int nslab, int p, int nsteps,
+                                                   double dt)
+{
+#pragma clang fp contract(off)
+   const int k = blockIdx.x * 64 + threadIdx.x;
+   if (k >= nslab || !slabs[k].active) return;
+   SlabDev &S = slabs[k];
+   const int q = (p + nsteps) & 1;
+   double t = S.time[p];
+   const int loop = S.loop[p] + nsteps;
+   for (int n = 0; n < nsteps; n++) t = t + dt;
+   S.time[q] = t;
+   S.loop[q] = loop;
+   uint32_t on;
+   double val[kSlabStim];
+   slab_stim_eval(S.stim, S.nstim, t, &on, val);
+   for (int n = 0; n < kSlabStim; n++) S.stim_val[q][n] = val[n];
+   S.stim_on[q] = on;
+}
+
+// The resident kernels of a mode, from the one with the fewest tiles on the
+// chip to the one with the most.  The FP64 kernel holds 3 wavefronts per SIMD
+// (3,072 tiles on 256 CUs) without spills; at 4 it spills some 12 registers,
+// which 64^3 cells repay (4,096 tiles: FMA 16.5 us a step against 24.5 by
+// step kernels, reference rounding 18.1 against 24.6) and fewer tiles do not
+// (54x56x64 cells: 13.0 us a step against 11.6 at 3).  The exact functions
+// spill too much at 4 (39 against 32 us at 64^3 by step kernels).
+using ResidentFn = void (*)(EngineArgs, ResidentArgs);
+std::vector<ResidentFn> resident_kernels(int mode, bool exact)
+{
+   if (mode == CDH_MODE_MIXED_FUSED) return {k_resident_mixed};
+   if (exact) return {k_resident_f64<kExact, 3>};
+   if (mode == CDH_MODE_FP64_FMA) return {k_resident_f64<kFitsFma, 3>, k_resident_f64<kFitsFma, 4>};
+   return {k_resident_f64<kFits, 3>, k_resident_f64<kFits, 4>};
 }
 
 using KernelFn = void (*)(EngineArgs);
@@ -294,6 +381,7 @@ void Engine::refresh_tiles()
    tile_base_ = list.empty() ? 0 : (int64_t)list.front();
    if (!tiles_direct_) put(tile_list_.p, list);
    list_dirty_ = false;
+   links_dirty_ = true;
 }
 
 void Engine::retire_staging()
@@ -364,6 +452,19 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
    track(bi_, S);
    track(blk_slab_, ntile);
    track(tile_list_, ntile);
+   CDH_HIP(hipHostMalloc((void **)&failed_, sizeof(uint32_t), hipHostMallocDefault));
+   *failed_ = 0;
+   int ncu = 0, coop = 0;
+   CDH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+   CDH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+   for (ResidentFn fn : resident_kernels(mode, exact_ != 0)) {
+      int per_cu = 0;
+      CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlk, 0));
+      resident_cap_.push_back(coop ? (int64_t)ncu * per_cu : 0);
+      resident_tiles_ = std::max(resident_tiles_, resident_cap_.back());
+   }
+   track(links_tile_, 6 * (size_t)resident_tiles_);
+   track(flags_, kFlagStride * (size_t)resident_tiles_);
    CDH_HIP(hipMemset(blk_slab_.p, 0xFF, ntile * sizeof(uint16_t)));
    track(slabdev_, cap_slabs);
    slabdev_.zero();
@@ -400,6 +501,7 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
 Engine::~Engine()
 {
    if (stream_) (void)hipStreamSynchronize(stream_);
+   if (failed_) (void)hipHostFree(failed_);
    if (graph_) (void)hipGraphExecDestroy(graph_);
    if (ev0_) (void)hipEventDestroy(ev0_);
    if (ev1_) (void)hipEventDestroy(ev1_);
@@ -740,6 +842,8 @@ void Engine::set_graph_steps(int k)
    drop_graph();
 }
 
+// A launch chosen by the caller is the step kernel's: it is launched step by
+// step as told, or replayed in graphs.
 void Engine::set_launch(const LaunchCfg &c)
 {
    CDH_REQUIRE(c.waves >= min_waves(mode_) && c.waves <= max_waves(mode_),
@@ -749,7 +853,67 @@ void Engine::set_launch(const LaunchCfg &c)
    CDH_REQUIRE(c.occ >= 0 && c.occ <= 8, "engine: occupancy cap must be 0..8");
    CDH_REQUIRE(c.xcd >= -1 && c.xcd <= 10, "engine: tile order must be -1 or 0..10");
    cfg_ = c;
+   resident_ = false;
    drop_graph();
+}
+
+// Whether the live tiles all fit on the chip at once, and nothing but the
+// step itself has to happen between two steps.
+bool Engine::resident_fits() const
+{
+   return resident_ && nlist_ > 0 && nhalo_ == 0 && (nlist_ + 7) / 8 * 8 <= resident_tiles_;
+}
+
+// Up to nsteps of every live slab by the resident kernel, at most
+// kResidentSteps in one launch; returns the steps that are left to the step
+// kernels, where the device would not take a cooperative launch.
+int Engine::run_resident(int nsteps)
+{
+   if (links_dirty_) {
+      const EngineArgs a = args(parity_);
+      hipLaunchKernelGGL(k_tile_links, dim3((unsigned)((3 * nlist_ + 63) / 64)), dim3(64), 0,
+                         stream_, a, links_tile_.p, flags_.p, epoch_);
+      CDH_LAUNCH_CHECK();
+      links_dirty_ = false;
+   }
+   const std::vector<ResidentFn> fns = resident_kernels(mode_, exact_ != 0);
+   size_t which = 0;
+   while (resident_cap_[which] < (nlist_ + 7) / 8 * 8) ++which;     // resident_fits()
+   const ResidentFn fn = fns[which];
+   while (nsteps > 0) {
+      const int n = std::min(nsteps, kResidentSteps);
+      EngineArgs a = args(parity_);
+      a.xcd_chunk_log2 = -1;
+      a.groups_per_xcd = (a.ntile + 7) / 8;
+      ResidentArgs r{};
+      r.flags = flags_.p;
+      r.links = links_tile_.p;
+      r.base = epoch_;
+      r.nsteps = n;
+      r.box[0] = box_[parity_].p;
+      r.box[1] = box_[parity_ ^ 1].p;
+      r.failed = failed_;
+      void *kargs[2] = {&a, &r};
+      if (hipLaunchCooperativeKernel((const void *)fn, dim3(8 * a.groups_per_xcd), dim3(kBlk),
+                                     kargs, 0, stream_) != hipSuccess) {
+         (void)hipGetLastError();
+         resident_ = false;
+         return nsteps;
+      }
+      hipLaunchKernelGGL(k_slab_clock, dim3((unsigned)((slabs_.size() + 63) / 64)), dim3(64), 0,
+                         stream_, slabdev_.p, (int)slabs_.size(), parity_, n, dt_);
+      CDH_LAUNCH_CHECK();
+      epoch_ += (uint32_t)n;
+      parity_ ^= n & 1;
+      for (Slab &s : slabs_)
+         if (s.live)
+            for (int k = 0; k < n; k++) {
+               s.time = s.time + dt_;
+               ++s.loop;
+            }
+      nsteps -= n;
+   }
+   return 0;
 }
 
 void Engine::run(int nsteps)
@@ -757,6 +921,7 @@ void Engine::run(int nsteps)
    CDH_REQUIRE(nsteps >= 0, "engine: negative step count");
    retire_staging();
    refresh_tiles();      // before any capture: an upload must not land in a graph
+   if (nsteps >= kResidentMin && resident_fits()) nsteps = run_resident(nsteps);
    while (nsteps > 0) {
       if (graph_steps_ > 0 && parity_ == 0 && nsteps >= graph_steps_) {
          if (!graph_ || graph_ntile_ != (int)nlist_ || graph_direct_ != tiles_direct_ ||
@@ -794,6 +959,9 @@ double Engine::run_timed(int nsteps)
 void Engine::sync()
 {
    CDH_HIP(hipStreamSynchronize(stream_));
+   if (failed_ && *(volatile uint32_t *)failed_)
+      throw Error(kErrHip, "engine: a resident tile waited past its bound for a neighbour; the "
+                           "states are not valid");
    retire_staging();
 }
 
@@ -856,8 +1024,23 @@ double Engine::autotune(int steps, std::vector<std::pair<LaunchCfg, double>> *ta
          bestc = cand[c];
       }
    }
-   CDH_HIP(hipStreamSynchronize(stream_));
+   // the resident form in the same way, over enough steps that its launch
+   // weighs as it does in a run
    set_launch(bestc);
+   resident_ = true;
+   refresh_tiles();
+   if (resident_fits()) {
+      const int n = std::max(steps, kResidentSteps);
+      const double t = run_timed(n) / n;
+      resident_ = t < best;
+      best = std::min(best, t);
+      for (size_t k = 0; k < regions.size(); k++)
+         CDH_HIP(hipMemcpyAsync(regions[k].first, saved[k]->p, regions[k].second,
+                                hipMemcpyDeviceToDevice, stream_));
+      parity_ = par0;
+      slabs_ = host0;
+   }
+   CDH_HIP(hipStreamSynchronize(stream_));
    graph_steps_ = gsteps;
    return best;
 }

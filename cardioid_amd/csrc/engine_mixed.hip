@@ -13,6 +13,7 @@
 #include <hip/hip_fp16.h>
 
 #include "engine.hpp"
+#include "engine_resident.hpp"
 #include "tt06_mixed.hpp"
 
 namespace cdh {
@@ -161,5 +162,92 @@ __global__ __launch_bounds__(256, WAVES) void k_engine_mixed(EngineArgs a)
 
 template __global__ void k_engine_mixed<3>(EngineArgs);
 template __global__ void k_engine_mixed<4>(EngineArgs);
+
+// ---- resident form (engine_resident.hpp)
+
+namespace {
+
+struct ResidentMixed {
+   struct Shared {};
+   float s32[N_STATE32];
+   double s64[N_STATE64];
+   uint32_t hw[9];
+   __amdgpu_buffer_rsrc_t R32, R64;
+   const float CDH_CONSTANT *ref;
+   float wscale;
+   uint32_t lc, rw;
+   double iK;
+
+   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t, Shared *)
+   {
+      rw = t.rw;
+      lc = t.lc;
+      R32 = stream_rsrc(a.st32 + t.run_cell * N_STATE32);
+      R64 = stream_rsrc(a.st64 + t.run_cell * N_STATE64);
+#pragma unroll
+      for (int s = 0; s < N_STATE32; s++) s32[s] = stream_load_f32(R32, 4u * lc, 4u * rw * s);
+#pragma unroll
+      for (int s = 0; s < N_STATE64; s++) s64[s] = stream_load_f64(R64, 8u * lc, 8u * rw * s);
+      const uint32_t *wp = a.Aw16 + (int64_t)t.blk * (9 * kBlk);
+#pragma unroll
+      for (int g = 0; g < 2; g++) {
+         const u32x4 q = *((const u32x4 *)(wp + g * 4 * kBlk) + t.lane);
+         hw[4 * g] = q.x;
+         hw[4 * g + 1] = q.y;
+         hw[4 * g + 2] = q.z;
+         hw[4 * g + 3] = q.w;
+      }
+      hw[8] = wp[8 * kBlk + t.lane];
+      ref = (const float CDH_CONSTANT *)(a.Aref + (int64_t)t.blk * 18);
+      wscale = t.S->wdelta_scale;
+   }
+   __device__ __forceinline__ void store()
+   {
+#pragma unroll
+      for (int s = 0; s < N_STATE32; s++) stream_store_f32(s32[s], R32, 4u * lc, 4u * rw * s);
+#pragma unroll
+      for (int s = 0; s < N_STATE64; s++) stream_store_f64(s64[s], R64, 8u * lc, 8u * rw * s);
+   }
+   __device__ __forceinline__ double react(const EngineArgs &a, const ModelTables &T,
+                                           const ParamSet &P, uint32_t meta, double V)
+   {
+      const double K_i = P.K0 + (double)s32[M_DK_I];
+      double dVR = 0.0;
+      iK = 0.0;
+      if (a.gate_mask & (1u << 12)) dVR = nongateM(*T.K, P, T.coef, a.dt, V, K_i, s32, s64, &iK);
+      gatesM(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(meta >> 8), V, s32, a.gate_mask);
+      return dVR;
+   }
+   // the sums of cell_mixed, in its order
+   __device__ __forceinline__ double diffuse(const ResidentTile &t, __amdgpu_buffer_rsrc_t R, double V,
+                                             double scale)
+   {
+      double nb[18];
+#pragma unroll
+      for (int k = 0; k < 18; k++) nb[k] = t.neighbour(R, k + 1);
+      __builtin_amdgcn_sched_barrier(0);   // all loads in flight before the first sum
+      float acc = 0.0f;
+#pragma unroll
+      for (int p = 0; p < 9; p++) {
+         const float w0 = half_lo_plus(hw[p], ref[2 * p]);
+         const float w1 = half_hi_plus(hw[p], ref[2 * p + 1]);
+         acc = __builtin_fmaf(w0, (float)(nb[2 * p] - V), acc);
+         acc = __builtin_fmaf(w1, (float)(nb[2 * p + 1] - V), acc);
+      }
+      return (double)acc * (scale * (double)wscale);
+   }
+   __device__ __forceinline__ void finish(const EngineArgs &a, const ModelTables &T, double dVD,
+                                          double iStim)
+   {
+      s32[M_DK_I] = (float)((double)s32[M_DK_I] + (a.dt * T.K->c9) * (iK - dVD - iStim));
+   }
+};
+
+}  // namespace
+
+__global__ __launch_bounds__(64, 4) void k_resident_mixed(EngineArgs a, ResidentArgs r)
+{
+   resident_run<ResidentMixed>(a, r, nullptr);
+}
 
 }  // namespace cdh

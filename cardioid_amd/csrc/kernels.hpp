@@ -96,9 +96,10 @@ __device__ __forceinline__ void sensor_count(uint32_t *counts, uint32_t per_lane
 }
 
 // per-lane packing of one cell's events for sensor_count
+constexpr uint32_t kEvTactPacked = 1u << 8;
 __device__ __forceinline__ uint32_t sensor_events_packed(unsigned ev)
 {
-   return ((ev & kEvTact0) ? 1u : 0u) | ((ev & kEvTact) ? 1u << 8 : 0u) |
+   return ((ev & kEvTact0) ? 1u : 0u) | ((ev & kEvTact) ? kEvTactPacked : 0u) |
           ((ev & kEvTrec) ? 1u << 16 : 0u);
 }
 

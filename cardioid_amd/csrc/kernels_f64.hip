@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void k_tt06_calc_exact_f64(ReactionArgs a)
    for (int s = 0; s < N_STATE; s++) st[s] = a.state[blk_index(s, i, N_STATE)];
    const ParamSet P = a.params[0];
    double dVR = 0.0;
-   if (a.gate_mask & (1u << 12)) dVR = nongate_core64(*a.K, P, ExactVoltageFns{a.E, a.K}, a.dt, V, st);
+   if (a.gate_mask & (1u << 12)) dVR = nongate_core64(*a.K, P, exact_voltage_fns(a.E, a.K), a.dt, V, st);
    if (!(a.flags[i] & kFlagGatesFixed)) gates_exact64(*a.E, P.s_switch, a.dt, V, st, a.gate_mask);
 #pragma unroll
    for (int s = 0; s < N_STATE; s++) a.state[blk_index(s, i, N_STATE)] = st[s];

@@ -284,7 +284,8 @@ int cdh_sim_create(const cdh_sim_params *p, int nstim, const cdh_box_stim *stim,
             LaunchCfg c;
             c.waves = p->variant ? p->variant : 3;
             c.block = 64;
-            s->eng->set_launch(c);
+            if (p->variant) s->eng->set_launch(c);
+            else s->eng->set_default_launch(c);
             s->slab = s->eng->add(h);
             CDH_REQUIRE(s->slab >= 0, "cdh_sim_create: engine arena too small (internal)");
             s->eng->sync();

@@ -119,7 +119,8 @@ __device__ __forceinline__ double sTauR1(double V)
 
 // TauRecipMod with the host's cubic {x0, x1, c0..c3}: the cubic inside
 // [x0, x1], the raw rate outside (elec/TT06Tau.cc:131-151)
-__device__ __forceinline__ double smoothed(const double *h, double V, double raw)
+template <class C>
+__device__ __forceinline__ double smoothed(C h, double V, double raw)
 {
    if (V < h[0] || V > h[1]) return raw;
    const double x = V - h[0];
@@ -129,9 +130,10 @@ __device__ __forceinline__ double smoothed(const double *h, double V, double raw
 }  // namespace exact
 
 // fv0..fv6 exactly (elec/TT06NonGates.c:319-364)
+template <class ET, class KT>
 struct ExactVoltageFns {
-   const TT06ExactConst *__restrict__ E;
-   const TT06Const *__restrict__ K;
+   ET *E;
+   KT *K;
    __device__ __forceinline__ void fv05(double V, double fv[6]) const
    {
       const double f1 = E->f1;
@@ -169,11 +171,18 @@ struct ExactVoltageFns {
    }
 };
 
+template <class ET, class KT>
+__device__ __forceinline__ ExactVoltageFns<ET, KT> exact_voltage_fns(ET *E, KT *K)
+{
+   return ExactVoltageFns<ET, KT>{E, K};
+}
+
 // TT06Func::updateGate (elec/TT06Func.cc:64-161) with the exact functions:
 // every cell, m by Rush-Larsen, the others by g += dt*(mhu - g)*tauR.
 // `gmask` (every bit set) puts each gate in a basic block of its own, as in
 // gates64.
-__device__ __forceinline__ void gates_exact64(const TT06ExactConst &E, int s_switch, double dt,
+template <class ET>
+__device__ __forceinline__ void gates_exact64(const ET &E, int s_switch, double dt,
                                               double V, double *st, uint32_t gmask)
 {
    using namespace exact;

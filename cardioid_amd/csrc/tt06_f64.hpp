@@ -79,12 +79,12 @@ __device__ __forceinline__ double horner64(P a, double x)
 }
 
 // rational fit i of the fixed layout (pade.cc:17-36: num/den, polynomial if l < 2)
-template <int I, bool FMA = false>
-__device__ __forceinline__ double fit64(const double *__restrict__ coef, double x)
+template <int I, bool FMA = false, class C>
+__device__ __forceinline__ double fit64(C coef, double x)
 {
    constexpr int off = fit_offset(I);
    constexpr int l = kFitOrder[I].l, m = kFitOrder[I].m;
-   const double *__restrict__ c = coef + off;
+   const C c = coef + off;
    const double num = horner64<0, m - 1, FMA>(c, x);
    if constexpr (l < 2) {
       return num;
@@ -97,9 +97,8 @@ __device__ __forceinline__ double fit64(const double *__restrict__ coef, double 
 enum GateForm { G_RL, G_DIF, G_SUM };
 
 // one gate: mhu and dt/tau from fits 7+2*eq and 8+2*eq, then the v2 update
-template <int EQ, GateForm FORM, bool FMA = false>
-__device__ __forceinline__ double gate64(const double *__restrict__ coef, const double *__restrict__ expc,
-                                         double V, double g, bool sub_form)
+template <int EQ, GateForm FORM, bool FMA = false, class C>
+__device__ __forceinline__ double gate64(C coef, C expc, double V, double g, bool sub_form)
 {
    const double mhu = fit64<7 + 2 * EQ, FMA>(coef, V);
    const double x = fit64<8 + 2 * EQ, FMA>(coef, V);
@@ -121,9 +120,9 @@ __device__ __forceinline__ double gate64(const double *__restrict__ coef, const 
 // fv6General, elec/TT06Func.cc:614-629) from the dt-independent rational
 // fits 0..6 (configuration B).  The exact functions of configuration A are
 // the other implementation of the same two calls (tt06_exact.hpp).
-template <bool FMA>
+template <bool FMA, class C>
 struct FitVoltageFns {
-   const double *__restrict__ coef;
+   C coef;
    __device__ __forceinline__ void fv05(double Vm, double fv[6]) const
    {
       fv[0] = fit64<0, FMA>(coef, Vm);
@@ -136,32 +135,41 @@ struct FitVoltageFns {
    __device__ __forceinline__ double fv6(double dV0) const { return fit64<6, FMA>(coef, dV0); }
 };
 
-// Non-gate update of one cell (update_nonGate, elec/TT06NonGates.c:374-563);
-// returns dVdt = -Iion and updates the seven concentration-like states in
-// st[].  Gates are read, not written.  FV supplies fv0..fv6.
-template <class FV>
-__device__ __forceinline__ double nongate_core64(const TT06Const &K, const ParamSet &P,
-                                                 const FV &fvs, double dt, double Vm, double *st)
+template <bool FMA, class C>
+__device__ __forceinline__ FitVoltageFns<FMA, C> fit_voltage_fns(C coef)
 {
-   double fvv[6];
-   fvs.fv05(Vm, fvv);
-   const double fv0 = fvv[0], fv1 = fvv[1], fv2 = fvv[2], fv3 = fvv[3], fv4 = fvv[4];
-   const double fv5 = fvv[5];
-   const double Na_i = st[S_NA_I], Ca_i = st[S_CA_I], Ca_ss = st[S_CA_SS], Ca_SR = st[S_CA_SR];
-   const double fCass = st[S_FCASS], R_prime = st[S_R_PRIME];
-   double dVK_i = st[S_DVK_I];
-   const double c_K1 = 1, c_bNa = 1 * K.c21, c_bCa = 1 * K.c7, c_NaCa = 1, c_pCa = 1 * K.c24;
-   const double c_pK = 1;
-   const double c_NaK = 1 * P.P_NaK, c_Ks = 1 * P.g_Ks, c_to = 1 * P.g_to, c_NaL = 1 * P.g_NaL;
+   return FitVoltageFns<FMA, C>{coef};
+}
 
-   double dVR = 0.0;
-   // calcium
+// Non-gate update of one cell (update_nonGate, elec/TT06NonGates.c:374-563)
+// in the parts that can run apart: the sodium-calcium exchanger, which both
+// others need; the calcium part, which updates Ca_i, Ca_ss, Ca_SR, R' and
+// fCass and gives the two currents that enter dVdt; the potassium and sodium
+// currents; and the sums.  Gates are read, not written.
+
+__device__ __forceinline__ double exchanger64(double Na_i, double Ca_i, double fv1, double fv2)
+{
+   const double c_NaCa = 1;
+   return c_NaCa * ((Na_i * Na_i * Na_i) * fv1 - Ca_i * fv2);
+}
+
+struct CalciumCurrents {
+   double I_sum, I_CaL;
+};
+
+template <class KT>
+__device__ __forceinline__ CalciumCurrents nongate_calcium64(const KT &K, const ParamSet &P,
+                                                             double dt, double Vm, double fv3,
+                                                             double fv4, double I_NaCa, double *st)
+{
+   const double Ca_i = st[S_CA_I], Ca_ss = st[S_CA_SS], Ca_SR = st[S_CA_SR];
+   const double fCass = st[S_FCASS], R_prime = st[S_R_PRIME];
+   const double c_bCa = 1 * K.c7, c_pCa = 1 * K.c24;
    const double x1 = Ca_i * K.c26;
    const double x2 = (Ca_i * K.c27) * (Ca_i * K.c27);
    const double x3 = (Ca_i * K.c28 + K.c29) * (Ca_i * K.c28 + K.c29);
    const double sg1 = CDH_SIGM(x1), sg2 = CDH_SIGM(x2), sg3 = CDH_SIGM(x3);
    const double dV3 = Vm - 0.5 * K.c3 * log(Ca_i) - K.c8;
-   const double I_NaCa = c_NaCa * ((Na_i * Na_i * Na_i) * fv1 - Ca_i * fv2);
    const double I_bCa = c_bCa * dV3;
    const double I_pCa = c_pCa * sg1;
    const double I_up = K.c44 * sg2;
@@ -170,31 +178,6 @@ __device__ __forceinline__ double nongate_core64(const TT06Const &K, const Param
    const double I_delta = I_leak - I_up;
    const double I_sum = I_bCa + I_pCa;
    st[S_CA_I] = Ca_i + (dt * K.c9) * (sg3 * (0.5 * I_sum - I_NaCa + I_xfer * K.c15 + I_delta * K.c16));
-   dVR -= I_sum;
-
-   // potassium and sodium
-   const double K_i = K.c9 * (dVK_i - Vm);
-   const double x0 = Na_i * K.c25;
-   const double dV0 = Vm - K.c3 * log(K_i) - K.c5;
-   const double dV1 = Vm - K.c3 * log(Na_i) - K.c4;
-   const double dV2 = dV0 - K.c3 * log(1 + K.c2 * Na_i / K_i) + K.c5 - K.c6;
-   const double fv6 = fvs.fv6(dV0);
-   const double m = st[S_M], h = st[S_H], j = st[S_J];
-   const double I_NaK = c_NaK * CDH_SIGM(x0) * fv0;
-   const double I_pK = c_pK * fv5 * dV0;
-   const double I_K1 = c_K1 * fv6 * dV0;
-   const double I_to = c_to * st[S_R] * st[S_S] * dV0;
-   const double I_Kr = P.c_Kr * st[S_XR1] * st[S_XR2] * dV0;
-   const double I_Na = P.c_Na * (m * m * m) * h * j * dV1;
-   const double I_NaL = c_NaL * (m * m * m) * st[S_JL] * dV1;
-   const double I_bNa = c_bNa * dV1;
-   const double I_Ks = c_Ks * (st[S_XS] * st[S_XS]) * dV2;
-   const double iNa = 3 * I_NaCa - 1.5 * I_NaK + I_Na + I_bNa + I_NaL;
-   const double iK = I_Ks + I_NaK + I_pK + I_K1 + I_to + I_Kr;
-   dVK_i += dt * iK;
-   dVR -= iNa + iK - 2.0 * I_NaCa;
-   st[S_NA_I] = Na_i + (dt * K.c9) * iNa;
-
    // Ca_ss, Ca_SR, R', fCass
    const double x4 = (Ca_SR * K.c30) * (Ca_SR * K.c30);
    const double x5 = (Ca_SR * K.c31 + K.c32) * (Ca_SR * K.c31 + K.c32);
@@ -212,18 +195,81 @@ __device__ __forceinline__ double nongate_core64(const TT06Const &K, const Param
    const double mhu = 0.600000 * t1 + 0.4000000;
    const double tauR = 1.0 / (80.0 * t1 + 2.0);
    st[S_FCASS] = fCass + dt * (mhu - fCass) * tauR;
-   dVR += I_CaL;
+   return CalciumCurrents{I_sum, I_CaL};
+}
+
+struct SodiumPotassiumCurrents {
+   double iNa, iK;
+};
+
+template <class KT, class FV>
+__device__ __forceinline__ SodiumPotassiumCurrents
+nongate_na_k64(const KT &K, const ParamSet &P, const FV &fvs, double Vm, double fv0,
+               double fv5, double I_NaCa, const double *st)
+{
+   const double c_K1 = 1, c_bNa = 1 * K.c21, c_pK = 1;
+   const double c_NaK = 1 * P.P_NaK, c_Ks = 1 * P.g_Ks, c_to = 1 * P.g_to, c_NaL = 1 * P.g_NaL;
+   const double Na_i = st[S_NA_I];
+   const double K_i = K.c9 * (st[S_DVK_I] - Vm);
+   const double x0 = Na_i * K.c25;
+   const double dV0 = Vm - K.c3 * log(K_i) - K.c5;
+   const double dV1 = Vm - K.c3 * log(Na_i) - K.c4;
+   const double dV2 = dV0 - K.c3 * log(1 + K.c2 * Na_i / K_i) + K.c5 - K.c6;
+   const double fv6 = fvs.fv6(dV0);
+   const double m = st[S_M], h = st[S_H], j = st[S_J];
+   const double I_NaK = c_NaK * CDH_SIGM(x0) * fv0;
+   const double I_pK = c_pK * fv5 * dV0;
+   const double I_K1 = c_K1 * fv6 * dV0;
+   const double I_to = c_to * st[S_R] * st[S_S] * dV0;
+   const double I_Kr = P.c_Kr * st[S_XR1] * st[S_XR2] * dV0;
+   const double I_Na = P.c_Na * (m * m * m) * h * j * dV1;
+   const double I_NaL = c_NaL * (m * m * m) * st[S_JL] * dV1;
+   const double I_bNa = c_bNa * dV1;
+   const double I_Ks = c_Ks * (st[S_XS] * st[S_XS]) * dV2;
+   return SodiumPotassiumCurrents{3 * I_NaCa - 1.5 * I_NaK + I_Na + I_bNa + I_NaL,
+                                  I_Ks + I_NaK + I_pK + I_K1 + I_to + I_Kr};
+}
+
+// dVdt = -Iion from the parts, and the Na_i and dVK_i updates
+template <class KT>
+__device__ __forceinline__ double nongate_sum64(const KT &K, double dt, double I_NaCa,
+                                                const CalciumCurrents &ca,
+                                                const SodiumPotassiumCurrents &nk, double *st)
+{
+   double dVR = 0.0;
+   dVR -= ca.I_sum;
+   const double dVK_i = st[S_DVK_I] + dt * nk.iK;
+   dVR -= nk.iNa + nk.iK - 2.0 * I_NaCa;
+   st[S_NA_I] = st[S_NA_I] + (dt * K.c9) * nk.iNa;
+   dVR += ca.I_CaL;
    st[S_DVK_I] = dVK_i + dt * dVR;
    return dVR;
 }
 
-// configuration B: the fits (FMA applies to the fit polynomials only)
-template <bool FMA = false>
-__device__ __forceinline__ double nongate64(const TT06Const &K, const ParamSet &P,
-                                           const double *__restrict__ coef, double dt, double Vm,
-                                           double *st)
+// The whole of it; returns dVdt and updates the seven concentration-like
+// states in st[].  FV supplies fv0..fv6.  APART keeps the compiler from
+// interleaving the parts, for kernels short of registers.
+template <bool APART = false, class KT, class FV>
+__device__ __forceinline__ double nongate_core64(const KT &K, const ParamSet &P,
+                                                 const FV &fvs, double dt, double Vm, double *st)
 {
-   return nongate_core64(K, P, FitVoltageFns<FMA>{coef}, dt, Vm, st);
+   double fv[6];
+   fvs.fv05(Vm, fv);
+   const double I_NaCa = exchanger64(st[S_NA_I], st[S_CA_I], fv[1], fv[2]);
+   if constexpr (APART) __builtin_amdgcn_sched_barrier(0);
+   const CalciumCurrents ca = nongate_calcium64(K, P, dt, Vm, fv[3], fv[4], I_NaCa, st);
+   if constexpr (APART) __builtin_amdgcn_sched_barrier(0);
+   const SodiumPotassiumCurrents nk = nongate_na_k64(K, P, fvs, Vm, fv[0], fv[5], I_NaCa, st);
+   if constexpr (APART) __builtin_amdgcn_sched_barrier(0);
+   return nongate_sum64(K, dt, I_NaCa, ca, nk, st);
+}
+
+// configuration B: the fits (FMA applies to the fit polynomials only)
+template <bool FMA = false, bool APART = false, class KT, class C>
+__device__ __forceinline__ double nongate64(const KT &K, const ParamSet &P, C coef, double dt,
+                                           double Vm, double *st)
+{
+   return nongate_core64<APART>(K, P, fit_voltage_fns<FMA>(coef), dt, Vm, st);
 }
 
 // The 12 gate updates at voltage Vm (the voltage of the step's start).
@@ -232,9 +278,8 @@ __device__ __forceinline__ double nongate64(const TT06Const &K, const ParamSet &
 // each gate in a basic block of its own, which keeps the compiler from
 // issuing the scalar loads of all 26 gate fits ahead of time (they would
 // not fit in SGPRs and get spilled to VGPR lanes).
-template <bool FMA = false>
-__device__ __forceinline__ void gates64(const double *__restrict__ coef, const double *__restrict__ expc,
-                                        int s_switch, uint8_t flags, double Vm, double *st,
+template <bool FMA = false, class C>
+__device__ __forceinline__ void gates64(C coef, C expc, int s_switch, uint8_t flags, double Vm, double *st,
                                         uint32_t gmask)
 {
    if (flags & kFlagGatesFixed) return;

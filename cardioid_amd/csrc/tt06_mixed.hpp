@@ -31,8 +31,8 @@ enum Slot32 : int {
 enum Slot64 : int { M_CA_I = 0, M_NA_I, N_STATE64 };
 
 // Horner with fused multiply-adds (tt06_f64.hpp)
-template <int LO, int HI>
-__device__ __forceinline__ double hornerFma(const double *__restrict__ a, double x)
+template <int LO, int HI, class C>
+__device__ __forceinline__ double hornerFma(C a, double x)
 {
    return horner64<LO, HI, true>(a, x);
 }
@@ -48,8 +48,8 @@ __device__ __forceinline__ double ratio(double num, double den)
 }
 __device__ __forceinline__ double log32(double x) { return (double)__logf((float)x); }
 
-template <int I>
-__device__ __forceinline__ double fitM(const double *__restrict__ coef, double x)
+template <int I, class C>
+__device__ __forceinline__ double fitM(C coef, double x)
 {
    constexpr int off = fit_offset(I);
    constexpr int l = kFitOrder[I].l, m = kFitOrder[I].m;
@@ -63,9 +63,8 @@ __device__ __forceinline__ double fitM(const double *__restrict__ coef, double x
 
 // one gate: g + r*(mhu - g); r = 1 - 1/T16(x) for m (Rush-Larsen with the
 // reference's degree-16 series), r = dt/tau for the rest
-template <int EQ, bool RL>
-__device__ __forceinline__ float gateM(const double *__restrict__ coef, const double *__restrict__ expc,
-                                       double V, float g)
+template <int EQ, bool RL, class C>
+__device__ __forceinline__ float gateM(C coef, C expc, double V, float g)
 {
    const float mhu = (float)fitM<7 + 2 * EQ>(coef, V);
    const double x = fitM<8 + 2 * EQ>(coef, V);
@@ -85,9 +84,9 @@ __device__ __forceinline__ double sigmM(double x) { return ratio(x, 1.0 + x); }
 // cell type.  Returns dVdt = -Iion and the potassium current iK (the
 // caller finishes the K_i update, which needs the step's diffusion and
 // stimulus currents).
-__device__ __forceinline__ double nongateM(const TT06Const &K, const ParamSet &P,
-                                           const double *__restrict__ coef, double dt, double Vm,
-                                           const double K_i, float *s32, double *s64, double *iK_out)
+template <class KT, class C>
+__device__ __forceinline__ double nongateM(const KT &K, const ParamSet &P, C coef, double dt,
+                                           double Vm, const double K_i, float *s32, double *s64, double *iK_out)
 {
    const double fv0 = fitM<0>(coef, Vm), fv1 = fitM<1>(coef, Vm), fv2 = fitM<2>(coef, Vm);
    const double fv3 = fitM<3>(coef, Vm), fv4 = fitM<4>(coef, Vm), fv5 = fitM<5>(coef, Vm);
@@ -161,9 +160,9 @@ __device__ __forceinline__ double nongateM(const TT06Const &K, const ParamSet &P
    return dVR;
 }
 
-__device__ __forceinline__ void gatesM(const double *__restrict__ coef, const double *__restrict__ expc,
-                                       int s_switch, uint8_t flags, double Vm, float *s32,
-                                       uint32_t gmask)
+template <class C>
+__device__ __forceinline__ void gatesM(C coef, C expc, int s_switch, uint8_t flags, double Vm,
+                                       float *s32, uint32_t gmask)
 {
    if (flags & kFlagGatesFixed) return;
    if (gmask & (1u << 0)) s32[M_M] = gateM<0, true>(coef, expc, Vm, s32[M_M]);

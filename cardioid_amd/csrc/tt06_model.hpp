@@ -45,6 +45,22 @@ struct TT06ExactConst {
    int pad_;
 };
 
+// The model's tables as the kernels read them: pointers to the constant
+// address space, whose loads at wave-uniform addresses are always scalar.
+// Through plain pointers the compiler makes them vector loads, which wait
+// for every outstanding access, wherever it cannot show that no store came
+// before (a kernel with a barrier or stores between its reads).
+#define CDH_CONSTANT __attribute__((address_space(4)))
+typedef const double CDH_CONSTANT *CoefPtr;
+typedef const TT06Const CDH_CONSTANT ModelConst;
+typedef const TT06ExactConst CDH_CONSTANT ExactConst;
+__device__ __forceinline__ CoefPtr constant_ptr(const double *p) { return (CoefPtr)p; }
+__device__ __forceinline__ ModelConst *constant_ptr(const TT06Const *p) { return (ModelConst *)p; }
+__device__ __forceinline__ ExactConst *constant_ptr(const TT06ExactConst *p)
+{
+   return (ExactConst *)p;
+}
+
 // Fit orders (l, m) in fit order; the kernels are specialised on them.
 struct FitOrder { int l, m; };
 constexpr FitOrder kFitOrder[33] = {

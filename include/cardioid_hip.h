@@ -419,18 +419,26 @@ int cdh_batch_read_checkpoint(cdh_batch *b, int slab, const char *state_file);
  * read checkpoint + set sensors resumes an evicted slab exactly. */
 int cdh_batch_get_sensors(cdh_batch *b, int slab, double *rows, double *time, int *loop);
 int cdh_batch_set_sensors(cdh_batch *b, int slab, const double *rows, double time, int loop);
-/* advances every slab by nsteps; asynchronous on the batch's stream */
+/* advances every slab by nsteps; asynchronous on the batch's stream.  While
+ * the live slabs' 64-cell tiles all fit the chip at once (about 200,000 to
+ * 260,000 cells, by mode), no halo is linked and no launch was chosen with
+ * cdh_batch_set_launch, a run of 16 steps or more keeps the cells resident
+ * over many steps of one cooperative launch, with the same results bit for
+ * bit.  Such launches of several batches follow one another on the device. */
 int cdh_batch_run(cdh_batch *b, int nsteps);
 int cdh_batch_run_timed(cdh_batch *b, int nsteps, double *ms);
 int cdh_batch_sync(cdh_batch *b);
-/* steps per captured HIP graph (even; 0 launches each step directly) */
+/* steps per captured HIP graph (even; 0 launches each step directly), for
+ * runs of the step kernels */
 int cdh_batch_set_graph(cdh_batch *b, int steps);
 /* launch configuration: the kernel instance's register target (waves/SIMD:
  * FP64 2..3, mixed 3..4), the workgroup size (64, 128, 256), a cap on the
  * waves per SIMD resident at run time (0: none; applied by reserving LDS per
  * workgroup) and the order in which tiles meet the 8 XCDs, each with its own
  * L2 (-1: XCD x serves the x-th contiguous eighth of the tiles; k >= 0: runs
- * of 2^k workgroups dealt to the XCDs in turn) */
+ * of 2^k workgroups dealt to the XCDs in turn).  From then on every step is
+ * the step kernel's (see cdh_batch_run), until an autotune finds the
+ * resident form faster. */
 int cdh_batch_set_launch(cdh_batch *b, int waves, int block, int occupancy, int tile_order);
 int cdh_batch_get_launch(cdh_batch *b, int *waves, int *block, int *occupancy, int *tile_order);
 /* times every launch configuration for `steps` steps from the current state

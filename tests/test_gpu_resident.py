@@ -1,0 +1,138 @@
+"""The resident kernels (csrc/engine_resident.hpp) against the step kernels,
+bit for bit: Vm, states, activation and APD90 times, counts, range record and
+clock.  A launch chosen with set_launch runs the step kernels; the default
+runs of 16 steps and more are resident where the tiles fit the chip (3,072
+tiles, for the fits also 4,096 at four wavefronts per SIMD; mixed 4,096)."""
+import numpy as np
+import pytest
+
+from cardioid_amd import hip, workloads as W
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+DT = 0.02
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    hip.lib()
+    yield
+
+
+def make(slabs, mode, chosen, exact=False, sensors=3):
+    ext = [s.extent() for s in slabs]
+    b = hip.Batch(DT, sum(e[0] for e in ext), sum(e[1] for e in ext), slab_capacity=len(slabs),
+                  mode=mode, sensors=sensors, exact_functions=exact, jhTauSmooth=int(exact))
+    if chosen:
+        b.set_launch(3, 64)
+    return b
+
+
+def slab(nx, ny, nz, phi=20.0, vm_max=100.0, holes=0.0, seed=0, dur=1.0):
+    a = W.fibre_slab(nx, ny, nz, phi)
+    if holes:
+        keep = np.random.default_rng(seed).random(a.ncell) >= holes
+        a = W.Anatomy(nx, ny, nz, a.dx, a.dy, a.dz, a.gid[keep], a.celltype[keep], a.sigma[keep])
+    st = [W.box_stimulus(xMax=3, nx=nx, ny=ny, nz=nz, duration=dur),
+          W.box_stimulus(zMax=2, nx=nx, ny=ny, nz=nz, tStart=1.5, duration=0.4, vStim=-30.0)]
+    return hip.Slab(a, ["midCellML"], W.DIFFUSION_SCALE, st, scales=(0.7, 0.9, 1.0),
+                    vm_max=vm_max)
+
+
+def results(b, ids):
+    out = []
+    for i in ids:
+        out += [b.vm(i), b.state(i), *b.activation(i), b.t90(i), np.array(b.sensor_counts(i)),
+                b.sensors(i)[0]]
+        r, info = b.range_report(i), b.slab_info(i)
+        out.append(np.array([info["time"], info["loop"], r["count"] if r else 0]))
+    return out
+
+
+def compare(slabs, mode, runs, exact=False):
+    got = []
+    for chosen in (False, True):
+        b = make(slabs, mode, chosen, exact)
+        ids = [b.add(s) for s in slabs]
+        for n in runs:
+            print(mode, "step kernels" if chosen else "resident", [s.ncell for s in slabs], n,
+                  flush=True)
+            b.run(n)
+        got.append(results(b, ids))
+        b.close()
+    for a, r in zip(*got):
+        assert np.array_equal(a, r)
+    return got[0]
+
+
+KINDS = [("fp64_fused", False), ("fp64_fma", False), ("mixed_fused", False), ("fp64_fused", True)]
+
+
+@pytest.mark.parametrize("mode,exact", KINDS)
+@pytest.mark.parametrize("dims,holes", [((1, 1, 1), 0.0), ((2, 4, 8), 0.0), ((5, 13, 1), 0.0),
+                                        ((9, 10, 11), 0.3), ((3, 5, 130), 0.0), ((70, 3, 2), 0.1)])
+def test_small_slabs_equal_the_step_kernels(mode, exact, dims, holes):
+    """From one cell and one whole tile on; odd chunks (both box parities),
+    chunks too short for the resident form in between, and more steps than
+    one launch takes."""
+    s = slab(*dims, holes=holes, vm_max=20.0)
+    out = compare([s], mode, (17, 3, 16, 301), exact)
+    assert np.ptp(out[0]) >= 0 and np.isfinite(out[0]).all()
+
+
+@pytest.mark.parametrize("mode,ntile", [("fp64_fused", 3072), ("fp64_fused", 3073),
+                                        ("fp64_fma", 4096), ("mixed_fused", 4096),
+                                        ("mixed_fused", 4097)])
+def test_tiles_at_the_edges_of_what_the_chip_holds(mode, ntile):
+    """64 x ntile cells in one slab: the last that fits each kernel, and the
+    first that does not."""
+    compare([slab(ntile // 64 if ntile % 64 == 0 else ntile, 64 if ntile % 64 == 0 else 8,
+                  64 if ntile % 64 == 0 else 8)], mode, (40,))
+
+
+@pytest.mark.parametrize("mode", ["fp64_fma", "mixed_fused"])
+def test_slabs_come_and_go(mode):
+    """Several slabs with clocks of their own; one leaves (the tiles then are
+    a list with a hole) and a smaller one takes its place."""
+    s = [slab(9, 10, 11, 5.0), slab(20, 6, 7, -40.0, holes=0.2), slab(4, 4, 40, 80.0),
+         slab(6, 7, 8, 33.0)]
+    got = []
+    for chosen in (False, True):
+        b = make(s, mode, chosen)
+        ids = [b.add(x) for x in s[:3]]
+        b.run(33)
+        b.remove(ids[1])
+        b.run(20)
+        ids[1] = b.add(s[3])
+        b.run(50)
+        b.run(21)
+        got.append(results(b, ids))
+        b.close()
+    for a, r in zip(*got):
+        assert np.array_equal(a, r)
+
+
+@pytest.mark.parametrize("mode", ["fp64_fma", "mixed_fused"])
+def test_apd90_over_a_whole_beat(mode):
+    """25,000 steps of a tiny slab: activation, Vmax and t90 of every cell."""
+    out = compare([slab(4, 5, 6)], mode, (20000,))
+    assert (out[5] > 0).all()
+
+
+def test_autotune_leaves_the_state_alone():
+    s = slab(12, 13, 14)
+    got = []
+    for tune in (False, True):
+        b = make([s], "fp64_fma", False)
+        ids = [b.add(s)]
+        b.run(31)
+        if tune:
+            best, rows = b.autotune(5)
+            assert best > 0 and len(rows) == 18
+        b.run(64)
+        got.append(results(b, ids))
+        b.close()
+    for a, r in zip(*got):
+        assert np.array_equal(a, r)
