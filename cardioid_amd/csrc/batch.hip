@@ -274,8 +274,7 @@ int cdh_batch_get_vm(cdh_batch *b, int slab, double *vm)
    return guard([&] {
       CDH_REQUIRE(vm, "cdh_batch_get_vm: null output");
       Engine &e = engine(b);
-      const std::vector<double> v = e.vm(slab);
-      scatter(e.slab(slab), v.data(), vm);
+      e.read_vm(slab, vm);
    });
 }
 
@@ -284,8 +283,7 @@ int cdh_batch_get_state(cdh_batch *b, int slab, double *state)
    return guard([&] {
       CDH_REQUIRE(state, "cdh_batch_get_state: null output");
       Engine &e = engine(b);
-      const std::vector<double> st = e.state19(slab);
-      scatter(e.slab(slab), st.data(), state, N_STATE);
+      e.read_state(slab, state);
    });
 }
 
@@ -293,13 +291,7 @@ int cdh_batch_get_activation(cdh_batch *b, int slab, double *tact0, double *tact
 {
    return guard([&] {
       Engine &e = engine(b);
-      const Engine::Slab &s = e.slab(slab);
-      std::vector<double> v[3];
-      for (auto &x : v) x.resize(s.n);
-      e.activation(slab, v[0].data(), v[1].data(), v[2].data());
-      double *dst[3] = {tact0, tact, trec};
-      for (int q = 0; q < 3; q++)
-         if (dst[q]) scatter(s, v[q].data(), dst[q]);
+      e.read_activation(slab, tact0, tact, trec);
    });
 }
 
@@ -308,10 +300,7 @@ int cdh_batch_get_t90(cdh_batch *b, int slab, double *t90)
    return guard([&] {
       CDH_REQUIRE(t90, "cdh_batch_get_t90: null output");
       Engine &e = engine(b);
-      const Engine::Slab &s = e.slab(slab);
-      std::vector<double> v(s.n);
-      e.t90(slab, v.data());
-      scatter(s, v.data(), t90);
+      e.read_t90(slab, t90);
    });
 }
 

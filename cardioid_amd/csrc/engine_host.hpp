@@ -46,6 +46,14 @@ struct LaunchCfg {
                       // runs of 2^k workgroups dealt in turn (engine_tile_group)
 };
 
+// rows of a slab's results in the caller's cell order
+struct RowArgs {
+   int64_t n, S;                // cells, and the slab's cells in whole tiles
+   const uint32_t *inv;         // per cell of the caller's order, its place in the slab
+   double *out;
+   int row0;                    // the number of the first row of a launch
+};
+
 class Engine {
  public:
    struct Slab {
@@ -61,6 +69,7 @@ class Engine {
       std::vector<int64_t> remote_gid;
       std::vector<uint32_t> remote_bi; // box index within the slab's box
       int sensors = 0;
+      bool order_up = false;           // the caller's order is on the device
       double time = 0.0;               // host copy of the slab clock
       int loop = 0;
    };
@@ -113,12 +122,15 @@ class Engine {
    // sets them and the clock exactly; the sensors then continue the run
    // (the step's Vm before is their previous one)
    void set_sensor_state(int id, const double *rows, double time, int loop);
-   void activation(int id, double *tact0, double *tact, double *trec);   // slab order
+   // results into the caller's arrays, in its cell order (the input's)
+   void read_vm(int id, double *host);                    // n
+   void read_state(int id, double *host);                 // [19][n]
+   void read_activation(int id, double *tact0, double *tact, double *trec);   // n; null: skipped
+   void read_t90(int id, double *host);                   // n
    // cells of the slab whose tact0, tact and trec have been recorded, kept
    // on the device by the step kernels (one wavefront ballot and atomic per
    // kind that occurs); the sensors' own counts, reset with them
    void sensor_counts(int id, int64_t *n_tact0, int64_t *n_tact, int64_t *n_trec);
-   void t90(int id, double *out);
    // out-of-range record since the last call (cell as a slab-order index);
    // clears it
    RangeRec range_report(int id);
@@ -135,6 +147,9 @@ class Engine {
 
  private:
    void step_eager();
+   RowArgs row_args(int id, int rows);
+   void copy_row(int64_t n, double *host);
+   void read_cols(int id, int ncol, const double *const *arena, double *const *host);
    bool resident_fits() const;
    int run_resident(int nsteps);
    void launch_step(int parity);
@@ -208,9 +223,9 @@ class Engine {
    bool list_dirty_ = true;
    bool tiles_direct_ = false;     // the live tiles are tile_base_ .. + nlist_ - 1
    int64_t tile_base_ = 0;
-   // the resident form (engine_resident.hpp): per tile its neighbours' tiles
-   // and the steps it has done, counted in epoch_ over all launches
-   DevBuf<uint32_t> links_tile_, flags_;
+   // the resident form (engine_resident.hpp): per tile the steps it has done,
+   // counted in epoch_ over all launches, and behind them its links
+   DevBuf<uint32_t> flags_;
    uint32_t epoch_ = 0;
    bool links_dirty_ = true;
    bool resident_ = true;          // off once the caller chooses a launch
@@ -231,6 +246,11 @@ class Engine {
    DevBuf<double> coef_;
    DevBuf<ParamSet> psets_;
    DevBuf<uint32_t> meta_, bi_;
+   DevBuf<double> row_;            // rows of results, as long as the longest read yet
+   static constexpr int64_t kReadPiece = int64_t(1) << 18;   // doubles (2 MiB)
+   static constexpr int kReadThreads = 8;
+   double *read_piece_[2] = {nullptr, nullptr};              // pinned
+   hipEvent_t read_ev_[2] = {nullptr, nullptr};
    DevBuf<uint16_t> blk_slab_;
    DevBuf<SlabDev> slabdev_;
    DevBuf<double> state_, st64_;

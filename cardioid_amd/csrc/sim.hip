@@ -356,9 +356,7 @@ int cdh_sim_get_vm(cdh_sim *s, double *host)
          s->loopsim->Vm.download(host, s->n);
          return;
       }
-      const std::vector<double> v = s->eng->vm(s->slab);
-      const std::vector<int64_t> &perm = sim_perm(s);
-      for (int64_t k = 0; k < s->n; k++) host[perm[k]] = v[k];
+      s->eng->read_vm(s->slab, host);
    });
 }
 
@@ -379,10 +377,7 @@ int cdh_sim_get_state(cdh_sim *s, double *host)
          }
          return;
       }
-      const std::vector<double> st = s->eng->state19(s->slab);
-      const std::vector<int64_t> &perm = sim_perm(s);
-      for (int q = 0; q < N_STATE; q++)
-         for (int64_t k = 0; k < n; k++) host[q * n + perm[k]] = st[q * n + k];
+      s->eng->read_state(s->slab, host);
    });
 }
 
@@ -431,15 +426,7 @@ int cdh_sim_get_activation(cdh_sim *s, double *tact0, double *tact, double *trec
          s->loopsim->sensor[0]->get(tact0, tact, trec);
          return;
       }
-      const int64_t n = s->n;
-      const std::vector<int64_t> &perm = sim_perm(s);
-      std::vector<double> v[3];
-      for (auto &x : v) x.resize(n);
-      s->eng->activation(s->slab, v[0].data(), v[1].data(), v[2].data());
-      double *dst[3] = {tact0, tact, trec};
-      for (int q = 0; q < 3; q++)
-         if (dst[q])
-            for (int64_t k = 0; k < n; k++) dst[q][perm[k]] = v[q][k];
+      s->eng->read_activation(s->slab, tact0, tact, trec);
    });
 }
 
@@ -474,10 +461,7 @@ int cdh_sim_get_t90(cdh_sim *s, double *t90)
          s->loopsim->sensor[0]->t90(t90);
          return;
       }
-      std::vector<double> v(s->n);
-      s->eng->t90(s->slab, v.data());
-      const std::vector<int64_t> &perm = sim_perm(s);
-      for (int64_t k = 0; k < s->n; k++) t90[perm[k]] = v[k];
+      s->eng->read_t90(s->slab, t90);
    });
 }
 
