@@ -225,6 +225,169 @@ struct ResidentF64 {
    }
 };
 
+// One wavefront's part of a cell for resident_split_run; each uses the states
+// it owns, and the others' from LDS.
+template <int KIND>
+struct SplitF64 {
+   using Shared = SplitShared<double, float, 18>;
+   double st[N_STATE];
+   SodiumPotassiumCurrents nk;
+   double I_NaCa, A0;
+
+   // one field of the pair layout (run_pair_index)
+   __device__ __forceinline__ static uint32_t lane_off(const ResidentTile &t, int q)
+   {
+      return q < N_STATE - 1 ? 16u * t.lc + 8u * (q & 1) : 8u * t.lc;
+   }
+   __device__ __forceinline__ static uint32_t field_off(const ResidentTile &t, int q)
+   {
+      return 8u * t.rw * (q < N_STATE - 1 ? (q & ~1) : q);
+   }
+   __amdgpu_buffer_rsrc_t RS;
+   __device__ __forceinline__ void load(const ResidentTile &t, int q)
+   {
+      st[q] = box_load(RS, lane_off(t, q), field_off(t, q));
+   }
+   __device__ __forceinline__ void store(const ResidentTile &t, int q)
+   {
+      stream_store_f64(st[q], RS, lane_off(t, q), field_off(t, q));
+   }
+   __device__ __forceinline__ void states(const EngineArgs &a, const ResidentTile &t)
+   {
+      RS = stream_rsrc(a.state + t.run_cell * N_STATE);
+   }
+
+   __device__ __forceinline__ void load_na_k(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+      load(t, S_DVK_I);
+      load(t, S_NA_I);
+   }
+   __device__ __forceinline__ void store_na_k(const ResidentTile &t)
+   {
+      store(t, S_DVK_I);
+      store(t, S_NA_I);
+   }
+   __device__ __forceinline__ void share_na(Shared *sh, int p, int lane)
+   {
+      sh->na[p][lane] = st[S_NA_I];
+   }
+   __device__ __forceinline__ void load_ca(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+      for (int q : {S_CA_I, S_CA_SS, S_CA_SR, S_R_PRIME, S_FCASS}) load(t, q);
+   }
+   __device__ __forceinline__ void store_ca(const ResidentTile &t)
+   {
+      for (int q : {S_CA_I, S_CA_SS, S_CA_SR, S_R_PRIME, S_FCASS}) store(t, q);
+   }
+   __device__ __forceinline__ void share_ca(Shared *sh, int p, int lane)
+   {
+      sh->ca[p][lane] = st[S_CA_I];
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void load_gates(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+#pragma unroll
+      for (int q = S_M; q < N_STATE; q++)
+         if ((GATES >> (q - S_M)) & 1) load(t, q);
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void store_gates(const ResidentTile &t)
+   {
+#pragma unroll
+      for (int q = S_M; q < N_STATE; q++)
+         if ((GATES >> (q - S_M)) & 1) store(t, q);
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void share_gates(Shared *sh, int p, int lane)
+   {
+#pragma unroll
+      for (int q = S_M; q < N_STATE; q++)
+         if ((GATES >> (q - S_M)) & 1) sh->gate[p][q - S_M][lane] = st[q];
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void take_gates(const Shared *sh, int p, int lane)
+   {
+#pragma unroll
+      for (int q = S_M; q < N_STATE; q++)
+         if ((GATES >> (q - S_M)) & 1) st[q] = sh->gate[p][q - S_M][lane];
+   }
+   template <class F>
+   __device__ __forceinline__ static void voltage_fns(const ModelTables &T, F &&f)
+   {
+      if constexpr (KIND == kExact) f(exact_voltage_fns(T.E, T.K));
+      else f(fit_voltage_fns<KIND == kFitsFma>(T.coef));
+   }
+   __device__ __forceinline__ void na_k(const EngineArgs &, const ModelTables &T, const ParamSet &P,
+                                        double V, const Shared *sh, int p, int lane)
+   {
+      take_gates<kGatesNaK>(sh, p, lane);
+      voltage_fns(T, [&](const auto &fvs) {
+         double fv[6];
+         fvs.fv05(V, fv);
+         I_NaCa = exchanger64(st[S_NA_I], sh->ca[p][lane], fv[1], fv[2]);
+         nk = nongate_na_k64(*T.K, P, fvs, V, fv[0], fv[5], I_NaCa, st);
+      });
+   }
+   __device__ __forceinline__ void calcium(const EngineArgs &a, const ModelTables &T,
+                                           const ParamSet &P, double V, Shared *sh, int p, int lane)
+   {
+      take_gates<kGatesCa>(sh, p, lane);
+      voltage_fns(T, [&](const auto &fvs) {
+         double fv[6];
+         fvs.fv05(V, fv);
+         const double I = exchanger64(sh->na[p][lane], st[S_CA_I], fv[1], fv[2]);
+         const CalciumCurrents ca = nongate_calcium64(*T.K, P, a.dt, V, fv[3], fv[4], I, st);
+         sh->I_sum[lane] = ca.I_sum;
+         sh->I_CaL[lane] = ca.I_CaL;
+      });
+   }
+   __device__ __forceinline__ double sum(const EngineArgs &a, const ModelTables &T,
+                                         const Shared *sh, int lane)
+   {
+      return nongate_sum64(*T.K, a.dt, I_NaCa, CalciumCurrents{sh->I_sum[lane], sh->I_CaL[lane]},
+                           nk, st);
+   }
+   __device__ __forceinline__ void finish(const EngineArgs &, const ModelTables &, double, double)
+   {
+   }
+   __device__ __forceinline__ void gates(const EngineArgs &a, const ModelTables &T, int s_switch,
+                                         uint32_t meta, double V, uint32_t mask)
+   {
+      if constexpr (KIND == kExact) {
+         if (!((meta >> 8) & kFlagGatesFixed))
+            gates_exact64(*T.E, s_switch, a.dt, V, st, mask);
+      } else {
+         gates64<KIND == kFitsFma>(T.coef, T.K->exp_coef, s_switch, (uint8_t)(meta >> 8), V, st,
+                                   mask);
+      }
+   }
+   __device__ __forceinline__ void load_weights(const EngineArgs &a, const ResidentTile &t,
+                                                Shared *sh)
+   {
+      const float *wp = a.Aw + (int64_t)t.blk * (18 * kBlk) + t.lane;
+#pragma unroll
+      for (int k = 0; k < 18; k++) sh->w[k][t.lane] = wp[kBlk * k];
+      A0 = 0.0;
+#pragma unroll
+      for (int k = 0; k < 18; k++) A0 -= sh->w[k][t.lane];
+   }
+   __device__ __forceinline__ double diffuse(const ResidentTile &t, __amdgpu_buffer_rsrc_t R,
+                                             double V, double scale, const Shared *sh)
+   {
+      double nb[18];
+#pragma unroll
+      for (int k = 0; k < 18; k++) nb[k] = t.neighbour(R, k + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      double tmp = A0 * V;
+#pragma unroll
+      for (int k = 1; k < 19; k++) tmp += (double)sh->w[k - 1][t.lane] * nb[k - 1];
+      return tmp * scale;
+   }
+};
+
 }  // namespace
 
 template <int KIND, int WAVES>
@@ -234,6 +397,20 @@ __global__ __launch_bounds__(64, WAVES) void k_resident_f64(EngineArgs a, Reside
    resident_run<ResidentF64<KIND>>(a, r, &sh);
 }
 
+template <int KIND, int WAVES>
+__global__ __launch_bounds__(kSplitWaves * 64, WAVES) void k_resident_split_f64(EngineArgs a,
+                                                                                ResidentArgs r)
+{
+   __shared__ typename SplitF64<KIND>::Shared sh;
+   resident_split_run<SplitF64<KIND>>(a, r, &sh);
+}
+
+template __global__ void k_resident_split_f64<kFits, 6>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_split_f64<kFits, 8>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_split_f64<kFitsFma, 6>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_split_f64<kFitsFma, 8>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_split_f64<kExact, 6>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_split_f64<kExact, 8>(EngineArgs, ResidentArgs);
 template __global__ void k_resident_f64<kFits, 3>(EngineArgs, ResidentArgs);
 template __global__ void k_resident_f64<kFits, 4>(EngineArgs, ResidentArgs);
 template __global__ void k_resident_f64<kFitsFma, 3>(EngineArgs, ResidentArgs);

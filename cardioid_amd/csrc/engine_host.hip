@@ -154,19 +154,27 @@ __global__ __launch_bounds__(64) void k_slab_clock(SlabDev *slabs, int nslab, in
 }
 
 // The resident kernels of a mode, from the one with the fewest tiles on the
-// chip to the one with the most.  The FP64 kernel holds 3 wavefronts per SIMD
-// (3,072 tiles on 256 CUs) without spills; at 4 it spills some 12 registers,
+// chip to the one with the most.  Six wavefronts to a tile leave room for
+// four tiles on a CU (1,024 on 256 CUs).  The FP64 kernel holds 3 wavefronts
+// per SIMD (3,072 tiles) without spills; at 4 it spills some 17 registers,
 // which 64^3 cells repay (4,096 tiles: FMA 16.5 us a step against 24.5 by
 // step kernels, reference rounding 18.1 against 24.6) and fewer tiles do not
 // (54x56x64 cells: 13.0 us a step against 11.6 at 3).  The exact functions
 // spill too much at 4 (39 against 32 us at 64^3 by step kernels).
-using ResidentFn = void (*)(EngineArgs, ResidentArgs);
-std::vector<ResidentFn> resident_kernels(int mode, bool exact)
+struct ResidentKernel {
+   void (*fn)(EngineArgs, ResidentArgs);
+   int threads;
+};
+std::vector<ResidentKernel> resident_kernels(int mode, bool exact)
 {
-   if (mode == CDH_MODE_MIXED_FUSED) return {k_resident_mixed};
-   if (exact) return {k_resident_f64<kExact, 3>};
-   if (mode == CDH_MODE_FP64_FMA) return {k_resident_f64<kFitsFma, 3>, k_resident_f64<kFitsFma, 4>};
-   return {k_resident_f64<kFits, 3>, k_resident_f64<kFits, 4>};
+   constexpr int split = kSplitWaves * kBlk;
+   if (mode == CDH_MODE_MIXED_FUSED) return {{k_resident_split_mixed, split}, {k_resident_mixed, kBlk}};
+   if (exact) return {{k_resident_split_f64<kExact, 6>, split}, {k_resident_split_f64<kExact, 8>, split}, {k_resident_f64<kExact, 3>, kBlk}};
+   if (mode == CDH_MODE_FP64_FMA)
+      return {{k_resident_split_f64<kFitsFma, 6>, split}, {k_resident_split_f64<kFitsFma, 8>, split}, {k_resident_f64<kFitsFma, 3>, kBlk},
+              {k_resident_f64<kFitsFma, 4>, kBlk}};
+   return {{k_resident_split_f64<kFits, 6>, split}, {k_resident_split_f64<kFits, 8>, split}, {k_resident_f64<kFits, 3>, kBlk},
+           {k_resident_f64<kFits, 4>, kBlk}};
 }
 
 using KernelFn = void (*)(EngineArgs);
@@ -516,9 +524,20 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
    int ncu = 0, coop = 0;
    CDH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
    CDH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-   for (ResidentFn fn : resident_kernels(mode, exact_ != 0)) {
+   for (const ResidentKernel &k : resident_kernels(mode, exact_ != 0)) {
       int per_cu = 0;
-      CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlk, 0));
+      CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, k.threads, 0));
+      // The call counts wavefronts per CU, as if a workgroup's could stand on
+      // any SIMD: it gives 4 workgroups of 6 wavefronts at 80 registers where
+      // 3 run at once (seen on the device).  A workgroup of several takes
+      // ceil(w / 4) places of the SIMD that has most of it, of the 512 / (its
+      // registers, by eights) that a SIMD has, at most 8.
+      if (k.threads > kBlk) {
+         hipFuncAttributes fa{};
+         CDH_HIP(hipFuncGetAttributes(&fa, (const void *)k.fn));
+         const int places = std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
+         per_cu = std::min(per_cu, places / ((k.threads / kBlk + 3) / 4));
+      }
       resident_cap_.push_back(coop ? (int64_t)ncu * per_cu : 0);
       resident_tiles_ = std::max(resident_tiles_, resident_cap_.back());
    }
@@ -938,10 +957,9 @@ int Engine::run_resident(int nsteps)
       CDH_LAUNCH_CHECK();
       links_dirty_ = false;
    }
-   const std::vector<ResidentFn> fns = resident_kernels(mode_, exact_ != 0);
    size_t which = 0;
    while (resident_cap_[which] < (nlist_ + 7) / 8 * 8) ++which;     // resident_fits()
-   const ResidentFn fn = fns[which];
+   const ResidentKernel kernel = resident_kernels(mode_, exact_ != 0)[which];
    while (nsteps > 0) {
       const int n = std::min(nsteps, kResidentSteps);
       EngineArgs a = args(parity_);
@@ -956,8 +974,8 @@ int Engine::run_resident(int nsteps)
       r.box[1] = box_[parity_ ^ 1].p;
       r.failed = failed_;
       void *kargs[2] = {&a, &r};
-      if (hipLaunchCooperativeKernel((const void *)fn, dim3(8 * a.groups_per_xcd), dim3(kBlk),
-                                     kargs, 0, stream_) != hipSuccess) {
+      if (hipLaunchCooperativeKernel((const void *)kernel.fn, dim3(8 * a.groups_per_xcd),
+                                     dim3(kernel.threads), kargs, 0, stream_) != hipSuccess) {
          (void)hipGetLastError();
          resident_ = false;
          return nsteps;

@@ -232,10 +232,10 @@ class Engine {
    std::vector<int64_t> resident_cap_;   // tiles at once, per kernel of resident_kernels()
    int64_t resident_tiles_ = 0;    // the most of them
    uint32_t *failed_ = nullptr;    // host memory the kernel writes
-   // A cooperative launch takes about 24 us more than a plain one: 8 steps of
-   // 504 cells gain next to nothing (94 us against 80), 16 do (130 against
-   // 160), and so do 16 of more cells (110,592: 176 against 232).
-   static constexpr int kResidentMin = 16;
+   // A cooperative launch takes about 24 us more than a plain one; a step
+   // then saves 3 to 8 us (see resident_kernels and engine_resident.hpp), so
+   // that 4 to 6 steps break even.
+   static constexpr int kResidentMin = 8;
    // Steps in one launch: 2 to 5 ms, after which other streams' kernels get
    // their turn.
    static constexpr int kResidentSteps = 256;

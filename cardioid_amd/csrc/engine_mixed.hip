@@ -243,11 +243,185 @@ struct ResidentMixed {
    }
 };
 
+// One wavefront's part of a cell for resident_split_run (SplitF64 in
+// engine_f64.hip).
+struct SplitMixed {
+   struct Shared : SplitShared<float, uint32_t, 9> {
+      double CaL_b[kBlk];      // I_CaL's second factor (its first is in I_CaL)
+   };
+   float s32[N_STATE32];
+   double s64[N_STATE64];
+   __amdgpu_buffer_rsrc_t R32, R64;
+   const float CDH_CONSTANT *ref;
+   SodiumPotassiumCurrents nk;
+   double I_NaCa;
+
+   __device__ __forceinline__ void states(const EngineArgs &a, const ResidentTile &t)
+   {
+      R32 = stream_rsrc(a.st32 + t.run_cell * N_STATE32);
+      R64 = stream_rsrc(a.st64 + t.run_cell * N_STATE64);
+   }
+   __device__ __forceinline__ void load32(const ResidentTile &t, int q)
+   {
+      s32[q] = stream_load_f32(R32, 4u * t.lc, 4u * t.rw * q);
+   }
+   __device__ __forceinline__ void store32(const ResidentTile &t, int q)
+   {
+      stream_store_f32(s32[q], R32, 4u * t.lc, 4u * t.rw * q);
+   }
+   __device__ __forceinline__ void load64(const ResidentTile &t, int q)
+   {
+      s64[q] = stream_load_f64(R64, 8u * t.lc, 8u * t.rw * q);
+   }
+   __device__ __forceinline__ void store64(const ResidentTile &t, int q)
+   {
+      stream_store_f64(s64[q], R64, 8u * t.lc, 8u * t.rw * q);
+   }
+
+   __device__ __forceinline__ void load_na_k(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+      load32(t, M_DK_I);
+      load64(t, M_NA_I);
+   }
+   __device__ __forceinline__ void store_na_k(const ResidentTile &t)
+   {
+      store32(t, M_DK_I);
+      store64(t, M_NA_I);
+   }
+   __device__ __forceinline__ void share_na(Shared *sh, int p, int lane)
+   {
+      sh->na[p][lane] = s64[M_NA_I];
+   }
+   __device__ __forceinline__ void load_ca(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+      for (int q : {M_CA_SS, M_CA_SR, M_R_PRIME, M_FCASS}) load32(t, q);
+      load64(t, M_CA_I);
+   }
+   __device__ __forceinline__ void store_ca(const ResidentTile &t)
+   {
+      for (int q : {M_CA_SS, M_CA_SR, M_R_PRIME, M_FCASS}) store32(t, q);
+      store64(t, M_CA_I);
+   }
+   __device__ __forceinline__ void share_ca(Shared *sh, int p, int lane)
+   {
+      sh->ca[p][lane] = s64[M_CA_I];
+   }
+   // gate g (from 0, the order of S_M .. S_S) is slot M_M + g
+   template <uint32_t GATES>
+   __device__ __forceinline__ void load_gates(const EngineArgs &a, const ResidentTile &t)
+   {
+      states(a, t);
+#pragma unroll
+      for (int g = 0; g < 12; g++)
+         if ((GATES >> g) & 1) load32(t, M_M + g);
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void store_gates(const ResidentTile &t)
+   {
+#pragma unroll
+      for (int g = 0; g < 12; g++)
+         if ((GATES >> g) & 1) store32(t, M_M + g);
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void share_gates(Shared *sh, int p, int lane)
+   {
+#pragma unroll
+      for (int g = 0; g < 12; g++)
+         if ((GATES >> g) & 1) sh->gate[p][g][lane] = s32[M_M + g];
+   }
+   template <uint32_t GATES>
+   __device__ __forceinline__ void take_gates(const Shared *sh, int p, int lane)
+   {
+#pragma unroll
+      for (int g = 0; g < 12; g++)
+         if ((GATES >> g) & 1) s32[M_M + g] = sh->gate[p][g][lane];
+   }
+   __device__ __forceinline__ void na_k(const EngineArgs &, const ModelTables &T, const ParamSet &P,
+                                        double V, const Shared *sh, int p, int lane)
+   {
+      take_gates<kGatesNaK>(sh, p, lane);
+      const double fv0 = fitM<0>(T.coef, V), fv1 = fitM<1>(T.coef, V), fv2 = fitM<2>(T.coef, V);
+      const double fv5 = fitM<5>(T.coef, V);
+      I_NaCa = exchangerM(s64[M_NA_I], sh->ca[p][lane], fv1, fv2);
+      nk = na_kM(*T.K, P, T.coef, V, P.K0 + (double)s32[M_DK_I], fv0, fv5, I_NaCa, s32, s64);
+   }
+   __device__ __forceinline__ void calcium(const EngineArgs &a, const ModelTables &T,
+                                           const ParamSet &P, double V, Shared *sh, int p, int lane)
+   {
+      take_gates<kGatesCa>(sh, p, lane);
+      const double fv1 = fitM<1>(T.coef, V), fv2 = fitM<2>(T.coef, V);
+      const double fv3 = fitM<3>(T.coef, V), fv4 = fitM<4>(T.coef, V);
+      const double I = exchangerM(sh->na[p][lane], s64[M_CA_I], fv1, fv2);
+      const CalciumCurrentsM ca = calciumM(*T.K, P, a.dt, V, fv3, fv4, I, s32, s64);
+      sh->I_sum[lane] = ca.I_sum;
+      sh->I_CaL[lane] = ca.CaL_a;
+      sh->CaL_b[lane] = ca.CaL_b;
+   }
+   __device__ __forceinline__ double sum(const EngineArgs &a, const ModelTables &T,
+                                         const Shared *sh, int lane)
+   {
+      return sumM(*T.K, a.dt, I_NaCa,
+                  CalciumCurrentsM{sh->I_sum[lane], sh->I_CaL[lane], sh->CaL_b[lane]}, nk, s64);
+   }
+   __device__ __forceinline__ void finish(const EngineArgs &a, const ModelTables &T, double dVD,
+                                          double iStim)
+   {
+      s32[M_DK_I] = (float)((double)s32[M_DK_I] + (a.dt * T.K->c9) * (nk.iK - dVD - iStim));
+   }
+   __device__ __forceinline__ void gates(const EngineArgs &, const ModelTables &T, int s_switch,
+                                         uint32_t meta, double V, uint32_t mask)
+   {
+      gatesM(T.coef, T.K->exp_coef, s_switch, (uint8_t)(meta >> 8), V, s32, mask);
+   }
+   __device__ __forceinline__ void load_weights(const EngineArgs &a, const ResidentTile &t,
+                                                Shared *sh)
+   {
+      const uint32_t *wp = a.Aw16 + (int64_t)t.blk * (9 * kBlk);
+#pragma unroll
+      for (int g = 0; g < 2; g++) {
+         const u32x4 q = *((const u32x4 *)(wp + g * 4 * kBlk) + t.lane);
+         sh->w[4 * g][t.lane] = q.x;
+         sh->w[4 * g + 1][t.lane] = q.y;
+         sh->w[4 * g + 2][t.lane] = q.z;
+         sh->w[4 * g + 3][t.lane] = q.w;
+      }
+      sh->w[8][t.lane] = wp[8 * kBlk + t.lane];
+      ref = (const float CDH_CONSTANT *)(a.Aref + (int64_t)t.blk * 18);
+   }
+   __device__ __forceinline__ double diffuse(const ResidentTile &t, __amdgpu_buffer_rsrc_t R,
+                                             double V, double scale, const Shared *sh)
+   {
+      double nb[18];
+#pragma unroll
+      for (int k = 0; k < 18; k++) nb[k] = t.neighbour(R, k + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      float acc = 0.0f;
+#pragma unroll
+      for (int p = 0; p < 9; p++) {
+         const uint32_t hw = sh->w[p][t.lane];
+         const float w0 = half_lo_plus(hw, ref[2 * p]);
+         const float w1 = half_hi_plus(hw, ref[2 * p + 1]);
+         acc = __builtin_fmaf(w0, (float)(nb[2 * p] - V), acc);
+         acc = __builtin_fmaf(w1, (float)(nb[2 * p + 1] - V), acc);
+      }
+      return (double)acc * (scale * (double)t.S->wdelta_scale);
+   }
+};
+
 }  // namespace
 
 __global__ __launch_bounds__(64, 4) void k_resident_mixed(EngineArgs a, ResidentArgs r)
 {
    resident_run<ResidentMixed>(a, r, nullptr);
+}
+
+__global__ __launch_bounds__(kSplitWaves * 64, 8) void k_resident_split_mixed(EngineArgs a,
+                                                                              ResidentArgs r)
+{
+   __shared__ SplitMixed::Shared sh;
+   resident_split_run<SplitMixed>(a, r, &sh);
 }
 
 }  // namespace cdh

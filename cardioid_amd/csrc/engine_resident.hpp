@@ -82,17 +82,60 @@ struct ModelTables {
 // what a wavefront knows of its tile
 struct ResidentTile {
    ConstSlab *S;
-   int blk, lane;
+   int j, blk, sl, lane;        // its place in the list of live tiles, the tile, its slab
+   uint32_t meta;
+   bool live;
    uint32_t b8;                 // this lane's box offset in bytes
    uint32_t lc, rw;             // its place in the run of cells its states are in, the run's width
    int64_t run_cell;            // the run's first cell in the arena
+   // false: nothing to do for the whole workgroup
+   __device__ __forceinline__ bool find(const EngineArgs &a)
+   {
+      j = engine_tile_group(a);
+      if (j >= a.ntile) return false;
+      lane = threadIdx.x & (kBlk - 1);
+      blk = __builtin_amdgcn_readfirstlane(a.tiles ? (int)a.tiles[j] : a.tile_base + j);
+      sl = __builtin_amdgcn_readfirstlane((int)a.blk_slab[blk]);
+      if (sl == kNoSlab) return false;
+      S = (ConstSlab *)(a.slabs + sl);
+      if (!S->active) return false;
+      const int64_t i = (int64_t)blk * kBlk + lane;
+      meta = a.meta[i];
+      live = !(meta & kMetaPad);
+      b8 = a.bi[i] * 8u;
+      const int64_t k0 = (int64_t)(blk - S->first_blk) * kBlk;
+      const int64_t r0 = k0 & ~(kRun - 1);
+      rw = (uint32_t)run_width(k0, (int64_t)S->ntile * kBlk);
+      run_cell = (int64_t)S->first_blk * kBlk + r0;
+      lc = (uint32_t)(k0 - r0 + lane);
+      return true;
+   }
    // node k's Vm from the box behind R, past the caches that other XCDs'
    // stores do not reach
    __device__ __forceinline__ double neighbour(__amdgpu_buffer_rsrc_t R, int k) const
    {
       return box_load_agent(R, b8, S->soff[k]);
    }
+   __device__ __forceinline__ const ParamSet *params(const EngineArgs &a) const
+   {
+      return a.params + S->param_base + (int)(meta & 0xFFu);
+   }
+   // The cell's number, made anew: the addresses that only a sensor event or
+   // an out-of-range cell needs are then made there, not held over the loop.
+   __device__ __forceinline__ uint32_t cell() const
+   {
+      uint32_t c = (uint32_t)blk * kBlk + lane;
+      asm volatile("" : "+v"(c));
+      return c;
+   }
 };
+
+// The tables' addresses made anew in every step: otherwise their loads move
+// out of the loop, hundreds of scalars that no wavefront can hold.
+__device__ __forceinline__ void renew(ModelTables &T)
+{
+   asm volatile("" : "+s"(T.K), "+s"(T.E), "+s"(T.coef));
+}
 
 // Waits until every tile of the three ranges has done `target` - base steps.
 __device__ __forceinline__ void resident_wait(const ResidentArgs &r, const uint32_t *lk, int lane,
@@ -122,132 +165,335 @@ __device__ __forceinline__ void resident_wait(const ResidentArgs &r, const uint3
    }
 }
 
-// The launch's steps of one tile.  C holds the cell's states and weights and
-// gives the reaction, the stencil sum and what follows Vm's update, each as
-// the step kernel of its precision has it.
-template <class C>
-__device__ __forceinline__ void resident_run(const EngineArgs &a, const ResidentArgs &r,
-                                             typename C::Shared *sh)
-{
-   const int lane = threadIdx.x;
-   const int j = engine_tile_group(a);
-   if (j >= a.ntile) return;
-   ResidentTile t;
-   t.lane = lane;
-   t.blk = __builtin_amdgcn_readfirstlane(a.tiles ? (int)a.tiles[j] : a.tile_base + j);
-   const int sl = __builtin_amdgcn_readfirstlane((int)a.blk_slab[t.blk]);
-   if (sl == kNoSlab) return;
-   t.S = (ConstSlab *)(a.slabs + sl);
-   if (!t.S->active) return;
-   const int64_t i = (int64_t)t.blk * kBlk + lane;
-   const uint32_t meta = a.meta[i];
-   const bool live = !(meta & kMetaPad);
-   const uint32_t b = a.bi[i];
-   t.b8 = b * 8u;
-   const int64_t k0 = (int64_t)(t.blk - t.S->first_blk) * kBlk;
-   const int64_t r0 = k0 & ~(kRun - 1);
-   t.rw = (uint32_t)run_width(k0, (int64_t)t.S->ntile * kBlk);
-   t.run_cell = (int64_t)t.S->first_blk * kBlk + r0;
-   t.lc = (uint32_t)(k0 - r0 + lane);
-   C c;
-   c.load(a, t, sh);
-   double V = r.box[0][b];
-   const ParamSet *const params = a.params + t.S->param_base + (int)(meta & 0xFFu);
+// The neighbours of a tile and the steps they have done.
+struct ResidentLinks {
    uint32_t lk[6];
-#pragma unroll
-   for (int q = 0; q < 6; q++) lk[q] = __builtin_amdgcn_readfirstlane(r.links[6 * j + q]);
-   // the stimuli that reach any cell of the tile
-   uint32_t tile_stim = 0;
-   for (int q = 0; q < kSlabStim; q++)
-      if (__ballot((meta >> (16 + q)) & 1u)) tile_stim |= 1u << q;
-   SlabView v;
-   v.scale = t.S->scale;
-   v.threshold = t.S->threshold;
-   v.check_range = t.S->check_range;
-   v.vm_min = t.S->vm_min;
-   v.vm_max = t.S->vm_max;
-   double time = t.S->time[a.parity];
-   int loop = t.S->loop[a.parity];
-   const int sensor_start = t.S->sensor_start;
-   // APD90's phase and largest Vm stay in registers between the steps
-   int apd_phase = 0;
-   double apd_vmax = 0.0, vrest = 0.0;
-   if (a.sensors & 2) {
-      apd_phase = a.apd_phase[i];
-      apd_vmax = a.vmax[i];
-      vrest = params->Vm0;
-   }
-   EngineArgs as = a;           // the sensors' arguments without APD90
-   as.sensors = a.sensors & 1;
    bool bail = false;
-   ModelTables T{constant_ptr(a.K), constant_ptr(a.E), constant_ptr(a.coef)};
-   for (int k = 0; k < r.nsteps; k++) {
-      // the tables' addresses made anew in every step: otherwise their loads
-      // move out of the loop, hundreds of scalars that no wavefront can hold
-      asm volatile("" : "+s"(T.K), "+s"(T.E), "+s"(T.coef));
-      // likewise the cell's place, so that the addresses that only a sensor
-      // event or an out-of-range cell needs are made there, not held
-      uint32_t cell = (uint32_t)t.blk * kBlk + lane;
-      asm volatile("" : "+v"(cell));
-      const ParamSet &P = *params;
-      const double dVR = c.react(a, T, P, meta, V);
+   __device__ __forceinline__ void load(const ResidentArgs &r, int j)
+   {
+#pragma unroll
+      for (int q = 0; q < 6; q++) lk[q] = __builtin_amdgcn_readfirstlane(r.links[6 * j + q]);
+   }
+   // before the stencil of step k of the launch
+   __device__ __forceinline__ void wait(const ResidentArgs &r, const ResidentTile &t, int k)
+   {
       if (k > 0) {
-         resident_wait(r, lk, lane, r.base + (uint32_t)k, bail);
+         resident_wait(r, lk, t.lane, r.base + (uint32_t)k, bail);
          asm volatile("" ::: "memory");
       }
-      const __amdgpu_buffer_rsrc_t from = box_rsrc(r.box[k & 1]);
-      const __amdgpu_buffer_rsrc_t to = box_rsrc(r.box[(k & 1) ^ 1]);
-      const double dVD = c.diffuse(t, from, V, v.scale);
-      if (v.check_range) {
-         const bool out = live && (V > v.vm_max || V < v.vm_min);
-         const uint64_t m = __ballot(out);
-         if (m) range_report(a.ranges + sl, m, lane, loop, cell, V, dVR, dVD);
-      }
-      double iStim = 0.0;
-      for (uint32_t m = tile_stim; m; m &= m - 1) {
+   }
+   // after the tile's Vm stores of step k
+   __device__ __forceinline__ void done(const ResidentArgs &r, const ResidentTile &t, int k)
+   {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (t.lane == 0)
+         __hip_atomic_store(r.flags + kFlagStride * t.j, r.base + (uint32_t)k + 1u,
+                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+   }
+};
+
+// The slab's clock and stimuli over the launch's steps, as slab_advance and
+// slab_stim keep them from step to step.
+struct ResidentClock {
+   double time;
+   int loop;
+   uint32_t stim;               // the stimuli that reach any cell of the tile
+   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t)
+   {
+      time = t.S->time[a.parity];
+      loop = t.S->loop[a.parity];
+      stim = 0;
+      for (int q = 0; q < kSlabStim; q++)
+         if (__ballot((t.meta >> (16 + q)) & 1u)) stim |= 1u << q;
+   }
+   __device__ __forceinline__ double iStim(const ResidentTile &t) const
+   {
+      double s = 0.0;
+      for (uint32_t m = stim; m; m &= m - 1) {
          const int q = __builtin_ctz(m);
          const PulseDev p{t.S->stim[q].t0, t.S->stim[q].tf, t.S->stim[q].period,
                           t.S->stim[q].phase, t.S->stim[q].duration, t.S->stim[q].amplitude};
          const double val = pulse_value(p, time);
          // later stimuli overwrite earlier ones where they are on
-         if (((meta >> (16 + q)) & 1u) && val != 0.0) iStim = val;
+         if (((t.meta >> (16 + q)) & 1u) && val != 0.0) s = val;
       }
-      const double Vn = V + a.dt * (dVR + dVD + iStim);
-      c.finish(a, T, dVD, iStim);
-      v.time1 = time + a.dt;
-      v.first_eval = loop == sensor_start;
-      if (live) box_store_agent(Vn, to, t.b8, t.S->soff[0]);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (lane == 0)
-         __hip_atomic_store(r.flags + kFlagStride * j, r.base + (uint32_t)k + 1u, __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
+      return s;
+   }
+   __device__ __forceinline__ void advance(double dt)
+   {
+      time = time + dt;
+      ++loop;
+   }
+};
+
+// The sensors of a step (engine_sensors), with APD90's phase and largest Vm
+// in registers between the steps.
+struct ResidentSensors {
+   int phase = 0;
+   double vmax = 0.0, vrest = 0.0;
+   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t)
+   {
+      if (a.sensors & 2) {
+         const uint32_t i = t.cell();
+         phase = a.apd_phase[i];
+         vmax = a.vmax[i];
+         vrest = t.params(a)->Vm0;
+      }
+   }
+   // Vm before and after the step that begins at clock c
+   __device__ __forceinline__ void eval(const EngineArgs &a, const ResidentTile &t,
+                                        const ResidentClock &c, double V, double Vn)
+   {
+      SlabView v{};
+      v.time1 = c.time + a.dt;
+      v.first_eval = c.loop == t.S->sensor_start;
+      v.threshold = t.S->threshold;
+      const uint32_t i = t.cell();
+      EngineArgs as = a;
+      as.sensors = a.sensors & 1;
       uint32_t ev = 0;
-      if (live && a.sensors) ev = engine_sensors(as, v, cell, V, Vn, 0.0);
+      if (t.live && a.sensors) ev = engine_sensors(as, v, i, V, Vn, 0.0);
       if (a.sensors & 2) {
          // apd_eval on the registers
-         if (apd_phase == 0) {
-            if (ev & (kEvTactPacked)) {
-               apd_phase = 1;
-               apd_vmax = Vn;
+         if (phase == 0) {
+            if (ev & kEvTactPacked) {
+               phase = 1;
+               vmax = Vn;
             }
-         } else if (apd_phase == 1) {
-            if (Vn > apd_vmax) {
-               apd_vmax = Vn;
-            } else if (Vn < vrest + 0.1 * (apd_vmax - vrest)) {
-               if (live) a.t90[cell] = v.time1;
-               apd_phase = 2;
+         } else if (phase == 1) {
+            if (Vn > vmax) {
+               vmax = Vn;
+            } else if (Vn < vrest + 0.1 * (vmax - vrest)) {
+               if (t.live) a.t90[i] = v.time1;
+               phase = 2;
             }
          }
       }
-      if (a.sensors & 1) sensor_count(a.counts + 4 * sl, ev);
+      if (a.sensors & 1) sensor_count(a.counts + 4 * t.sl, ev);
+   }
+   __device__ __forceinline__ void store(const EngineArgs &a, const ResidentTile &t) const
+   {
+      if ((a.sensors & 2) && t.live) {
+         const uint32_t i = t.cell();
+         a.apd_phase[i] = (uint8_t)phase;
+         a.vmax[i] = vmax;
+      }
+   }
+};
+
+__device__ __forceinline__ void resident_range(const EngineArgs &a, const ResidentTile &t,
+                                               const ResidentClock &c, double V, double dVR,
+                                               double dVD)
+{
+   if (!t.S->check_range) return;
+   const bool out = t.live && (V > t.S->vm_max || V < t.S->vm_min);
+   const uint64_t m = __ballot(out);
+   if (m) range_report(a.ranges + t.sl, m, t.lane, c.loop, t.cell(), V, dVR, dVD);
+}
+
+// The launch's steps of one tile by one wavefront.  C holds the cell's states
+// and weights and gives the reaction, the stencil sum and what follows Vm's
+// update, each as the step kernel of its precision has it.
+template <class C>
+__device__ __forceinline__ void resident_run(const EngineArgs &a, const ResidentArgs &r,
+                                             typename C::Shared *sh)
+{
+   ResidentTile t;
+   if (!t.find(a)) return;
+   C c;
+   c.load(a, t, sh);
+   double V = r.box[0][t.b8 / 8u];
+   const ParamSet *const params = t.params(a);
+   ResidentLinks links;
+   links.load(r, t.j);
+   ResidentClock clock;
+   clock.load(a, t);
+   ResidentSensors sensors;
+   sensors.load(a, t);
+   ModelTables T{constant_ptr(a.K), constant_ptr(a.E), constant_ptr(a.coef)};
+   for (int k = 0; k < r.nsteps; k++) {
+      renew(T);
+      const ParamSet &P = *params;
+      const double dVR = c.react(a, T, P, t.meta, V);
+      links.wait(r, t, k);
+      const double dVD = c.diffuse(t, box_rsrc(r.box[k & 1]), V, t.S->scale);
+      resident_range(a, t, clock, V, dVR, dVD);
+      const double iStim = clock.iStim(t);
+      const double Vn = V + a.dt * (dVR + dVD + iStim);
+      c.finish(a, T, dVD, iStim);
+      if (t.live) box_store_agent(Vn, box_rsrc(r.box[(k & 1) ^ 1]), t.b8, t.S->soff[0]);
+      links.done(r, t, k);
+      sensors.eval(a, t, clock, V, Vn);
       V = Vn;
-      time = v.time1;
-      ++loop;
+      clock.advance(a.dt);
    }
    c.store();
-   if ((a.sensors & 2) && live) {
-      a.apd_phase[i] = (uint8_t)apd_phase;
-      a.vmax[i] = apd_vmax;
+   sensors.store(a, t);
+}
+
+// ---- six wavefronts to a tile
+//
+// With at most four tiles to a CU (1,024 in all) a step is still one
+// wavefront's chain of dependent instructions, at some 7 cycles each.  The
+// gates depend on Vm and themselves alone, and the non-gate update falls into
+// a calcium and a sodium and potassium part that meet in two currents, so the
+// chain is dealt to six wavefronts of a workgroup:
+//   0     sodium and potassium currents; the sums, the stimulus, Vm
+//   1     calcium part
+//   2     Vm's exchange with the neighbouring tiles and the stencil
+//   3..5  four gates each; 4 evaluates the sensors too
+// Each keeps its states in registers.  What others read of them crosses in
+// LDS: gates, Na_i and Ca_i in two copies by step parity, so that the next
+// values are written while the present ones are read.  Two barriers to a
+// step: before the sums, when every part is there, and after Vm.
+//
+// Per step on one MI355X, step kernels, one wavefront to a tile, and this:
+// reference rounding 504 cells 10.1, 6.6 and 2.5 us, 52,500 cells 12.1, 7.0
+// and 5.3 (821 tiles: the kernel of 64 registers), 46,656 cells 11.6 and 4.2;
+// FMA 52,500 cells 11.7 and 4.4; mixed 504 cells 9.1, 5.8 and 2.6, 52,500
+// cells 10.5, 5.8 and 3.6; exact functions 504 cells 11.9, 9.7 and 3.6.
+// Bounded by the exchange of Vm between tiles (a store to its acknowledgement,
+// a flag, a load: some 3,000 cycles) and by the longest part's chain.
+constexpr int kSplitWaves = 6;
+constexpr int kSplitGateWaves = 3;
+
+// gates (S_M .. S_S, from 0) of each gate wavefront: about 310 VALU
+// instructions each with the fits
+constexpr uint32_t split_bits(int a, int b, int c, int d = -1, int e = -1)
+{
+   uint32_t m = (1u << (a - S_M)) | (1u << (b - S_M)) | (1u << (c - S_M));
+   if (d >= 0) m |= 1u << (d - S_M);
+   if (e >= 0) m |= 1u << (e - S_M);
+   return m;
+}
+constexpr uint32_t kSplitGates[kSplitGateWaves] = {split_bits(S_M, S_H, S_F),
+                                                   split_bits(S_J, S_XR1, S_XR2, S_XS, S_R),
+                                                   split_bits(S_D, S_F2, S_JL, S_S)};
+constexpr uint32_t kGatesNaK = 0xFFFu & ~split_bits(S_D, S_F, S_F2);
+constexpr uint32_t kGatesCa = split_bits(S_D, S_F, S_F2);
+
+// all wavefronts of the workgroup: LDS writes before it are there after it
+// (a full __syncthreads would wait for the global stores as well)
+__device__ __forceinline__ void lds_barrier()
+{
+   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+   __builtin_amdgcn_s_barrier();
+   asm volatile("" ::: "memory");
+}
+
+// G: the gates' type, WT the weights' (words of them per cell: NW).  C: see
+// SplitF64 (engine_f64.hip).
+template <class G, class WT, int NW>
+struct SplitShared {
+   WT w[NW][kBlk];
+   G gate[2][12][kBlk];
+   double ca[2][kBlk], na[2][kBlk];
+   double I_sum[kBlk], I_CaL[kBlk], dVD[kBlk], V[kBlk];
+};
+
+template <class C, int W>
+__device__ __forceinline__ void split_gate_wave(const EngineArgs &a, const ResidentArgs &r,
+                                                const ResidentTile &t, ModelTables T,
+                                                typename C::Shared *sh)
+{
+   C c;
+   c.template load_gates<kSplitGates[W]>(a, t);
+   c.template share_gates<kSplitGates[W]>(sh, 0, t.lane);
+   const int s_switch = t.params(a)->s_switch;
+   ResidentClock clock;
+   ResidentSensors sensors;
+   if constexpr (W == 1) {
+      clock.load(a, t);
+      sensors.load(a, t);
+   }
+   lds_barrier();
+   for (int k = 0; k < r.nsteps; k++) {
+      renew(T);
+      const double V = sh->V[t.lane];
+      c.gates(a, T, s_switch, t.meta, V, a.gate_mask & kSplitGates[W]);
+      c.template share_gates<kSplitGates[W]>(sh, (k & 1) ^ 1, t.lane);
+      lds_barrier();
+      lds_barrier();
+      if constexpr (W == 1) {
+         sensors.eval(a, t, clock, V, sh->V[t.lane]);
+         clock.advance(a.dt);
+      }
+   }
+   c.template store_gates<kSplitGates[W]>(t);
+   if constexpr (W == 1) sensors.store(a, t);
+}
+
+template <class C>
+__device__ __forceinline__ void resident_split_run(const EngineArgs &a, const ResidentArgs &r,
+                                                   typename C::Shared *sh)
+{
+   ResidentTile t;
+   if (!t.find(a)) return;      // the whole workgroup: the tile is its tile
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlk);
+   ModelTables T{constant_ptr(a.K), constant_ptr(a.E), constant_ptr(a.coef)};
+   // every branch passes the same barriers: one at the start, two to a step
+   if (wave == 0) {
+      C c;
+      c.load_na_k(a, t);
+      double V = r.box[0][t.b8 / 8u];
+      sh->V[t.lane] = V;
+      c.share_na(sh, 0, t.lane);
+      const ParamSet *const params = t.params(a);
+      ResidentClock clock;
+      clock.load(a, t);
+      lds_barrier();
+      for (int k = 0; k < r.nsteps; k++) {
+         renew(T);
+         c.na_k(a, T, *params, V, sh, k & 1, t.lane);
+         lds_barrier();
+         const double dVD = sh->dVD[t.lane];
+         const double dVR = c.sum(a, T, sh, t.lane);
+         resident_range(a, t, clock, V, dVR, dVD);
+         const double iStim = clock.iStim(t);
+         V = V + a.dt * (dVR + dVD + iStim);
+         c.finish(a, T, dVD, iStim);
+         sh->V[t.lane] = V;
+         c.share_na(sh, (k & 1) ^ 1, t.lane);
+         lds_barrier();
+         clock.advance(a.dt);
+      }
+      c.store_na_k(t);
+   } else if (wave == 1) {
+      C c;
+      c.load_ca(a, t);
+      c.share_ca(sh, 0, t.lane);
+      const ParamSet *const params = t.params(a);
+      lds_barrier();
+      for (int k = 0; k < r.nsteps; k++) {
+         renew(T);
+         c.calcium(a, T, *params, sh->V[t.lane], sh, k & 1, t.lane);
+         c.share_ca(sh, (k & 1) ^ 1, t.lane);
+         lds_barrier();
+         lds_barrier();
+      }
+      c.store_ca(t);
+   } else if (wave == 2) {
+      C c;
+      c.load_weights(a, t, sh);
+      ResidentLinks links;
+      links.load(r, t.j);
+      lds_barrier();
+      for (int k = 0; k < r.nsteps; k++) {
+         const double V = sh->V[t.lane];
+         links.wait(r, t, k);
+         sh->dVD[t.lane] = c.diffuse(t, box_rsrc(r.box[k & 1]), V, t.S->scale, sh);
+         lds_barrier();
+         lds_barrier();
+         const double Vn = sh->V[t.lane];
+         if (t.live) box_store_agent(Vn, box_rsrc(r.box[(k & 1) ^ 1]), t.b8, t.S->soff[0]);
+         links.done(r, t, k);
+      }
+   } else if (wave == 3) {
+      split_gate_wave<C, 0>(a, r, t, T, sh);
+   } else if (wave == 4) {
+      split_gate_wave<C, 1>(a, r, t, T, sh);
+   } else {
+      split_gate_wave<C, 2>(a, r, t, T, sh);
    }
 }
 

@@ -80,28 +80,33 @@ __device__ __forceinline__ float gateM(C coef, C expc, double V, float g)
 
 __device__ __forceinline__ double sigmM(double x) { return ratio(x, 1.0 + x); }
 
-// Non-gate update.  s32/s64 are the cell's states; dK0 is the rest K_i of its
-// cell type.  Returns dVdt = -Iion and the potassium current iK (the
-// caller finishes the K_i update, which needs the step's diffusion and
-// stimulus currents).
-template <class KT, class C>
-__device__ __forceinline__ double nongateM(const KT &K, const ParamSet &P, C coef, double dt,
-                                           double Vm, const double K_i, float *s32, double *s64, double *iK_out)
+// Non-gate update, in the parts of nongate_core64 (tt06_f64.hpp).  s32/s64 are
+// the cell's states.
+__device__ __forceinline__ double exchangerM(double Na_i, double Ca_i, double fv1, double fv2)
 {
-   const double fv0 = fitM<0>(coef, Vm), fv1 = fitM<1>(coef, Vm), fv2 = fitM<2>(coef, Vm);
-   const double fv3 = fitM<3>(coef, Vm), fv4 = fitM<4>(coef, Vm), fv5 = fitM<5>(coef, Vm);
-   const double Na_i = s64[M_NA_I], Ca_i = s64[M_CA_I];
+   return (Na_i * Na_i * Na_i) * fv1 - Ca_i * fv2;
+}
+
+// The calcium part's currents; I_CaL as its last product's two factors, whose
+// product enters dVdt in one fused multiply-add.
+struct CalciumCurrentsM {
+   double I_sum, CaL_a, CaL_b;
+};
+
+template <class KT>
+__device__ __forceinline__ CalciumCurrentsM calciumM(const KT &K, const ParamSet &P, double dt,
+                                                     double Vm, double fv3, double fv4,
+                                                     double I_NaCa, float *s32, double *s64)
+{
+   const double Ca_i = s64[M_CA_I];
    const double Ca_ss = s32[M_CA_SS], Ca_SR = s32[M_CA_SR];
    const double fCass = s32[M_FCASS], R_prime = s32[M_R_PRIME];
    const double dtc9 = dt * K.c9;
-
-   // calcium
    const double x1 = Ca_i * K.c26;
    const double a2 = Ca_i * K.c27, x2 = a2 * a2;
    const double a3 = Ca_i * K.c28 + K.c29, x3 = a3 * a3;
    const double sg1 = sigmM(x1), sg2 = sigmM(x2), sg3 = sigmM(x3);
    const double dV3 = Vm - 0.5 * K.c3 * log32(Ca_i) - K.c8;
-   const double I_NaCa = (Na_i * Na_i * Na_i) * fv1 - Ca_i * fv2;
    const double I_bCa = K.c7 * dV3;
    const double I_pCa = K.c24 * sg1;
    const double I_up = K.c44 * sg2;
@@ -110,9 +115,37 @@ __device__ __forceinline__ double nongateM(const KT &K, const ParamSet &P, C coe
    const double I_delta = I_leak - I_up;
    const double I_sum = I_bCa + I_pCa;
    s64[M_CA_I] = Ca_i + dtc9 * (sg3 * (0.5 * I_sum - I_NaCa + I_xfer * K.c15 + I_delta * K.c16));
-   double dVR = -I_sum;
+   // Ca_ss, Ca_SR, R', fCass
+   const double a4 = Ca_SR * K.c30, x4 = a4 * a4;
+   const double a5 = Ca_SR * K.c31 + K.c32, x5 = a5 * a5;
+   const double a6 = Ca_ss * K.c33 + K.c34, x6 = a6 * a6;
+   const double sg4 = sigmM(x4), sg5 = sigmM(x5), sg6 = sigmM(x6);
+   const double tmp8 = K.c18 + K.c19 * sg4;
+   const double tmp9 = tmp8 * Ca_ss + K.c36;
+   const double CaL_a = P.c_CaL * (double)s32[M_D] * (double)s32[M_F] * (double)s32[M_F2] * fCass;
+   const double CaL_b = fv4 - Ca_ss * fv3;
+   const double I_CaL = CaL_a * CaL_b;
+   const double css2 = Ca_ss * Ca_ss;
+   const double O = ratio(css2 * R_prime, tmp8 * K.c17 + css2);
+   const double I_rel = K.c40 * O * (Ca_SR - Ca_ss);
+   s32[M_CA_SS] = (float)(Ca_ss + dtc9 * sg6 * (I_xfer + I_rel * K.c14 + I_CaL * K.c13));
+   s32[M_CA_SR] = (float)(Ca_SR - dtc9 * sg5 * (I_delta + I_rel));
+   s32[M_R_PRIME] = (float)(R_prime + dtc9 * (K.c36 - tmp9 * R_prime));
+   const double z = 20 * Ca_ss;
+   const float t1 = rcp32((float)(1.0 + z * z));
+   const float mhu = 0.6f * t1 + 0.4f;
+   const float tauR = rcp32(80.0f * t1 + 2.0f);
+   s32[M_FCASS] = (float)(fCass + dt * (mhu - fCass) * tauR);
+   return CalciumCurrentsM{I_sum, CaL_a, CaL_b};
+}
 
-   // potassium and sodium
+template <class KT, class C>
+__device__ __forceinline__ SodiumPotassiumCurrents na_kM(const KT &K, const ParamSet &P, C coef,
+                                                         double Vm, double K_i, double fv0,
+                                                         double fv5, double I_NaCa,
+                                                         const float *s32, const double *s64)
+{
+   const double Na_i = s64[M_NA_I];
    const double lK = log32(K_i);
    const double dV0 = Vm - K.c3 * lK - K.c5;
    const double dV1 = Vm - K.c3 * log32(Na_i) - K.c4;
@@ -130,34 +163,38 @@ __device__ __forceinline__ double nongateM(const KT &K, const ParamSet &P, C coe
    const double I_bNa = K.c21 * dV1;
    const double xs = s32[M_XS];
    const double I_Ks = P.g_Ks * (xs * xs) * dV2;
-   const double iNa = 3 * I_NaCa - 1.5 * I_NaK + I_Na + I_bNa + I_NaL;
-   const double iK = I_Ks + I_NaK + I_pK + I_K1 + I_to + I_Kr;
-   dVR -= iNa + iK - 2.0 * I_NaCa;
-   s64[M_NA_I] = Na_i + dtc9 * iNa;
+   return SodiumPotassiumCurrents{3 * I_NaCa - 1.5 * I_NaK + I_Na + I_bNa + I_NaL,
+                                  I_Ks + I_NaK + I_pK + I_K1 + I_to + I_Kr};
+}
 
-   // Ca_ss, Ca_SR, R', fCass
-   const double a4 = Ca_SR * K.c30, x4 = a4 * a4;
-   const double a5 = Ca_SR * K.c31 + K.c32, x5 = a5 * a5;
-   const double a6 = Ca_ss * K.c33 + K.c34, x6 = a6 * a6;
-   const double sg4 = sigmM(x4), sg5 = sigmM(x5), sg6 = sigmM(x6);
-   const double tmp8 = K.c18 + K.c19 * sg4;
-   const double tmp9 = tmp8 * Ca_ss + K.c36;
-   const double I_CaL = P.c_CaL * (double)s32[M_D] * (double)s32[M_F] * (double)s32[M_F2] * fCass *
-                        (fv4 - Ca_ss * fv3);
-   const double css2 = Ca_ss * Ca_ss;
-   const double O = ratio(css2 * R_prime, tmp8 * K.c17 + css2);
-   const double I_rel = K.c40 * O * (Ca_SR - Ca_ss);
-   s32[M_CA_SS] = (float)(Ca_ss + dtc9 * sg6 * (I_xfer + I_rel * K.c14 + I_CaL * K.c13));
-   s32[M_CA_SR] = (float)(Ca_SR - dtc9 * sg5 * (I_delta + I_rel));
-   s32[M_R_PRIME] = (float)(R_prime + dtc9 * (K.c36 - tmp9 * R_prime));
-   const double z = 20 * Ca_ss;
-   const float t1 = rcp32((float)(1.0 + z * z));
-   const float mhu = 0.6f * t1 + 0.4f;
-   const float tauR = rcp32(80.0f * t1 + 2.0f);
-   s32[M_FCASS] = (float)(fCass + dt * (mhu - fCass) * tauR);
-   dVR += I_CaL;
-   *iK_out = iK;
-   return dVR;
+// dVdt = -Iion and the Na_i update
+template <class KT>
+__device__ __forceinline__ double sumM(const KT &K, double dt, double I_NaCa,
+                                       const CalciumCurrentsM &ca,
+                                       const SodiumPotassiumCurrents &nk, double *s64)
+{
+   const double dtc9 = dt * K.c9;
+   double dVR = -ca.I_sum;
+   dVR -= nk.iNa + nk.iK - 2.0 * I_NaCa;
+   s64[M_NA_I] = s64[M_NA_I] + dtc9 * nk.iNa;
+   return __builtin_fma(ca.CaL_a, ca.CaL_b, dVR);
+}
+
+// The whole of it.  Returns dVdt = -Iion and the potassium current iK (the
+// caller finishes the K_i update, which needs the step's diffusion and
+// stimulus currents).
+template <class KT, class C>
+__device__ __forceinline__ double nongateM(const KT &K, const ParamSet &P, C coef, double dt,
+                                           double Vm, const double K_i, float *s32, double *s64,
+                                           double *iK_out)
+{
+   const double fv0 = fitM<0>(coef, Vm), fv1 = fitM<1>(coef, Vm), fv2 = fitM<2>(coef, Vm);
+   const double fv3 = fitM<3>(coef, Vm), fv4 = fitM<4>(coef, Vm), fv5 = fitM<5>(coef, Vm);
+   const double I_NaCa = exchangerM(s64[M_NA_I], s64[M_CA_I], fv1, fv2);
+   const CalciumCurrentsM ca = calciumM(K, P, dt, Vm, fv3, fv4, I_NaCa, s32, s64);
+   const SodiumPotassiumCurrents nk = na_kM(K, P, coef, Vm, K_i, fv0, fv5, I_NaCa, s32, s64);
+   *iK_out = nk.iK;
+   return sumM(K, dt, I_NaCa, ca, nk, s64);
 }
 
 template <class C>

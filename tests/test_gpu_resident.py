@@ -1,7 +1,7 @@
 """The resident kernels (csrc/engine_resident.hpp) against the step kernels,
 bit for bit: Vm, states, activation and APD90 times, counts, range record and
 clock.  A launch chosen with set_launch runs the step kernels; the default
-runs of 16 steps and more are resident where the tiles fit the chip (3,072
+runs of 8 steps and more are resident where the tiles fit the chip (3,072
 tiles, for the fits also 4,096 at four wavefronts per SIMD; mixed 4,096)."""
 import numpy as np
 import pytest
@@ -78,7 +78,7 @@ def test_small_slabs_equal_the_step_kernels(mode, exact, dims, holes):
     chunks too short for the resident form in between, and more steps than
     one launch takes."""
     s = slab(*dims, holes=holes, vm_max=20.0)
-    out = compare([s], mode, (17, 3, 16, 301), exact)
+    out = compare([s], mode, (17, 3, 8, 301), exact)
     assert np.ptp(out[0]) >= 0 and np.isfinite(out[0]).all()
 
 
@@ -90,6 +90,17 @@ def test_tiles_at_the_edges_of_what_the_chip_holds(mode, ntile):
     first that does not."""
     compare([slab(ntile // 64 if ntile % 64 == 0 else ntile, 64 if ntile % 64 == 0 else 8,
                   64 if ntile % 64 == 0 else 8)], mode, (40,))
+
+
+@pytest.mark.parametrize("mode,exact", KINDS)
+@pytest.mark.parametrize("ntile", [767, 769, 1024, 1025])
+def test_tiles_at_the_edges_of_six_wavefronts_to_a_tile(mode, exact, ntile):
+    """The last tiles that fit six wavefronts each (768 at 80 registers, 1,024
+    at 64), and the first that do not; the last tile ragged."""
+    nz = 64 * ntile // 32
+    compare([slab(4, 8, nz, holes=0.0)], mode, (16, 31), exact)
+    a = slab(2, 16, nz + 1 if ntile % 2 else nz - 1)
+    compare([a], mode, (33,), exact)
 
 
 @pytest.mark.parametrize("mode", ["fp64_fma", "mixed_fused"])
