@@ -355,22 +355,6 @@ __device__ __forceinline__ void resident_run(const EngineArgs &a, const Resident
 // Bounded by the exchange of Vm between tiles (a store to its acknowledgement,
 // a flag, a load: some 3,000 cycles) and by the longest part's chain.
 constexpr int kSplitWaves = 6;
-constexpr int kSplitGateWaves = 3;
-
-// gates (S_M .. S_S, from 0) of each gate wavefront: about 310 VALU
-// instructions each with the fits
-constexpr uint32_t split_bits(int a, int b, int c, int d = -1, int e = -1)
-{
-   uint32_t m = (1u << (a - S_M)) | (1u << (b - S_M)) | (1u << (c - S_M));
-   if (d >= 0) m |= 1u << (d - S_M);
-   if (e >= 0) m |= 1u << (e - S_M);
-   return m;
-}
-constexpr uint32_t kSplitGates[kSplitGateWaves] = {split_bits(S_M, S_H, S_F),
-                                                   split_bits(S_J, S_XR1, S_XR2, S_XS, S_R),
-                                                   split_bits(S_D, S_F2, S_JL, S_S)};
-constexpr uint32_t kGatesNaK = 0xFFFu & ~split_bits(S_D, S_F, S_F2);
-constexpr uint32_t kGatesCa = split_bits(S_D, S_F, S_F2);
 
 // all wavefronts of the workgroup: LDS writes before it are there after it
 // (a full __syncthreads would wait for the global stores as well)

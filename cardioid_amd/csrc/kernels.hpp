@@ -219,8 +219,13 @@ __device__ __forceinline__ void range_report(RangeRec *r, uint64_t mask, int lan
    }
 }
 
+// wavefronts to a tile of k_tt06_calc_split_f64
+constexpr int kCalcSplitWaves = 5;
+
 // kernels (kernels_f64.hip)
 __global__ void k_tt06_calc_pipe_f64(ReactionArgs a);
+template <bool EXACT>
+__global__ void k_tt06_calc_split_f64(ReactionArgs a);
 __global__ void k_tt06_gate_f64(ReactionArgs a);
 __global__ void k_tt06_calc_exact_f64(ReactionArgs a);
 __global__ void k_tt06_gate_exact_f64(ReactionArgs a);

@@ -122,6 +122,120 @@ __global__ __launch_bounds__(256, 3) void k_tt06_calc_pipe_f64(ReactionArgs a)
              a.gate_mask);
 }
 
+// TT06Dev_Reaction::calc with a tile's work dealt to five wavefronts of a
+// workgroup, for objects of few tiles.  There a call is bound by one
+// wavefront's dependent chain, some 1,700 VALU instructions (3,300 with the
+// exact functions) at about 7 cycles each; here the longest of the five has
+// about 400:
+//   wave 0     sodium and potassium currents, the sums, dVm
+//   wave 1     calcium part
+//   wave 2..4  gates (kSplitGates)
+// Waves 0 and 1 read gates that the others advance: every wavefront stores
+// after the one barrier, behind which all have read what they need.  The
+// expressions are those of the other kernels, the results the same bit for
+// bit.  With more tiles the five wavefronts of each only take each other's
+// place: see kSplitTiles (plugins.hip) for where that begins.
+namespace {
+
+template <bool EXACT, uint32_t GATES>
+__device__ __forceinline__ void calc_split_gates(const ReactionArgs &a, int i, bool live, double V,
+                                                 double *sp)
+{
+   double st[N_STATE];
+#pragma unroll
+   for (int q = S_M; q < N_STATE; q++)
+      if ((GATES >> (q - S_M)) & 1) st[q] = sp[kBlk * q];
+   const int s_switch = a.params[0].s_switch;
+   const uint8_t fl = a.flags[i];
+   const uint32_t mask = a.gate_mask & GATES;
+   if constexpr (EXACT) {
+      if (!(fl & kFlagGatesFixed))
+         gates_exact64(*constant_ptr(a.E), s_switch, a.dt, V, st, mask);
+   } else {
+      gates64(constant_ptr(a.coef), constant_ptr(a.K)->exp_coef, s_switch, fl, V, st, mask);
+   }
+   __syncthreads();
+   if (!live) return;
+#pragma unroll
+   for (int q = S_M; q < N_STATE; q++)
+      if ((GATES >> (q - S_M)) & 1) sp[kBlk * q] = st[q];
+}
+
+}  // namespace
+
+template <bool EXACT>
+__global__ __launch_bounds__(kCalcSplitWaves * 64) void k_tt06_calc_split_f64(ReactionArgs a)
+{
+   __shared__ double xc[2][kBlk];     // I_sum, I_CaL
+   const int lane = threadIdx.x & (kBlk - 1);
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlk);
+   // states and flags are padded to a whole tile; lanes past n take the first
+   // cell's Vm and store nothing
+   const int i = blockIdx.x * kBlk + lane;
+   const bool live = i < a.n;
+   const int e = live ? (a.index ? a.index[i] : i) : 0;
+   const double V = live ? a.Vm[e] : a.Vm[a.index ? a.index[0] : 0];
+   double *sp = a.state + blk_base(i, N_STATE);
+   ModelConst *K = constant_ptr(a.K);
+   const ParamSet &P = a.params[0];
+   double st[N_STATE];
+   auto voltage_fns = [&](auto &&f) {
+      if constexpr (EXACT) f(exact_voltage_fns(constant_ptr(a.E), K));
+      else f(fit_voltage_fns<false>(constant_ptr(a.coef)));
+   };
+   if (wave == 0) {
+#pragma unroll
+      for (int q = 0; q < N_STATE; q++)
+         if (q == S_DVK_I || q == S_NA_I || q == S_CA_I ||
+             (q >= S_M && ((kGatesNaK >> (q - S_M)) & 1)))
+            st[q] = sp[kBlk * q];
+      double fv[6], I_NaCa = 0.0;
+      SodiumPotassiumCurrents nk{};
+      voltage_fns([&](const auto &fvs) {
+         fvs.fv05(V, fv);
+         I_NaCa = exchanger64(st[S_NA_I], st[S_CA_I], fv[1], fv[2]);
+         nk = nongate_na_k64(*K, P, fvs, V, fv[0], fv[5], I_NaCa, st);
+      });
+      __syncthreads();
+      const double dVR =
+          nongate_sum64(*K, a.dt, I_NaCa, CalciumCurrents{xc[0][lane], xc[1][lane]}, nk, st);
+      if (live) {
+         sp[kBlk * S_DVK_I] = st[S_DVK_I];
+         sp[kBlk * S_NA_I] = st[S_NA_I];
+         a.dVm[e] = dVR;
+      }
+   } else if (wave == 1) {
+#pragma unroll
+      for (int q = 0; q < N_STATE; q++)
+         if (q == S_NA_I || (q < S_M && q != S_DVK_I) ||
+             (q >= S_M && ((kGatesCa >> (q - S_M)) & 1)))
+            st[q] = sp[kBlk * q];
+      voltage_fns([&](const auto &fvs) {
+         double fv[6];
+         fvs.fv05(V, fv);
+         const double I_NaCa = exchanger64(st[S_NA_I], st[S_CA_I], fv[1], fv[2]);
+         const CalciumCurrents ca = nongate_calcium64(*K, P, a.dt, V, fv[3], fv[4], I_NaCa, st);
+         xc[0][lane] = ca.I_sum;
+         xc[1][lane] = ca.I_CaL;
+      });
+      __syncthreads();
+      if (live) {
+#pragma unroll
+         for (int q = 0; q < S_M; q++)
+            if (q != S_DVK_I && q != S_NA_I) sp[kBlk * q] = st[q];
+      }
+   } else if (wave == 2) {
+      calc_split_gates<EXACT, kSplitGates[0]>(a, i, live, V, sp);
+   } else if (wave == 3) {
+      calc_split_gates<EXACT, kSplitGates[1]>(a, i, live, V, sp);
+   } else {
+      calc_split_gates<EXACT, kSplitGates[2]>(a, i, live, V, sp);
+   }
+}
+
+template __global__ void k_tt06_calc_split_f64<false>(ReactionArgs);
+template __global__ void k_tt06_calc_split_f64<true>(ReactionArgs);
+
 // Gate update only (Reaction::updateGate of the pdr loop): the 12 gates at Vm.
 __global__ __launch_bounds__(256) void k_tt06_gate_f64(ReactionArgs a)
 {

@@ -112,11 +112,23 @@ void scatter(int64_t n, const uint32_t *bi, const double *src, double *box, hipS
    CDH_LAUNCH_CHECK();
 }
 
-// The reaction over the object's n cells: configuration A's kernel, or the
-// pipelined kernel of configuration B on its resident grid.
+// Tiles up to which five wavefronts to a tile are the faster form, with the
+// fits and with the exact functions (one MI355X, us a call, one wavefront to
+// a tile and five: fits 500 cells 11.1 and 4.6, 32,768 cells 11.7 and 5.8,
+// 98,304 cells 13.7 and 12.2, 131,072 cells 14.6 and 15.4; exact functions 500
+// cells 11.6 and 5.8, 49,152 cells 13.2 and 10.7, 65,536 cells 13.8 and 13.9).
+constexpr int64_t kSplitTiles = 1536, kSplitTilesExact = 896;
+
+// The reaction over the object's n cells: five wavefronts to a tile where
+// there are few tiles; else configuration A's kernel, or the pipelined kernel
+// of configuration B on its resident grid.
 void launch_calc(cdh_tt06 *r, const ReactionArgs &a, hipStream_t s)
 {
-   if (r->exact) {
+   const int64_t ntile = ((int64_t)a.n + kBlk - 1) / kBlk;
+   if (ntile <= (r->exact ? kSplitTilesExact : kSplitTiles)) {
+      hipLaunchKernelGGL(r->exact ? k_tt06_calc_split_f64<true> : k_tt06_calc_split_f64<false>,
+                         dim3((unsigned)ntile), dim3(kCalcSplitWaves * kBlk), 0, s, a);
+   } else if (r->exact) {
       hipLaunchKernelGGL(k_tt06_calc_exact_f64, dim3(grid_for(a.n, kBlock)), dim3(kBlock), 0, s,
                          a);
    } else {

@@ -301,4 +301,23 @@ __device__ __forceinline__ void gates64(C coef, C expc, int s_switch, uint8_t fl
    }
 }
 
+// A cell's update dealt to several wavefronts (engine_resident.hpp,
+// k_tt06_calc_split_f64): the gates (S_M .. S_S, from 0) of each of three
+// gate wavefronts, about 310 VALU instructions each with the fits, and the
+// gates that the sodium and potassium part and the calcium part read.
+constexpr int kSplitGateWaves = 3;
+
+constexpr uint32_t split_bits(int a, int b, int c, int d = -1, int e = -1)
+{
+   uint32_t m = (1u << (a - S_M)) | (1u << (b - S_M)) | (1u << (c - S_M));
+   if (d >= 0) m |= 1u << (d - S_M);
+   if (e >= 0) m |= 1u << (e - S_M);
+   return m;
+}
+constexpr uint32_t kSplitGates[kSplitGateWaves] = {split_bits(S_M, S_H, S_F),
+                                                   split_bits(S_J, S_XR1, S_XR2, S_XS, S_R),
+                                                   split_bits(S_D, S_F2, S_JL, S_S)};
+constexpr uint32_t kGatesNaK = 0xFFFu & ~split_bits(S_D, S_F, S_F2);
+constexpr uint32_t kGatesCa = split_bits(S_D, S_F, S_F2);
+
 }  // namespace cdh
