@@ -132,14 +132,30 @@ __global__ __launch_bounds__(64) void k_tile_links(EngineArgs a, uint32_t *links
 }
 
 // The slabs' clocks after `nsteps` resident steps from parity p, as
-// slab_advance moves them step by step.
-__global__ __launch_bounds__(64) void k_slab_clock(SlabDev *slabs, int nslab, int p, int nsteps,
-                                                   double dt)
+// slab_advance moves them step by step, and the range record of a slab that
+// has out-of-range cells and none yet: the earliest step's of its tiles'.
+__global__ __launch_bounds__(64) void k_slab_clock(EngineArgs a, ResidentArgs r, int nslab)
 {
 #pragma clang fp contract(off)
    const int k = blockIdx.x * 64 + threadIdx.x;
-   if (k >= nslab || !slabs[k].active) return;
-   SlabDev &S = slabs[k];
+   if (k >= nslab || !a.slabs[k].active) return;
+   SlabDev &S = a.slabs[k];
+   const int p = a.parity, nsteps = r.nsteps;
+   const double dt = a.dt;
+   RangeRec &rec = a.ranges[k];
+   if (rec.count && !rec.taken)
+      for (int j = 0; j < a.ntile; j++) {
+         const RangeRec &t = a.ranges[r.tile_ranges + j];
+         if (!t.count || t.taken != (int32_t)r.base) continue;
+         if (a.blk_slab[a.tiles ? (int)a.tiles[j] : a.tile_base + j] != k) continue;
+         if (rec.taken && rec.loop <= t.loop) continue;
+         rec.taken = 1;
+         rec.loop = t.loop;
+         rec.cell = t.cell;
+         rec.V = t.V;
+         rec.dVmR = t.dVmR;
+         rec.dVmD = t.dVmD;
+      }
    const int q = (p + nsteps) & 1;
    double t = S.time[p];
    const int loop = S.loop[p] + nsteps;
@@ -193,8 +209,8 @@ KernelFn kernel_for(int mode, bool exact, int waves)
 int min_waves(int mode) { return mode == CDH_MODE_MIXED_FUSED ? 3 : 2; }
 int max_waves(int mode) { return mode == CDH_MODE_MIXED_FUSED ? 4 : 3; }
 
-// Results in the caller's cell order, rows of n doubles: out[c] of a row is
-// the value of the slab's cell inv[c].  The gather is what reading costs the
+// Results in the caller's cell order, rows of n doubles (a piece of one row
+// where it is long): out[c] of a row is the value of the slab's cell inv[c].  The gather is what reading costs the
 // device (about 0.1 ms for 5 million cells); the host then takes the rows
 // into the caller's array without passes of its own.  blockIdx.y: the row.
 __device__ __forceinline__ int64_t row_cell(const RowArgs &r)
@@ -208,14 +224,15 @@ __global__ __launch_bounds__(256) void k_rows_vm(RowArgs r, const uint32_t *bi, 
    if (c < r.n) r.out[c] = box[bi[r.inv[c]]];
 }
 
-// up to three columns (the launch takes the ones that are asked for)
+// up to three columns
 struct Columns {
    const double *col[3];
 };
 __global__ __launch_bounds__(256) void k_rows_col(RowArgs r, Columns cols)
 {
    const int64_t c = row_cell(r);
-   const double *col = blockIdx.y == 0 ? cols.col[0] : blockIdx.y == 1 ? cols.col[1] : cols.col[2];
+   const int q = r.row0 + blockIdx.y;
+   const double *col = q == 0 ? cols.col[0] : q == 1 ? cols.col[1] : cols.col[2];
    if (c < r.n) r.out[blockIdx.y * r.n + c] = col[r.inv[c]];
 }
 
@@ -545,7 +562,7 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
    CDH_HIP(hipMemset(blk_slab_.p, 0xFF, ntile * sizeof(uint16_t)));
    track(slabdev_, cap_slabs);
    slabdev_.zero();
-   track(ranges_, cap_slabs);
+   track(ranges_, cap_slabs + (size_t)resident_tiles_);
    ranges_.zero();
    track(counts_, 4 * (size_t)cap_slabs);
    counts_.zero();
@@ -973,6 +990,7 @@ int Engine::run_resident(int nsteps)
       r.box[0] = box_[parity_].p;
       r.box[1] = box_[parity_ ^ 1].p;
       r.failed = failed_;
+      r.tile_ranges = (int)(ranges_.n - (size_t)resident_tiles_);
       void *kargs[2] = {&a, &r};
       if (hipLaunchCooperativeKernel((const void *)kernel.fn, dim3(8 * a.groups_per_xcd),
                                      dim3(kernel.threads), kargs, 0, stream_) != hipSuccess) {
@@ -981,7 +999,7 @@ int Engine::run_resident(int nsteps)
          return nsteps;
       }
       hipLaunchKernelGGL(k_slab_clock, dim3((unsigned)((slabs_.size() + 63) / 64)), dim3(64), 0,
-                         stream_, slabdev_.p, (int)slabs_.size(), parity_, n, dt_);
+                         stream_, a, r, (int)slabs_.size());
       CDH_LAUNCH_CHECK();
       epoch_ += (uint32_t)n;
       parity_ ^= n & 1;
@@ -1141,10 +1159,18 @@ std::vector<double> Engine::vm(int id)
 
 // ---- results in the caller's order
 
-// The rows' arguments: the slab's place of each of the caller's cells, on
-// the device from the first read on, and room for as many of `rows` rows as
-// one launch may gather (all of them while they are short).
-RowArgs Engine::row_args(int id, int rows)
+// Rows of a slab's results into the caller's arrays: `gather` launches the
+// kernel that puts `rows` rows from row `row` on into RowArgs::out; host[q] is
+// where row q goes.  What one launch may gather is bounded (kReadRoom), so
+// that reading needs the same few MiB on the device for every slab.
+//
+// Short rows are gathered together and go straight to one array.  Longer ones
+// take two pinned pieces in turn: the next piece crosses the bus while
+// several threads move the last one into the caller's pages, which a fresh
+// array has yet to be given (three rows of 4.9 million cells into new arrays:
+// 11.7 ms straight, 7.3 ms this way; one into an array in use 2.3 and 1.1 ms).
+template <class F>
+void Engine::read_rows(int id, int rows, double *const *host, F &&gather)
 {
    Slab &s = slabs_[id];
    uint32_t *order = bi_.p + tiles_.capacity() * kBlk + s.tile0 * kBlk;
@@ -1154,51 +1180,69 @@ RowArgs Engine::row_args(int id, int rows)
       put(order, inv);
       s.order_up = true;
    }
-   const int64_t room = s.n * rows <= kReadPiece ? s.n * rows : s.n;
+   const int64_t n = s.n;
+   const int64_t room = std::min(n * rows <= kReadPiece ? n * rows : n, kReadRoom);
    if ((int64_t)row_.n < room) {
       bytes_ -= (int64_t)(row_.n * sizeof(double));
       track(row_, room);
    }
-   return RowArgs{s.n, s.ntile * kBlk, order, row_.p, 0};
-}
-
-// The row into the caller's array.  Short rows go straight there.  Longer
-// ones take two pinned pieces in turn: the next piece crosses the bus while
-// several threads move the last one into the caller's pages, which a fresh
-// array has yet to be given (three rows of 4.9 million cells into new arrays:
-// 11.7 ms straight, 7.3 ms this way; one into an array in use 2.3 and 1.1 ms).
-void Engine::copy_row(int64_t n, double *host)
-{
-   CDH_LAUNCH_CHECK();
-   if (n < 2 * kReadPiece) {
-      CDH_HIP(hipMemcpyAsync(host, row_.p, n * sizeof(double), hipMemcpyDeviceToHost, stream_));
+   RowArgs r{n, s.ntile * kBlk, order, row_.p, 0};
+   auto launch = [&](int count, int64_t cells) {
+      gather(dim3((unsigned)((cells + 255) / 256), count), r);
+      CDH_LAUNCH_CHECK();
+   };
+   auto fetch = [&](double *to, int64_t from, int64_t count) {
+      CDH_HIP(hipMemcpyAsync(to, row_.p + from, count * sizeof(double), hipMemcpyDeviceToHost,
+                             stream_));
+   };
+   if (n * rows <= kReadPiece) {
+      launch(rows, n);
+      bool together = true;
+      for (int q = 1; q < rows; q++) together = together && host[q] == host[0] + q * n;
+      if (together) fetch(host[0], 0, rows * n);
+      else for (int q = 0; q < rows; q++) fetch(host[q], q * n, n);
       CDH_HIP(hipStreamSynchronize(stream_));
       return;
    }
-   for (int k = 0; k < 2; k++)
+   const bool straight = n < 2 * kReadPiece;
+   for (int k = 0; k < 2 && !straight; k++)
       if (!read_piece_[k]) {
          CDH_HIP(hipHostMalloc((void **)&read_piece_[k], kReadPiece * sizeof(double),
                                hipHostMallocDefault));
          CDH_HIP(hipEventCreateWithFlags(&read_ev_[k], hipEventDisableTiming));
       }
-   const int64_t pieces = (n + kReadPiece - 1) / kReadPiece;
-   auto length = [&](int64_t p) { return std::min<int64_t>(kReadPiece, n - p * kReadPiece); };
-   auto fetch = [&](int64_t p) {
-      CDH_HIP(hipMemcpyAsync(read_piece_[p & 1], row_.p + p * kReadPiece,
-                             length(p) * sizeof(double), hipMemcpyDeviceToHost, stream_));
-      CDH_HIP(hipEventRecord(read_ev_[p & 1], stream_));
-   };
-   fetch(0);
-   for (int64_t p = 0; p < pieces; p++) {
-      if (p + 1 < pieces) fetch(p + 1);
-      CDH_HIP(hipEventSynchronize(read_ev_[p & 1]));
-      const char *from = (const char *)read_piece_[p & 1];
-      char *to = (char *)(host + p * kReadPiece);
-      const int64_t bytes = length(p) * (int64_t)sizeof(double);
+   for (r.row0 = 0; r.row0 < rows; r.row0++) {
+      if (straight) {
+         launch(1, n);
+         fetch(host[r.row0], 0, n);
+         CDH_HIP(hipStreamSynchronize(stream_));
+         continue;
+      }
+      const int64_t pieces = (n + kReadPiece - 1) / kReadPiece;
+      auto length = [&](int64_t p) { return std::min<int64_t>(kReadPiece, n - p * kReadPiece); };
+      auto start = [&](int64_t p) {
+         const int64_t c = p * kReadPiece, at = c % kReadRoom;
+         if (at == 0) {
+            const int64_t cells = std::min(kReadRoom, n - c);
+            r.n = cells;
+            r.inv = order + c;
+            launch(1, cells);
+         }
+         fetch(read_piece_[p & 1], at, length(p));
+         CDH_HIP(hipEventRecord(read_ev_[p & 1], stream_));
+      };
+      start(0);
+      for (int64_t p = 0; p < pieces; p++) {
+         if (p + 1 < pieces) start(p + 1);
+         CDH_HIP(hipEventSynchronize(read_ev_[p & 1]));
+         const char *from = (const char *)read_piece_[p & 1];
+         char *to = (char *)(host[r.row0] + p * kReadPiece);
+         const int64_t bytes = length(p) * (int64_t)sizeof(double);
 #pragma omp parallel for schedule(static) num_threads(kReadThreads)
-      for (int k = 0; k < kReadThreads; k++) {
-         const int64_t a = bytes * k / kReadThreads, b = bytes * (k + 1) / kReadThreads;
-         std::memcpy(to + a, from + a, b - a);
+         for (int k = 0; k < kReadThreads; k++) {
+            const int64_t a = bytes * k / kReadThreads, b = bytes * (k + 1) / kReadThreads;
+            std::memcpy(to + a, from + a, b - a);
+         }
       }
    }
 }
@@ -1208,10 +1252,10 @@ void Engine::read_vm(int id, double *host)
    check_slab(id);
    sync();
    const Slab &s = slabs_[id];
-   const RowArgs r = row_args(id, 1);
-   hipLaunchKernelGGL(k_rows_vm, dim3((unsigned)((s.n + 255) / 256)), dim3(256), 0, stream_, r,
-                      bi_.p + s.tile0 * kBlk, box_[parity_].p);
-   copy_row(s.n, host);
+   read_rows(id, 1, &host, [&](dim3 grid, const RowArgs &r) {
+      hipLaunchKernelGGL(k_rows_vm, grid, dim3(256), 0, stream_, r, bi_.p + s.tile0 * kBlk,
+                         box_[parity_].p);
+   });
 }
 
 void Engine::read_state(int id, double *host)
@@ -1219,19 +1263,18 @@ void Engine::read_state(int id, double *host)
    check_slab(id);
    sync();
    const Slab &s = slabs_[id];
-   const int64_t c0 = s.tile0 * kBlk, n = s.n;
-   RowArgs r = row_args(id, N_STATE);
-   const int rows = n * N_STATE <= kReadPiece ? N_STATE : 1;
-   const dim3 grid((unsigned)((n + 255) / 256), rows), blk(256);
-   for (r.row0 = 0; r.row0 < N_STATE; r.row0 += rows) {
+   const int64_t c0 = s.tile0 * kBlk;
+   double *row[N_STATE];
+   for (int q = 0; q < N_STATE; q++) row[q] = host + q * s.n;
+   read_rows(id, N_STATE, row, [&](dim3 grid, const RowArgs &r) {
       if (mode_ != CDH_MODE_MIXED_FUSED)
-         hipLaunchKernelGGL(k_rows_state64, grid, blk, 0, stream_, r, state_.p + c0 * N_STATE);
+         hipLaunchKernelGGL(k_rows_state64, grid, dim3(256), 0, stream_, r,
+                            state_.p + c0 * N_STATE);
       else
-         hipLaunchKernelGGL(k_rows_mixed, grid, blk, 0, stream_, r, st32_.p + c0 * kMixed32,
+         hipLaunchKernelGGL(k_rows_mixed, grid, dim3(256), 0, stream_, r, st32_.p + c0 * kMixed32,
                             st64_.p + c0 * 2, meta_.p + c0, psets_.p + s.param0, K_.c9,
                             bi_.p + c0, box_[parity_].p);
-      copy_row(rows * n, host + r.row0 * n);
-   }
+   });
 }
 
 // the columns (per-cell arrays of the arena) whose host array is given
@@ -1247,20 +1290,9 @@ void Engine::read_cols(int id, int ncol, const double *const *arena, double *con
          to[m++] = host[q];
       }
    if (m == 0) return;
-   const RowArgs r = row_args(id, m);
-   const dim3 blk(256);
-   const unsigned g = (unsigned)((s.n + 255) / 256);
-   if (s.n * m <= kReadPiece) {
-      hipLaunchKernelGGL(k_rows_col, dim3(g, m), blk, 0, stream_, r, c);
-      std::vector<double> all(s.n * m);
-      copy_row(s.n * m, all.data());
-      for (int q = 0; q < m; q++) std::memcpy(to[q], &all[q * s.n], s.n * sizeof(double));
-      return;
-   }
-   for (int q = 0; q < m; q++) {
-      hipLaunchKernelGGL(k_rows_col, dim3(g), blk, 0, stream_, r, Columns{{c.col[q]}});
-      copy_row(s.n, to[q]);
-   }
+   read_rows(id, m, to, [&](dim3 grid, const RowArgs &r) {
+      hipLaunchKernelGGL(k_rows_col, grid, dim3(256), 0, stream_, r, c);
+   });
 }
 
 void Engine::read_activation(int id, double *tact0, double *tact, double *trec)

@@ -48,7 +48,7 @@ struct LaunchCfg {
 
 // rows of a slab's results in the caller's cell order
 struct RowArgs {
-   int64_t n, S;                // cells, and the slab's cells in whole tiles
+   int64_t n, S;                // cells of a row, and the slab's cells in whole tiles
    const uint32_t *inv;         // per cell of the caller's order, its place in the slab
    double *out;
    int row0;                    // the number of the first row of a launch
@@ -147,8 +147,8 @@ class Engine {
 
  private:
    void step_eager();
-   RowArgs row_args(int id, int rows);
-   void copy_row(int64_t n, double *host);
+   template <class F>
+   void read_rows(int id, int rows, double *const *host, F &&gather);
    void read_cols(int id, int ncol, const double *const *arena, double *const *host);
    bool resident_fits() const;
    int run_resident(int nsteps);
@@ -246,8 +246,9 @@ class Engine {
    DevBuf<double> coef_;
    DevBuf<ParamSet> psets_;
    DevBuf<uint32_t> meta_, bi_;
-   DevBuf<double> row_;            // rows of results, as long as the longest read yet
+   DevBuf<double> row_;            // rows of results, at most kReadRoom
    static constexpr int64_t kReadPiece = int64_t(1) << 18;   // doubles (2 MiB)
+   static constexpr int64_t kReadRoom = 8 * kReadPiece;         // 16 MiB: a launch to 8 pieces
    static constexpr int kReadThreads = 8;
    double *read_piece_[2] = {nullptr, nullptr};              // pinned
    hipEvent_t read_ev_[2] = {nullptr, nullptr};
@@ -259,7 +260,7 @@ class Engine {
    DevBuf<double> box_[2];
    DevBuf<double> tact0_, tact_, trec_, vmax_, t90_;
    DevBuf<uint8_t> apd_phase_;
-   DevBuf<RangeRec> ranges_;
+   DevBuf<RangeRec> ranges_;       // per slab, and behind them per resident tile
    DevBuf<uint32_t> counts_;      // per slab: recorded tact0, tact, trec, (unused)
    int exact_ = 0;                 // configuration A
    DevBuf<TT06ExactConst> dE_;     // its constants

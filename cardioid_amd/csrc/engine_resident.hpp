@@ -69,6 +69,7 @@ struct ResidentArgs {
    int nsteps;
    double *box[2];              // box[k & 1] is read in step k of this launch
    uint32_t *failed;            // host memory; 1 once a wait has passed its bound
+   int tile_ranges;             // the tiles' range records in EngineArgs::ranges (resident_range)
 };
 
 typedef const SlabDev CDH_CONSTANT ConstSlab;
@@ -281,14 +282,24 @@ struct ResidentSensors {
    }
 };
 
-__device__ __forceinline__ void resident_range(const EngineArgs &a, const ResidentTile &t,
-                                               const ResidentClock &c, double V, double dVR,
-                                               double dVD)
+// The range check of a step (engine_range).  The tiles are at different steps,
+// so the slab's record cannot be the first one that comes: each tile keeps
+// the first of its own in this launch (count 1, taken the launch's base)
+// behind the slabs' records, and k_slab_clock gives the slab the one of the
+// earliest step.
+__device__ __forceinline__ void resident_range(const EngineArgs &a, const ResidentArgs &r,
+                                               const ResidentTile &t, const ResidentClock &c,
+                                               double V, double dVR, double dVD)
 {
    if (!t.S->check_range) return;
    const bool out = t.live && (V > t.S->vm_max || V < t.S->vm_min);
    const uint64_t m = __ballot(out);
-   if (m) range_report(a.ranges + t.sl, m, t.lane, c.loop, t.cell(), V, dVR, dVD);
+   if (__builtin_expect(m != 0, 0) && t.lane == __builtin_ctzll(m)) {
+      atomicAdd(&a.ranges[t.sl].count, (unsigned long long)__builtin_popcountll(m));
+      RangeRec &f = a.ranges[r.tile_ranges + t.j];
+      if (!f.count || f.taken != (int32_t)r.base)
+         f = RangeRec{1ull, (int32_t)r.base, c.loop, (int64_t)t.cell(), V, dVR, dVD};
+   }
 }
 
 // The launch's steps of one tile by one wavefront.  C holds the cell's states
@@ -317,7 +328,7 @@ __device__ __forceinline__ void resident_run(const EngineArgs &a, const Resident
       const double dVR = c.react(a, T, P, t.meta, V);
       links.wait(r, t, k);
       const double dVD = c.diffuse(t, box_rsrc(r.box[k & 1]), V, t.S->scale);
-      resident_range(a, t, clock, V, dVR, dVD);
+      resident_range(a, r, t, clock, V, dVR, dVD);
       const double iStim = clock.iStim(t);
       const double Vn = V + a.dt * (dVR + dVD + iStim);
       c.finish(a, T, dVD, iStim);
@@ -432,7 +443,7 @@ __device__ __forceinline__ void resident_split_run(const EngineArgs &a, const Re
          lds_barrier();
          const double dVD = sh->dVD[t.lane];
          const double dVR = c.sum(a, T, sh, t.lane);
-         resident_range(a, t, clock, V, dVR, dVD);
+         resident_range(a, r, t, clock, V, dVR, dVD);
          const double iStim = clock.iStim(t);
          V = V + a.dt * (dVR + dVD + iStim);
          c.finish(a, T, dVD, iStim);

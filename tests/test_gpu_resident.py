@@ -173,3 +173,51 @@ def test_results_come_in_the_callers_order(mode, dims):
         assert np.array_equal(first[0][p], second[0])
     for x, y in zip(first, second):
         assert np.array_equal(x[..., p], y)
+
+
+@pytest.mark.parametrize("mode,nz", [("fp64_fused", 1400), ("fp64_fma", 4000), ("mixed_fused", 4000)])
+def test_range_record_is_the_earliest_steps(mode, nz):
+    """Cells leave the range at six places along a slab, each a step later
+    than the last, in an order unlike the tiles': the record is the first
+    step's, and the next record that of the steps after the first is read."""
+    nx, ny = 4, 8
+    a = W.fibre_slab(nx, ny, nz, 0.0)
+    z = [nz * f // 16 for f in (9, 3, 14, 1, 12, 6)]
+    st = [W.box_stimulus(zMin=p, zMax=p + 4, nx=nx, ny=ny, nz=nz, tStart=1.0 + k * DT,
+                         duration=0.5, vStim=-45.0) for k, p in enumerate(z)]
+    s = hip.Slab(a, ["midCellML"], W.DIFFUSION_SCALE, st, vm_max=-84.0)
+    got = []
+    for chosen in (False, True):
+        b = make([s], mode, chosen)
+        i = b.add(s)
+        b.run(80)
+        first = b.range_report(i)
+        b.run(30)
+        got.append((first, b.range_report(i)))
+        b.close()
+    for r, want in zip(*got):
+        assert r["count"] == want["count"] and r["loop"] == want["loop"]
+        assert r["V"] > -84.0
+    first, cell = got[0][0], got[0][0]["cell"]
+    assert z[0] < cell // (nx * ny) < z[0] + 4, first
+
+
+def test_results_of_a_slab_longer_than_one_gather():
+    """Rows of more cells than one gather takes (2,097,152), in the caller's
+    (shuffled) order.  The exact functions: their gates do not depend on a
+    cell's place, as the fits' loop bounds do."""
+    nx, ny, nz = 128, 128, 130
+    a = W.fibre_slab(nx, ny, nz, 10.0)
+    order = np.random.default_rng(3).permutation(a.ncell)
+    b = W.Anatomy(nx, ny, nz, a.dx, a.dy, a.dz, a.gid[order], a.celltype[order], a.sigma[order])
+    got = []
+    for an in (a, b):
+        st = [W.box_stimulus(xMax=4, nx=nx, ny=ny, nz=nz)]
+        sim = hip.Simulation(an, ["endoCellML"], DT, W.DIFFUSION_SCALE, st, mode="fp64_fused", sensors=3,
+                             exact_functions=True, jhTauSmooth=1)
+        sim.run(60)
+        got.append([sim.vm(), *sim.activation(), sim.t90(), *sim.state()])
+        sim.close()
+    for x, y in zip(*got):
+        assert np.array_equal(x[order], y)
+    assert np.unique(got[0][0]).size > 4
