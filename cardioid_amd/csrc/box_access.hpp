@@ -64,7 +64,11 @@ __device__ __forceinline__ void stream_store_f64(double v, __amdgpu_buffer_rsrc_
    typedef unsigned int u32x2 __attribute__((__vector_size__(2 * sizeof(unsigned int))));
    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, kNT);
 }
-// two adjacent FP64 fields of a cell (a pair of run_pair_index), 16 bytes
+// Two adjacent FP64 fields of a cell (a pair of run_pair_index), 16 bytes.
+// The store is followed by a wait state in which its registers stay as they
+// are: a 16-byte store still reads them one cycle after it issued, and the
+// compiler leaves that cycle out where the offset is an SGPR.  A v_mov right
+// behind such a store changed the low words of what sixteen lanes stored.
 __device__ __forceinline__ void stream_load_f64x2(__amdgpu_buffer_rsrc_t r, uint32_t voff,
                                                   uint32_t soff, double &a, double &b)
 {
@@ -85,6 +89,7 @@ __device__ __forceinline__ void stream_store_f64x2(double a, double b, __amdgpu_
    v[2] = (uint32_t)ub;
    v[3] = (uint32_t)(ub >> 32);
    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, kNT);
+   asm volatile("s_nop 0" : : "v"(v));
 }
 __device__ __forceinline__ float stream_load_f32(__amdgpu_buffer_rsrc_t r, uint32_t voff,
                                                  uint32_t soff)
