@@ -30,10 +30,8 @@ struct ReactionArgs {
    const double *Vm;
    double *dVm;
    double dt;
-   uint32_t gate_mask;          // bits 0..12 set; see gates64 and k_tt06_calc_pipe_f64
+   uint32_t gate_mask;          // bits 0..12 set; see gates64 and k_tt06_calc_f64
    const TT06ExactConst *E;     // configuration A (exact functions) constants, or null
-   double *sink;                // 20 x 64 doubles: the pipelined kernel's stores of
-                                // lanes past n (k_tt06_calc_pipe_f64)
 };
 
 struct StencilArgs {
@@ -223,11 +221,11 @@ __device__ __forceinline__ void range_report(RangeRec *r, uint64_t mask, int lan
 constexpr int kCalcSplitWaves = 5;
 
 // kernels (kernels_f64.hip)
-__global__ void k_tt06_calc_pipe_f64(ReactionArgs a);
+template <bool EXACT>
+__global__ void k_tt06_calc_f64(ReactionArgs a);
 template <bool EXACT>
 __global__ void k_tt06_calc_split_f64(ReactionArgs a);
 __global__ void k_tt06_gate_f64(ReactionArgs a);
-__global__ void k_tt06_calc_exact_f64(ReactionArgs a);
 __global__ void k_tt06_gate_exact_f64(ReactionArgs a);
 __global__ void k_scatter_f64(int n, const uint32_t *bi, const double *src, double *box);
 __global__ void k_scatter4_f64(int n, const uint32_t *bi, const double *src, double *box);

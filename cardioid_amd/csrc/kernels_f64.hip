@@ -3,9 +3,9 @@
 // Compiled with -ffp-contract=off: every kernel here reproduces the
 // reference CPU path's rounding, operation by operation.
 //
-//   k_tt06_calc_pipe_f64  TT06Dev_Reaction::calc        elec/TT06Dev_Reaction.cc:393-407
-//   k_tt06_calc_exact_f64  the same in configuration A (exact functions,
-//                       generic gates)                  elec/TT06Func.cc:64-161
+//   k_tt06_calc_f64, k_tt06_calc_split_f64  TT06Dev_Reaction::calc
+//                       elec/TT06Dev_Reaction.cc:393-407; configuration A
+//                       (exact functions, generic gates) elec/TT06Func.cc:64-161
 //   k_scatter_f64       FGRDiffusionOMP::updateLocalVoltage  elec/FGRDiffusionOMP.cc:75-89
 //   k_fgr_calc_f64      FGRDiffusionOMP::calc           elec/FGRDiffusionOMP.cc:109-131
 //   k_integrate_f64     Vm += dt*(dVmR+dVmD+iStim)      elec/simulationLoop.cc:221-227
@@ -25,102 +25,80 @@ namespace cdh {
 // field q of cell i at blk_index(q, i, nq), a wavefront's fields one
 // contiguous run.
 //
-// TT06Dev_Reaction::calc, software pipelined.  The grid holds only as many
-// wavefronts as are resident at once (G); wavefront w walks the tiles
-// w, w + G, w + 2G, ... and issues the loads of its next tile (its 19
-// states, gate flags and Vm, and the index of the tile after) before the
-// arithmetic of the current one, so that its memory traffic runs under its
-// own arithmetic rather than only under other wavefronts'.  The loads are
-// unconditional (past the last tile the current one is read again and the
-// values dropped), which keeps the compiler's wait for the current tile's
-// data from also waiting on the next tile's.  The stores are unconditional
-// too: lanes past n (the last tile's padding; their states are padded to a
-// whole tile, and they read Vm[0]) store into the object's 20 x 64-double
-// sink instead of its states and dVm.  A store block skipped under a lane
-// mask would make the compiler's waits assume no stores were issued and
-// wait for every store before touching the next tile.  One parameter set
-// per object (pid is not used).  Against one tile per wavefront with
-// every load up front (4 waves/SIMD at 108 VGPRs), this form (3 waves/SIMD)
-// took the reference-structured step on the 20.1 M-cell shell from 2.28 to
-// 2.10 ms on one MI355X, bit for bit the same states, Vm and activation.
+// TT06Dev_Reaction::calc, one tile to a wavefront, a wavefront to a
+// workgroup.  A call reads its states first and computes after, and what
+// fills the one phase with the other is wavefronts that are not in step: four
+// to a SIMD (at most 128 VGPRs), each its own workgroup, so that the next tile
+// begins when one ends and not when four have.  Workgroups of four wavefronts
+// and a persistent grid of 3 wavefronts per SIMD, each with its next tile's
+// loads in flight, kept them in step; us a call on one MI355X, persistent and
+// this: fits 131,072 cells 14.3 and 12.8, 300,007 cells 26.6 and 24.4,
+// 600,000 cells 50.0 and 44.1, 6.7 million cells 491 and 450 (4.8 TB/s);
+// exact functions, in workgroups of four and this: 300,007 cells 40.3 and
+// 37.3, 600,000 cells 71 and 67, 6.7 million cells 694 and 676.  3 and 5
+// wavefronts per SIMD are within 1 % of 4; streaming (nontemporal) states
+// beat cached ones by 3 % and more.  Bounded by VALU issue with the states'
+// bytes close behind.
 //
-// The body takes its arrays as restrict-qualified arguments: the stores of
-// one tile then provably leave the constants and fit coefficients alone,
-// and the next tile's reads of those stay scalar loads instead of vector
-// loads that would wait on every outstanding access.
+// EXACT: configuration A, the non-gate update with the exact fv0..fv6, then
+// the generic gate update with the exact steady states and rates, at the
+// step's Vm.  Gate flags bit 0 holds every gate of a cell (the pdr loop's
+// updateNonGate); the generic loop has no v2 loop bounds, so otherwise every
+// cell's gates advance.
+//
+// The body takes its arrays as restrict-qualified arguments: the stores then
+// provably leave the constants and fit coefficients alone, and their reads
+// stay scalar loads.  One parameter set per object (pid is not used).
 namespace {
 
-__device__ __forceinline__ void calc_pipe(const TT06Const *__restrict__ K,
+template <bool EXACT>
+__device__ __forceinline__ void calc_tile(const TT06Const *__restrict__ K,
+                                          const TT06ExactConst *__restrict__ E,
                                           const double *__restrict__ coef,
                                           const ParamSet *__restrict__ params,
                                           const uint8_t *__restrict__ flags,
                                           double *__restrict__ state, const int *__restrict__ index,
                                           const double *__restrict__ Vm, double *__restrict__ dVm,
-                                          double *__restrict__ sink, int n, double dt,
-                                          uint32_t gate_mask)
+                                          int n, double dt, uint32_t gate_mask)
 {
-   const int lane = threadIdx.x & 63;
-   const int G = __builtin_amdgcn_readfirstlane(gridDim.x * (blockDim.x >> 6));
-   const int ntile = (n + kBlk - 1) / kBlk;
-   int t = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-   if (t >= ntile) return;
+   // states and flags are padded to a whole tile; lanes past n take Vm[0] and
+   // store nothing
+   const int i = blockIdx.x * kBlk + threadIdx.x;
+   const bool live = i < n;
+   const int e = live ? (index ? index[i] : i) : 0;
+   const double V = Vm[e];
+   const uint8_t fl = flags[i];
+   double *sp = state + blk_base(i, N_STATE);
+   double st[N_STATE];
+#pragma unroll
+   for (int s = 0; s < N_STATE; s++) st[s] = __builtin_nontemporal_load(sp + kBlk * s);
    const ParamSet P = params[0];
-   auto cell_index = [&](int tt) -> int {
-      const int i = tt * kBlk + lane;
-      return i < n ? (index ? index[i] : i) : 0;
-   };
-   auto load_states = [&](int tt, double *st) {
-      const double *sp = state + blk_base((int64_t)tt * kBlk + lane, N_STATE);
-#pragma unroll
-      for (int s = 0; s < N_STATE; s++) st[s] = __builtin_nontemporal_load(sp + kBlk * s);
-   };
-   // this tile's data, and the next tile's index
-   int e = cell_index(t);
-   int tn = t + G < ntile ? t + G : t;
-   int en = cell_index(tn);
-   double V = Vm[e];
-   uint8_t fl = flags[t * kBlk + lane];
-   double sa[N_STATE], sb[N_STATE];
-   load_states(t, sa);
-   // One tile: the next tile's loads into nxt (and the index of the one
-   // after), then the arithmetic and stores of the current tile, held in
-   // cur.  Returns false after the last tile.  The loop alternates the two
-   // state buffers rather than copying one into the other.
-   auto tile = [&](double *cur, double *nxt) -> bool {
-      const int tnn = tn + G < ntile ? tn + G : tn;
-      const int enn = cell_index(tnn);
-      const double Vn = Vm[en];
-      const uint8_t fln = flags[tn * kBlk + lane];
-      load_states(tn, nxt);
-      double dVR = 0.0;
-      if (gate_mask & (1u << 12)) dVR = nongate64(*K, P, coef, dt, V, cur);
-      gates64(coef, K->exp_coef, P.s_switch, fl, V, cur, gate_mask);
-      const int i = t * kBlk + lane;
-      const bool live = i < n;
-      double *sp = live ? state + blk_base(i, N_STATE) : sink + lane;
-#pragma unroll
-      for (int s = 0; s < N_STATE; s++) __builtin_nontemporal_store(cur[s], sp + kBlk * s);
-      *(live ? dVm + e : sink + kBlk * N_STATE + lane) = dVR;
-      if (tn == t) return false;
-      t = tn;
-      tn = tnn;
-      e = en;
-      en = enn;
-      V = Vn;
-      fl = fln;
-      return true;
-   };
-   while (tile(sa, sb) && tile(sb, sa)) {
+   double dVR = 0.0;
+   if constexpr (EXACT) {
+      if (gate_mask & (1u << 12))
+         dVR = nongate_core64(*K, P, exact_voltage_fns(E, K), dt, V, st);
+      if (!(fl & kFlagGatesFixed)) gates_exact64(*E, P.s_switch, dt, V, st, gate_mask);
+   } else {
+      if (gate_mask & (1u << 12)) dVR = nongate64(*K, P, coef, dt, V, st);
+      gates64(coef, K->exp_coef, P.s_switch, fl, V, st, gate_mask);
    }
+   if (!live) return;
+#pragma unroll
+   for (int s = 0; s < N_STATE; s++) __builtin_nontemporal_store(st[s], sp + kBlk * s);
+   dVm[e] = dVR;
 }
 
 }  // namespace
 
-__global__ __launch_bounds__(256, 3) void k_tt06_calc_pipe_f64(ReactionArgs a)
+template <bool EXACT>
+__global__ __launch_bounds__(kBlk, 4) void k_tt06_calc_f64(ReactionArgs a)
 {
-   calc_pipe(a.K, a.coef, a.params, a.flags, a.state, a.index, a.Vm, a.dVm, a.sink, a.n, a.dt,
-             a.gate_mask);
+   calc_tile<EXACT>(a.K, a.E, a.coef, a.params, a.flags, a.state, a.index, a.Vm, a.dVm, a.n, a.dt,
+                    a.gate_mask);
 }
+
+template __global__ void k_tt06_calc_f64<false>(ReactionArgs);
+template __global__ void k_tt06_calc_f64<true>(ReactionArgs);
 
 // TT06Dev_Reaction::calc with a tile's work dealt to five wavefronts of a
 // workgroup, for objects of few tiles.  There a call is bound by one
@@ -250,29 +228,6 @@ __global__ __launch_bounds__(256) void k_tt06_gate_f64(ReactionArgs a)
    gates64(a.coef, a.K->exp_coef, P.s_switch, a.flags[i], V, st, a.gate_mask);
 #pragma unroll
    for (int s = S_M; s < N_STATE; s++) a.state[blk_index(s, i, N_STATE)] = st[s];
-}
-
-// Configuration A: the non-gate update with the exact fv0..fv6, then the
-// generic gate update with the exact steady states and rates, at the
-// step's Vm.  Gate flags bit 0 holds every gate of a cell (the pdr loop's
-// updateNonGate); the generic loop has no v2 loop bounds, so otherwise every
-// cell's gates advance.
-__global__ __launch_bounds__(256) void k_tt06_calc_exact_f64(ReactionArgs a)
-{
-   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= a.n) return;
-   const int e = a.index ? a.index[i] : i;
-   const double V = a.Vm[e];
-   double st[N_STATE];
-#pragma unroll
-   for (int s = 0; s < N_STATE; s++) st[s] = a.state[blk_index(s, i, N_STATE)];
-   const ParamSet P = a.params[0];
-   double dVR = 0.0;
-   if (a.gate_mask & (1u << 12)) dVR = nongate_core64(*a.K, P, exact_voltage_fns(a.E, a.K), a.dt, V, st);
-   if (!(a.flags[i] & kFlagGatesFixed)) gates_exact64(*a.E, P.s_switch, a.dt, V, st, a.gate_mask);
-#pragma unroll
-   for (int s = 0; s < N_STATE; s++) a.state[blk_index(s, i, N_STATE)] = st[s];
-   if (a.dVm) a.dVm[e] = dVR;
 }
 
 // Configuration A gate update only (Reaction::updateGate of the pdr loop).

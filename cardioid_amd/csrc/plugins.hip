@@ -41,8 +41,6 @@ struct TT06Reaction {
    DevBuf<uint8_t> flags;
    DevBuf<double> state;
    DevBuf<uint8_t> flagsAllFixed;   // gates skipped (updateNonGate-only launches)
-   int64_t pipe_blocks = 0;         // resident workgroups of k_tt06_calc_pipe_f64
-   DevBuf<double> sink;             // its stores of lanes past n (20 x 64 doubles)
 };
 
 }  // namespace cdh
@@ -93,7 +91,6 @@ ReactionArgs reaction_args(cdh_tt06 *r, double dt, const int *index, int n, cons
    a.dt = dt;
    a.gate_mask = 0x1FFFu;
    a.E = r->exact ? r->Ed.p : nullptr;
-   a.sink = r->sink.p;
    return a;
 }
 
@@ -114,29 +111,22 @@ void scatter(int64_t n, const uint32_t *bi, const double *src, double *box, hipS
 
 // Tiles up to which five wavefronts to a tile are the faster form, with the
 // fits and with the exact functions (one MI355X, us a call, one wavefront to
-// a tile and five: fits 500 cells 11.1 and 4.6, 32,768 cells 11.7 and 5.8,
-// 98,304 cells 13.7 and 12.2, 131,072 cells 14.6 and 15.4; exact functions 500
-// cells 11.6 and 5.8, 49,152 cells 13.2 and 10.7, 65,536 cells 13.8 and 13.9).
-constexpr int64_t kSplitTiles = 1536, kSplitTilesExact = 896;
+// a tile and five: fits 500 cells 8.6 and 4.6, 65,536 cells 10.9 and 8.5,
+// 81,920 cells 11.2 and 9.7, 90,112 cells 11.7 and 11.5, 98,304 cells 11.8 and
+// 12.1; exact functions 32,768 cells 11.6 and 8.5, 65,536 cells 12.3 and 13.2).
+constexpr int64_t kSplitTiles = 1408, kSplitTilesExact = 896;
 
 // The reaction over the object's n cells: five wavefronts to a tile where
-// there are few tiles; else configuration A's kernel, or the pipelined kernel
-// of configuration B on its resident grid.
+// there are few tiles, else one.
 void launch_calc(cdh_tt06 *r, const ReactionArgs &a, hipStream_t s)
 {
    const int64_t ntile = ((int64_t)a.n + kBlk - 1) / kBlk;
-   if (ntile <= (r->exact ? kSplitTilesExact : kSplitTiles)) {
+   if (ntile <= (r->exact ? kSplitTilesExact : kSplitTiles))
       hipLaunchKernelGGL(r->exact ? k_tt06_calc_split_f64<true> : k_tt06_calc_split_f64<false>,
                          dim3((unsigned)ntile), dim3(kCalcSplitWaves * kBlk), 0, s, a);
-   } else if (r->exact) {
-      hipLaunchKernelGGL(k_tt06_calc_exact_f64, dim3(grid_for(a.n, kBlock)), dim3(kBlock), 0, s,
-                         a);
-   } else {
-      const int64_t tiles = ((int64_t)a.n + kBlk - 1) / kBlk;
-      const int64_t blocks = std::min<int64_t>((tiles + kBlock / 64 - 1) / (kBlock / 64),
-                                               r->pipe_blocks);
-      hipLaunchKernelGGL(k_tt06_calc_pipe_f64, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
-   }
+   else
+      hipLaunchKernelGGL(r->exact ? k_tt06_calc_f64<true> : k_tt06_calc_f64<false>,
+                         dim3((unsigned)ntile), dim3(kBlk), 0, s, a);
    CDH_LAUNCH_CHECK();
 }
 
@@ -218,17 +208,6 @@ int cdh_tt06_create(const cdh_tt06_params *p, int numPoints, cdh_tt06 **out)
          for (int64_t i = 0; i < r->stride; i++) tiled[blk_index(s, i, N_STATE)] = st[s * r->stride + i];
       r->state.alloc(tiled.size());
       r->state.upload(tiled.data(), tiled.size());
-      if (!exact) {
-         // the pipelined kernel's grid: as many workgroups as are resident at once
-         int dev = 0, ncu = 0, per_cu = 0;
-         CDH_HIP(hipGetDevice(&dev));
-         CDH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-         CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tt06_calc_pipe_f64,
-                                                              kBlock, 0));
-         CDH_REQUIRE(ncu > 0 && per_cu > 0, "cdh_tt06_create: no resident workgroups");
-         r->pipe_blocks = (int64_t)ncu * per_cu;
-         r->sink.alloc((N_STATE + 1) * kBlk);
-      }
       *out = r.release();
    });
 }

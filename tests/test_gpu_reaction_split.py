@@ -58,7 +58,7 @@ def calc(n, V, st, exact, index, nongate_only=False):
     return out, got.reshape(19, n)
 
 
-@pytest.mark.parametrize("exact,limit", [(False, 1536), (True, 896)])
+@pytest.mark.parametrize("exact,limit", [(False, 1408), (True, 896)])
 @pytest.mark.parametrize("index", [False, True])
 @pytest.mark.parametrize("nongate_only", [False, True])
 def test_few_tiles_equal_many(exact, limit, index, nongate_only):
