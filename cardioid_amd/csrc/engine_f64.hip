@@ -14,6 +14,8 @@
 // rounds them, so that the fused step equals the unfused loop bit for bit.
 #pragma clang fp contract(off)
 
+#include <utility>
+
 #include "engine.hpp"
 #include "engine_resident.hpp"
 #include "tt06_exact.hpp"
@@ -156,13 +158,38 @@ template __global__ void k_engine_f64<3, kExact>(EngineArgs);
 namespace {
 
 // The 18 weights wait in LDS between the steps' stencils, the states in
-// registers.
-template <int KIND>
+// registers.  At four wavefronts per SIMD (128 VGPRs) the first kParked gates
+// wait in LDS too, from one use to the next: 9.5 KB to a tile, so that 16
+// tiles take the CU's 160 KB.  With all states in registers that kernel
+// spilled 9 of them to scratch: 64^3 cells FMA 16.1 us a step, reference
+// rounding 18.3; now 15.1 and 17.3.
+constexpr int kParked = 10;
+
+template <int KIND, int NPARK>
 struct ResidentF64 {
    struct Shared {
       float w[18][kBlk];
+      double park[NPARK > 0 ? NPARK : 1][kBlk];
    };
    double st[N_STATE];
+   // f(g) for the 12 gates, g a constant
+   template <class F>
+   __device__ __forceinline__ static void each_gate(F &&f)
+   {
+      [&]<int... G>(std::integer_sequence<int, G...>) {
+         (f(std::integral_constant<int, G>{}), ...);
+      }(std::make_integer_sequence<int, N_STATE - S_M>{});
+   }
+   template <class G>
+   __device__ __forceinline__ void fetch(G, int lane)
+   {
+      if constexpr (G::value < NPARK) st[S_M + G::value] = sh->park[G::value][lane];
+   }
+   template <class G>
+   __device__ __forceinline__ void park(G, int lane)
+   {
+      if constexpr (G::value < NPARK) sh->park[G::value][lane] = st[S_M + G::value];
+   }
    Shared *sh;
    __amdgpu_buffer_rsrc_t RS;
    uint32_t lc, rw;
@@ -180,27 +207,46 @@ struct ResidentF64 {
       for (int s = 0; s + 1 < N_STATE; s += 2)
          stream_load_f64x2(RS, 16u * lc, 8u * rw * s, st[s], st[s + 1]);
       st[N_STATE - 1] = stream_load_f64(RS, 8u * lc, 8u * rw * (N_STATE - 1));
+      each_gate([&](auto g) { park(g, t.lane); });
    }
-   __device__ __forceinline__ void store()
+   __device__ __forceinline__ void store(const ResidentTile &t)
    {
+      each_gate([&](auto g) { fetch(g, t.lane); });
 #pragma unroll
       for (int s = 0; s + 1 < N_STATE; s += 2)
          stream_store_f64x2(st[s], st[s + 1], RS, 16u * lc, 8u * rw * s);
       stream_store_f64(st[N_STATE - 1], RS, 8u * lc, 8u * rw * (N_STATE - 1));
    }
    __device__ __forceinline__ double react(const EngineArgs &a, const ModelTables &T,
-                                           const ParamSet &P, uint32_t meta, double V)
+                                           const ParamSet &P, const ResidentTile &t, double V)
    {
+      const uint32_t meta = t.meta;
       double dVR = 0.0;
-      if constexpr (KIND == kExact) {
-         if (a.gate_mask & (1u << 12))
+      each_gate([&](auto g) { fetch(g, t.lane); });
+      if (a.gate_mask & (1u << 12)) {
+         if constexpr (KIND == kExact)
             dVR = nongate_core64<true>(*T.K, P, exact_voltage_fns(T.E, T.K), a.dt, V, st);
-         if (!((meta >> 8) & kFlagGatesFixed))
-            gates_exact64(*T.E, P.s_switch, a.dt, V, st, a.gate_mask);
+         else
+            dVR = nongate64<KIND == kFitsFma, true>(*T.K, P, T.coef, a.dt, V, st);
+      }
+      auto gates = [&](uint32_t mask) {
+         if constexpr (KIND == kExact) {
+            if (!((meta >> 8) & kFlagGatesFixed))
+               gates_exact64(*T.E, P.s_switch, a.dt, V, st, mask);
+         } else {
+            gates64<KIND == kFitsFma>(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(meta >> 8), V,
+                                      st, mask);
+         }
+      };
+      if constexpr (NPARK == 0) {
+         gates(a.gate_mask);
       } else {
-         constexpr bool FMA = KIND == kFitsFma;
-         if (a.gate_mask & (1u << 12)) dVR = nongate64<FMA, true>(*T.K, P, T.coef, a.dt, V, st);
-         gates64<FMA>(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(meta >> 8), V, st, a.gate_mask);
+         each_gate([&](auto g) {
+            asm volatile("" ::: "memory");   // fetched here, not before
+            fetch(g, t.lane);
+            gates(a.gate_mask & (1u << g.value));
+            park(g, t.lane);
+         });
       }
       return dVR;
    }
@@ -393,8 +439,9 @@ struct SplitF64 {
 template <int KIND, int WAVES>
 __global__ __launch_bounds__(64, WAVES) void k_resident_f64(EngineArgs a, ResidentArgs r)
 {
-   __shared__ typename ResidentF64<KIND>::Shared sh;
-   resident_run<ResidentF64<KIND>>(a, r, &sh);
+   using C = ResidentF64<KIND, WAVES == 4 ? kParked : 0>;
+   __shared__ typename C::Shared sh;
+   resident_run<C>(a, r, &sh);
 }
 
 template <int KIND, int WAVES>

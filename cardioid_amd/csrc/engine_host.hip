@@ -172,10 +172,9 @@ __global__ __launch_bounds__(64) void k_slab_clock(EngineArgs a, ResidentArgs r,
 // The resident kernels of a mode, from the one with the fewest tiles on the
 // chip to the one with the most.  Six wavefronts to a tile leave room for
 // four tiles on a CU (1,024 on 256 CUs).  The FP64 kernel holds 3 wavefronts
-// per SIMD (3,072 tiles) without spills; at 4 it spills some 17 registers,
-// which 64^3 cells repay (4,096 tiles: FMA 16.5 us a step against 24.5 by
-// step kernels, reference rounding 18.1 against 24.6) and fewer tiles do not
-// (54x56x64 cells: 13.0 us a step against 11.6 at 3).  The exact functions
+// per SIMD (3,072 tiles) with its states in registers; at 4 most gates wait
+// in LDS (ResidentF64; 4,096 tiles: FMA 15.1 us a step against 24.5 by step
+// kernels, reference rounding 17.3 against 24.6).  The exact functions would
 // spill too much at 4 (39 against 32 us at 64^3 by step kernels).
 struct ResidentKernel {
    void (*fn)(EngineArgs, ResidentArgs);

@@ -201,7 +201,7 @@ struct ResidentMixed {
       ref = (const float CDH_CONSTANT *)(a.Aref + (int64_t)t.blk * 18);
       wscale = t.S->wdelta_scale;
    }
-   __device__ __forceinline__ void store()
+   __device__ __forceinline__ void store(const ResidentTile &)
    {
 #pragma unroll
       for (int s = 0; s < N_STATE32; s++) stream_store_f32(s32[s], R32, 4u * lc, 4u * rw * s);
@@ -209,13 +209,13 @@ struct ResidentMixed {
       for (int s = 0; s < N_STATE64; s++) stream_store_f64(s64[s], R64, 8u * lc, 8u * rw * s);
    }
    __device__ __forceinline__ double react(const EngineArgs &a, const ModelTables &T,
-                                           const ParamSet &P, uint32_t meta, double V)
+                                           const ParamSet &P, const ResidentTile &t, double V)
    {
       const double K_i = P.K0 + (double)s32[M_DK_I];
       double dVR = 0.0;
       iK = 0.0;
       if (a.gate_mask & (1u << 12)) dVR = nongateM(*T.K, P, T.coef, a.dt, V, K_i, s32, s64, &iK);
-      gatesM(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(meta >> 8), V, s32, a.gate_mask);
+      gatesM(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(t.meta >> 8), V, s32, a.gate_mask);
       return dVR;
    }
    // the sums of cell_mixed, in its order

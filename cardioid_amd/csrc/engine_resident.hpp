@@ -38,7 +38,7 @@
 // Per step on one MI355X, step kernels against this: reference rounding
 // 504 cells 10.1 and 6.7 us, 52,500 cells 12.2 and 7.0, 110,592 cells 14.5
 // and 9.7, 193,536 cells 18.9 and 12.9; FMA 262,144 cells (4 wavefronts per
-// SIMD) 24.5 and 16.5; mixed 52,500 cells 10.6 and 5.9, 262,144 cells 15.4
+// SIMD) 24.5 and 15.1; mixed 52,500 cells 10.6 and 5.9, 262,144 cells 15.4
 // and 10.4; exact functions 52,500 cells 13.5 and 9.7.  What bounds it: up
 // to 1,024 tiles the latency of one wavefront's chain (12,000 of 17,000 cycles
 // in the reaction), with more tiles VALU issue.
@@ -325,7 +325,7 @@ __device__ __forceinline__ void resident_run(const EngineArgs &a, const Resident
    for (int k = 0; k < r.nsteps; k++) {
       renew(T);
       const ParamSet &P = *params;
-      const double dVR = c.react(a, T, P, t.meta, V);
+      const double dVR = c.react(a, T, P, t, V);
       links.wait(r, t, k);
       const double dVD = c.diffuse(t, box_rsrc(r.box[k & 1]), V, t.S->scale);
       resident_range(a, r, t, clock, V, dVR, dVD);
@@ -338,7 +338,7 @@ __device__ __forceinline__ void resident_run(const EngineArgs &a, const Resident
       V = Vn;
       clock.advance(a.dt);
    }
-   c.store();
+   c.store(t);
    sensors.store(a, t);
 }
 
