@@ -111,10 +111,10 @@ void scatter(int64_t n, const uint32_t *bi, const double *src, double *box, hipS
 
 // Tiles up to which five wavefronts to a tile are the faster form, with the
 // fits and with the exact functions (one MI355X, us a call, one wavefront to
-// a tile and five: fits 500 cells 8.6 and 4.6, 65,536 cells 10.9 and 8.5,
-// 81,920 cells 11.2 and 9.7, 90,112 cells 11.7 and 11.5, 98,304 cells 11.8 and
-// 12.1; exact functions 32,768 cells 11.6 and 8.5, 65,536 cells 12.3 and 13.2).
-constexpr int64_t kSplitTiles = 1408, kSplitTilesExact = 896;
+// a tile and five: fits 500 cells 8.6 and 4.7, 81,920 cells 11.0 and 9.4,
+// 98,304 cells 11.3 and 11.0, 106,496 cells 11.4 and 12.0; exact functions
+// 49,152 cells 9.8 and 7.8, 81,920 cells 13.7 and 12.3).
+constexpr int64_t kSplitTiles = 1536, kSplitTilesExact = 1280;
 
 // The reaction over the object's n cells: five wavefronts to a tile where
 // there are few tiles, else one.

@@ -193,6 +193,12 @@ void tt06_exact_constants(TT06ExactConst *e, int mod)
    e->f10 = g_pK;
    bridge(-64.20, -23.3, h_rate, e->hmod);
    bridge(-48.85, -17.6, j_rate, e->jmod);
+   const double ex[14] = {0x1.71547652b82fep+0, -0x1.62e42fefa39efp-1, -0x1.abc9e3b39803fp-56,
+                          0x1.0000000000000p-1, 0x1.5555555555557p-3, 0x1.5555555555556p-5,
+                          0x1.11111111100cep-7, 0x1.6c16c16c162ccp-10, 0x1.a01a01abef415p-13,
+                          0x1.a01a01a6dcaffp-16, 0x1.71de021a90822p-19, 0x1.27e4db57442fbp-22,
+                          0x1.af4e196027428p-26, 0x1.1f731ea5352cap-29};
+   std::memcpy(e->ex, ex, sizeof(ex));
    e->mod = mod ? 1 : 0;
    e->pad_ = 0;
 }

@@ -41,6 +41,7 @@ struct TT06Const {
 struct TT06ExactConst {
    double f1, f2, f3, f4, f5, f6, f7a, f9a, f10;
    double hmod[6], jmod[6];
+   double ex[14];               // 1 / ln 2, -ln 2 in two parts, q_0 .. q_10 (ExactMath::ex)
    int mod;
    int pad_;
 };
