@@ -66,9 +66,10 @@ void ActivationSensor::t90(double *out) const
 void simulationLoop(Simulate &sim, int nsteps)
 {
    const int64_t n = sim.nLocal;
+   // iStim = 0 (simulationLoop.cc:186); each step's end leaves it so
+   if (nsteps > 0) check(cdh_fill(n, 0.0, sim.iStim.p, sim.stream));
    for (int step = 0; step < nsteps; step++) {
-      // iStim = 0, then every stimulus (simulationLoop.cc:186-193)
-      check(cdh_fill(n, 0.0, sim.iStim.p, sim.stream));
+      // every stimulus (:187-193)
       for (auto &s : sim.stimulus) s->stim(sim.time, sim.iStim.p);
       // reaction (:195-200)
       sim.reaction->calc(sim.dt, sim.Vm.p, sim.iStim.p, sim.dVmReaction.p);
@@ -76,16 +77,15 @@ void simulationLoop(Simulate &sim, int nsteps)
       sim.diffusion->updateLocalVoltage(sim.Vm.p);
       sim.diffusion->updateRemoteVoltage(nullptr);
       sim.diffusion->calc(sim.dVmDiffusion.p);
-      // range check before the integrator (:214-217)
-      if (sim.checkRange && n > 0) {
-         hipLaunchKernelGGL(k_check_range_f64, dim3(grid_for(n, 256)), dim3(256), 0, sim.stream,
-                            (int)n, sim.Vm.p, sim.dVmReaction.p, sim.dVmDiffusion.p, sim.vMin,
+      // the range check, then the integrator (:214-227), then time and loop
+      // (:229-231)
+      if (n > 0) {
+         hipLaunchKernelGGL(sim.checkRange ? k_step_end_f64<true> : k_step_end_f64<false>,
+                            dim3(grid_for(n, 256)), dim3(256), 0, sim.stream, (int)n, sim.dt,
+                            sim.Vm.p, sim.dVmReaction.p, sim.dVmDiffusion.p, sim.iStim.p, sim.vMin,
                             sim.vMax, sim.loop, sim.range.p);
          CDH_LAUNCH_CHECK();
       }
-      // integrator (:218-227), then time and loop (:229-231)
-      check(cdh_integrate(n, sim.dt, sim.Vm.p, sim.dVmReaction.p, sim.dVmDiffusion.p,
-                          sim.iStim.p, sim.stream));
       sim.time += sim.dt;
       ++sim.loop;
       // sensors at the new time (:233-241)

@@ -236,7 +236,9 @@ __global__ void k_fill_f64(int n, double v, double *x);
 __global__ void k_set_list_f64(int n, const int *list, double v, double *x);
 __global__ void k_sensor_f64(SensorArgs a, const double *Vm, const double *vrest);
 __global__ void k_sensor4_f64(SensorArgs a, const double *Vm, const double *vrest);
-__global__ void k_check_range_f64(int n, const double *Vm, const double *dVmR, const double *dVmD,
-                                  double vmin, double vmax, int loop, RangeRec *r);
+template <bool CHECK>
+__global__ void k_step_end_f64(int n, double dt, double *Vm, const double *dVmR,
+                               const double *dVmD, double *iStim, double vmin, double vmax,
+                               int loop, RangeRec *r);
 
 }  // namespace cdh
