@@ -250,6 +250,7 @@ __global__ void k_resident_f64(EngineArgs a, ResidentArgs r);
 template <int KIND, int WAVES>
 __global__ void k_resident_split_f64(EngineArgs a, ResidentArgs r);
 __global__ void k_resident_split_mixed(EngineArgs a, ResidentArgs r);
+template <int WAVES>
 __global__ void k_resident_mixed(EngineArgs a, ResidentArgs r);
 
 }  // namespace cdh

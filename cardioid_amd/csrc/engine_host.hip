@@ -183,7 +183,8 @@ struct ResidentKernel {
 std::vector<ResidentKernel> resident_kernels(int mode, bool exact)
 {
    constexpr int split = kSplitWaves * kBlk;
-   if (mode == CDH_MODE_MIXED_FUSED) return {{k_resident_split_mixed, split}, {k_resident_mixed, kBlk}};
+   if (mode == CDH_MODE_MIXED_FUSED) return {{k_resident_split_mixed, split}, {k_resident_mixed<4>, kBlk},
+              {k_resident_mixed<6>, kBlk}};
    if (exact) return {{k_resident_split_f64<kExact, 6>, split}, {k_resident_split_f64<kExact, 8>, split}, {k_resident_f64<kExact, 3>, kBlk}};
    if (mode == CDH_MODE_FP64_FMA)
       return {{k_resident_split_f64<kFitsFma, 6>, split}, {k_resident_split_f64<kFitsFma, 8>, split}, {k_resident_f64<kFitsFma, 3>, kBlk},
@@ -548,9 +549,14 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
       // 3 run at once (seen on the device).  A workgroup of several takes
       // ceil(w / 4) places of the SIMD that has most of it, of the 512 / (its
       // registers, by eights) that a SIMD has, at most 8.
+      // It rounds LDS up by less than the 1,280 bytes it is allocated in, too
+      // (of 160 KB to a CU): it counts 28 workgroups of 5,376 bytes where 25
+      // find room.
+      hipFuncAttributes fa{};
+      CDH_HIP(hipFuncGetAttributes(&fa, (const void *)k.fn));
+      if (fa.sharedSizeBytes > 0)
+         per_cu = std::min(per_cu, 128 / (int)((fa.sharedSizeBytes + 1279) / 1280));
       if (k.threads > kBlk) {
-         hipFuncAttributes fa{};
-         CDH_HIP(hipFuncGetAttributes(&fa, (const void *)k.fn));
          const int places = std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
          per_cu = std::min(per_cu, places / ((k.threads / kBlk + 3) / 4));
       }

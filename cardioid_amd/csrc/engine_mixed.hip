@@ -12,6 +12,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <utility>
+
 #include "engine.hpp"
 #include "engine_resident.hpp"
 #include "tt06_mixed.hpp"
@@ -167,19 +169,49 @@ template __global__ void k_engine_mixed<4>(EngineArgs);
 
 namespace {
 
+// PARK: the weights and the gates wait in LDS from one use to the next, 5.25 KB
+// to a tile (6.25 as it is allocated, so that 24 of 25 that a CU has room for
+// are used), for six wavefronts per SIMD (80 VGPRs); else all is in registers,
+// for four.  Up to 6,144 tiles instead of 4,096: us a step by step kernels and
+// this, 287,496 cells 21.2 and 12.0, 373,248 cells 24.9 and 14.2, 389,017 cells
+// 26.3 and 14.1.
+template <bool PARK>
 struct ResidentMixed {
-   struct Shared {};
+   struct Shared {
+      uint32_t w[9][kBlk];
+      float gate[12][kBlk];
+   };
    float s32[N_STATE32];
    double s64[N_STATE64];
    uint32_t hw[9];
+   Shared *sh;
+   // f(g) for the 12 gates, g a constant
+   template <class F>
+   __device__ __forceinline__ static void each_gate(F &&f)
+   {
+      [&]<int... G>(std::integer_sequence<int, G...>) {
+         (f(std::integral_constant<int, G>{}), ...);
+      }(std::make_integer_sequence<int, 12>{});
+   }
+   template <class G>
+   __device__ __forceinline__ void fetch(G, int lane)
+   {
+      if constexpr (PARK) s32[M_M + G::value] = sh->gate[G::value][lane];
+   }
+   template <class G>
+   __device__ __forceinline__ void park(G, int lane)
+   {
+      if constexpr (PARK) sh->gate[G::value][lane] = s32[M_M + G::value];
+   }
    __amdgpu_buffer_rsrc_t R32, R64;
    const float CDH_CONSTANT *ref;
    float wscale;
    uint32_t lc, rw;
    double iK;
 
-   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t, Shared *)
+   __device__ __forceinline__ void load(const EngineArgs &a, const ResidentTile &t, Shared *shared)
    {
+      sh = shared;
       rw = t.rw;
       lc = t.lc;
       R32 = stream_rsrc(a.st32 + t.run_cell * N_STATE32);
@@ -198,11 +230,17 @@ struct ResidentMixed {
          hw[4 * g + 3] = q.w;
       }
       hw[8] = wp[8 * kBlk + t.lane];
+      if constexpr (PARK) {
+#pragma unroll
+         for (int g = 0; g < 9; g++) sh->w[g][t.lane] = hw[g];
+      }
+      each_gate([&](auto g) { park(g, t.lane); });
       ref = (const float CDH_CONSTANT *)(a.Aref + (int64_t)t.blk * 18);
       wscale = t.S->wdelta_scale;
    }
-   __device__ __forceinline__ void store(const ResidentTile &)
+   __device__ __forceinline__ void store(const ResidentTile &t)
    {
+      each_gate([&](auto g) { fetch(g, t.lane); });
 #pragma unroll
       for (int s = 0; s < N_STATE32; s++) stream_store_f32(s32[s], R32, 4u * lc, 4u * rw * s);
 #pragma unroll
@@ -214,8 +252,21 @@ struct ResidentMixed {
       const double K_i = P.K0 + (double)s32[M_DK_I];
       double dVR = 0.0;
       iK = 0.0;
+      each_gate([&](auto g) { fetch(g, t.lane); });
       if (a.gate_mask & (1u << 12)) dVR = nongateM(*T.K, P, T.coef, a.dt, V, K_i, s32, s64, &iK);
-      gatesM(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(t.meta >> 8), V, s32, a.gate_mask);
+      auto gates = [&](uint32_t mask) {
+         gatesM(T.coef, T.K->exp_coef, P.s_switch, (uint8_t)(t.meta >> 8), V, s32, mask);
+      };
+      if constexpr (!PARK) {
+         gates(a.gate_mask);
+      } else {
+         each_gate([&](auto g) {
+            asm volatile("" ::: "memory");   // fetched here, not before
+            fetch(g, t.lane);
+            gates(a.gate_mask & (1u << g.value));
+            park(g, t.lane);
+         });
+      }
       return dVR;
    }
    // the sums of cell_mixed, in its order
@@ -229,8 +280,9 @@ struct ResidentMixed {
       float acc = 0.0f;
 #pragma unroll
       for (int p = 0; p < 9; p++) {
-         const float w0 = half_lo_plus(hw[p], ref[2 * p]);
-         const float w1 = half_hi_plus(hw[p], ref[2 * p + 1]);
+         const uint32_t h = PARK ? sh->w[p][t.lane] : hw[p];
+         const float w0 = half_lo_plus(h, ref[2 * p]);
+         const float w1 = half_hi_plus(h, ref[2 * p + 1]);
          acc = __builtin_fmaf(w0, (float)(nb[2 * p] - V), acc);
          acc = __builtin_fmaf(w1, (float)(nb[2 * p + 1] - V), acc);
       }
@@ -412,10 +464,20 @@ struct SplitMixed {
 
 }  // namespace
 
-__global__ __launch_bounds__(64, 4) void k_resident_mixed(EngineArgs a, ResidentArgs r)
+template <int WAVES>
+__global__ __launch_bounds__(64, WAVES) void k_resident_mixed(EngineArgs a, ResidentArgs r)
 {
-   resident_run<ResidentMixed>(a, r, nullptr);
+   using C = ResidentMixed<(WAVES > 4)>;
+   if constexpr (WAVES > 4) {
+      __shared__ typename C::Shared sh;
+      resident_run<C>(a, r, &sh);
+   } else {
+      resident_run<C>(a, r, nullptr);
+   }
 }
+
+template __global__ void k_resident_mixed<4>(EngineArgs, ResidentArgs);
+template __global__ void k_resident_mixed<6>(EngineArgs, ResidentArgs);
 
 __global__ __launch_bounds__(kSplitWaves * 64, 8) void k_resident_split_mixed(EngineArgs a,
                                                                               ResidentArgs r)

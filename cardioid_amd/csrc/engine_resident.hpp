@@ -39,7 +39,8 @@
 // 504 cells 10.1 and 6.7 us, 52,500 cells 12.2 and 7.0, 110,592 cells 14.5
 // and 9.7, 193,536 cells 18.9 and 12.9; FMA 262,144 cells (4 wavefronts per
 // SIMD) 24.5 and 15.1; mixed 52,500 cells 10.6 and 5.9, 262,144 cells 15.4
-// and 10.4; exact functions 52,500 cells 13.5 and 9.7.  What bounds it: up
+// and 10.0, 373,248 cells (6 per SIMD) 24.9 and 14.2; exact functions 193,536
+// cells 32 and 17.7.  What bounds it: up
 // to 1,024 tiles the latency of one wavefront's chain (12,000 of 17,000 cycles
 // in the reaction), with more tiles VALU issue.
 #pragma once
@@ -360,9 +361,9 @@ __device__ __forceinline__ void resident_run(const EngineArgs &a, const Resident
 //
 // Per step on one MI355X, step kernels, one wavefront to a tile, and this:
 // reference rounding 504 cells 10.1, 6.6 and 2.5 us, 52,500 cells 12.1, 7.0
-// and 5.3 (821 tiles: the kernel of 64 registers), 46,656 cells 11.6 and 4.2;
-// FMA 52,500 cells 11.7 and 4.4; mixed 504 cells 9.1, 5.8 and 2.6, 52,500
-// cells 10.5, 5.8 and 3.6; exact functions 504 cells 11.9, 9.7 and 3.6.
+// and 4.9 (821 tiles: the kernel of 64 registers), 46,656 cells 11.6 and 4.0;
+// FMA 52,500 cells 11.7 and 4.2; mixed 504 cells 9.1, 5.8 and 2.5, 52,500
+// cells 10.5, 5.8 and 3.4; exact functions 504 cells 11.9, 9.7 and 3.1.
 // Bounded by the exchange of Vm between tiles (a store to its acknowledgement,
 // a flag, a load: some 3,000 cycles) and by the longest part's chain.
 constexpr int kSplitWaves = 6;

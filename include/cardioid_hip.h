@@ -421,7 +421,7 @@ int cdh_batch_get_sensors(cdh_batch *b, int slab, double *rows, double *time, in
 int cdh_batch_set_sensors(cdh_batch *b, int slab, const double *rows, double time, int loop);
 /* advances every slab by nsteps; asynchronous on the batch's stream.  While
  * the live slabs' 64-cell tiles all fit the chip at once (about 200,000 to
- * 260,000 cells, by mode), no halo is linked and no launch was chosen with
+ * 390,000 cells, by mode), no halo is linked and no launch was chosen with
  * cdh_batch_set_launch, a run of 8 steps or more keeps the cells resident
  * over many steps of one cooperative launch, with the same results bit for
  * bit.  Such launches of several batches follow one another on the device. */

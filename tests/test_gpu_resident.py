@@ -2,7 +2,7 @@
 bit for bit: Vm, states, activation and APD90 times, counts, range record and
 clock.  A launch chosen with set_launch runs the step kernels; the default
 runs of 8 steps and more are resident where the tiles fit the chip (3,072
-tiles, for the fits also 4,096 at four wavefronts per SIMD; mixed 4,096)."""
+tiles, for the fits also 4,096 at four wavefronts per SIMD; mixed 6,144)."""
 import numpy as np
 import pytest
 
@@ -84,7 +84,9 @@ def test_small_slabs_equal_the_step_kernels(mode, exact, dims, holes):
 
 @pytest.mark.parametrize("mode,ntile", [("fp64_fused", 3072), ("fp64_fused", 3073),
                                         ("fp64_fma", 4096), ("mixed_fused", 4096),
-                                        ("mixed_fused", 4097)])
+                                        ("mixed_fused", 4097), ("mixed_fused", 5120),
+                                        ("mixed_fused", 5184), ("mixed_fused", 6144),
+                                        ("mixed_fused", 6145)])
 def test_tiles_at_the_edges_of_what_the_chip_holds(mode, ntile):
     """64 x ntile cells in one slab: the last that fits each kernel, and the
     first that does not."""
