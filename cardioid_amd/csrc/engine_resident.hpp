@@ -39,8 +39,8 @@
 // 504 cells 10.1 and 6.7 us, 52,500 cells 12.2 and 7.0, 110,592 cells 14.5
 // and 9.7, 193,536 cells 18.9 and 12.9; FMA 262,144 cells (4 wavefronts per
 // SIMD) 24.5 and 15.1; mixed 52,500 cells 10.6 and 5.9, 262,144 cells 15.4
-// and 10.0, 373,248 cells (6 per SIMD) 24.9 and 14.2; exact functions 193,536
-// cells 32 and 17.7.  What bounds it: up
+// and 10.0, 373,248 cells (6 per SIMD) 24.9 and 14.2; exact functions 262,144
+// cells by step kernels 26.7, 193,536 cells by this 17.7.  What bounds it: up
 // to 1,024 tiles the latency of one wavefront's chain (12,000 of 17,000 cycles
 // in the reaction), with more tiles VALU issue.
 #pragma once
