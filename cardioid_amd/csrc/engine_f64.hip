@@ -14,8 +14,6 @@
 // rounds them, so that the fused step equals the unfused loop bit for bit.
 #pragma clang fp contract(off)
 
-#include <utility>
-
 #include "engine.hpp"
 #include "engine_resident.hpp"
 #include "tt06_exact.hpp"
@@ -172,14 +170,6 @@ struct ResidentF64 {
       double park[NPARK > 0 ? NPARK : 1][kBlk];
    };
    double st[N_STATE];
-   // f(g) for the 12 gates, g a constant
-   template <class F>
-   __device__ __forceinline__ static void each_gate(F &&f)
-   {
-      [&]<int... G>(std::integer_sequence<int, G...>) {
-         (f(std::integral_constant<int, G>{}), ...);
-      }(std::make_integer_sequence<int, N_STATE - S_M>{});
-   }
    template <class G>
    __device__ __forceinline__ void fetch(G, int lane)
    {

@@ -12,8 +12,6 @@
 
 #include <hip/hip_fp16.h>
 
-#include <utility>
-
 #include "engine.hpp"
 #include "engine_resident.hpp"
 #include "tt06_mixed.hpp"
@@ -185,14 +183,6 @@ struct ResidentMixed {
    double s64[N_STATE64];
    uint32_t hw[9];
    Shared *sh;
-   // f(g) for the 12 gates, g a constant
-   template <class F>
-   __device__ __forceinline__ static void each_gate(F &&f)
-   {
-      [&]<int... G>(std::integer_sequence<int, G...>) {
-         (f(std::integral_constant<int, G>{}), ...);
-      }(std::make_integer_sequence<int, 12>{});
-   }
    template <class G>
    __device__ __forceinline__ void fetch(G, int lane)
    {

@@ -48,6 +48,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <utility>
 
 #include "engine.hpp"
 #include "tt06_model.hpp"
@@ -301,6 +302,18 @@ __device__ __forceinline__ void resident_range(const EngineArgs &a, const Reside
       if (!f.count || f.taken != (int32_t)r.base)
          f = RangeRec{1ull, (int32_t)r.base, c.loop, (int64_t)t.cell(), V, dVR, dVD};
    }
+}
+
+// f(g) for the 12 gates, g a constant
+template <class F, int... G>
+__device__ __forceinline__ void each_gate(F &&f, std::integer_sequence<int, G...>)
+{
+   (f(std::integral_constant<int, G>{}), ...);
+}
+template <class F>
+__device__ __forceinline__ void each_gate(F &&f)
+{
+   each_gate(f, std::make_integer_sequence<int, N_STATE - S_M>{});
 }
 
 // The launch's steps of one tile by one wavefront.  C holds the cell's states
