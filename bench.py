@@ -527,7 +527,7 @@ def main():
             "value": u["rate"], "unit": "Gcell-steps/s", "steps": u["steps"],
             "ms_per_step": u["ms"] / u["steps"],
             "note": "TT06Dev tolerance 0, mod 1 (the reaction factory's default deck): exact "
-                    "functions with the device's exp/log/pow, generic gate update; the same "
+                    "functions, generic gate update; the same "
                     "loop and diffusion as fp64_unfused"}
     if "fp64_fused_exact" in res:
         ex = res["fp64_fused_exact"]
