@@ -968,7 +968,7 @@ bool Engine::resident_fits() const
 }
 
 // Up to nsteps of every live slab by the resident kernel, at most
-// kResidentSteps in one launch; returns the steps that are left to the step
+// kResidentSteps (kResidentStepsFew) in one launch; returns the steps that are left to the step
 // kernels, where the device would not take a cooperative launch.
 int Engine::run_resident(int nsteps)
 {
@@ -983,7 +983,7 @@ int Engine::run_resident(int nsteps)
    while (resident_cap_[which] < (nlist_ + 7) / 8 * 8) ++which;     // resident_fits()
    const ResidentKernel kernel = resident_kernels(mode_, exact_ != 0)[which];
    while (nsteps > 0) {
-      const int n = std::min(nsteps, kResidentSteps);
+      const int n = std::min(nsteps, kernel.threads > kBlk ? kResidentStepsFew : kResidentSteps);
       EngineArgs a = args(parity_);
       a.xcd_chunk_log2 = -1;
       a.groups_per_xcd = (a.ntile + 7) / 8;
@@ -1169,10 +1169,10 @@ std::vector<double> Engine::vm(int id)
 // where row q goes.  What one launch may gather is bounded (kReadRoom), so
 // that reading needs the same few MiB on the device for every slab.
 //
-// Short rows are gathered together and go straight to one array.  Longer ones
-// take two pinned pieces in turn: the next piece crosses the bus while
-// several threads move the last one into the caller's pages, which a fresh
-// array has yet to be given (three rows of 4.9 million cells into new arrays:
+// Few short rows cross the bus as the kernel writes them.  Others go one at a
+// time, those of 4 MiB and more by two pinned pieces in turn: the next piece
+// crosses the bus while several threads move the last one into the caller's
+// pages, which a fresh array has yet to be given (three rows of 4.9 million cells into new arrays:
 // 11.7 ms straight, 7.3 ms this way; one into an array in use 2.3 and 1.1 ms).
 template <class F>
 void Engine::read_rows(int id, int rows, double *const *host, F &&gather)
@@ -1201,12 +1201,18 @@ void Engine::read_rows(int id, int rows, double *const *host, F &&gather)
                              stream_));
    };
    if (n * rows <= kReadPiece) {
+      // few enough that the kernel writes them over the bus itself, into a
+      // staging block
+      hipEvent_t ev = nullptr;
+      double *staged = (double *)pinned(n * rows * sizeof(double), &ev);
+      if (staged) r.out = staged;
       launch(rows, n);
-      bool together = true;
-      for (int q = 1; q < rows; q++) together = together && host[q] == host[0] + q * n;
-      if (together) fetch(host[0], 0, rows * n);
-      else for (int q = 0; q < rows; q++) fetch(host[q], q * n, n);
+      if (staged) CDH_HIP(hipEventRecord(ev, stream_));
+      else
+         for (int q = 0; q < rows; q++) fetch(host[q], q * n, n);
       CDH_HIP(hipStreamSynchronize(stream_));
+      if (staged)
+         for (int q = 0; q < rows; q++) std::memcpy(host[q], staged + q * n, n * sizeof(double));
       return;
    }
    const bool straight = n < 2 * kReadPiece;

@@ -239,6 +239,7 @@ class Engine {
    // Steps in one launch: 2 to 5 ms, after which other streams' kernels get
    // their turn.
    static constexpr int kResidentSteps = 256;
+   static constexpr int kResidentStepsFew = 1024;   // six wavefronts to a tile: 2 to 5 us a step
    bool graph_direct_ = false;     // the captured graph's tile mapping
    int64_t graph_base_ = -1;
 
