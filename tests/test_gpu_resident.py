@@ -223,3 +223,36 @@ def test_results_of_a_slab_longer_than_one_gather():
     for x, y in zip(*got):
         assert np.array_equal(x[order], y)
     assert np.unique(got[0][0]).size > 4
+
+
+@pytest.mark.parametrize("modes", [("fp64_fma", "fp64_fma"), ("mixed_fused", "fp64_fused")])
+def test_engines_side_by_side(modes):
+    """Two engines that each fill the chip, queued on their own streams from
+    two threads: their resident launches follow one another, and each one's
+    results are those it has alone."""
+    import threading
+    s = [slab(50, 60, 63, 5.0), slab(48, 56, 70, -40.0, holes=0.1)]
+    alone = []
+    for k in range(2):
+        b = make([s[k]], modes[k], False)
+        i = b.add(s[k])
+        b.run(530)
+        alone.append(results(b, [i]))
+        b.close()
+    bs = [make([s[k]], modes[k], False) for k in range(2)]
+    ids = [b.add(x) for b, x in zip(bs, s)]
+
+    def work(k):
+        for n in (300, 9, 221):
+            bs[k].run(n)
+        bs[k].sync()
+
+    t = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for x in t:
+        x.start()
+    for x in t:
+        x.join()
+    for k in range(2):
+        for a, r in zip(alone[k], results(bs[k], [ids[k]])):
+            assert np.array_equal(a, r)
+        bs[k].close()
