@@ -20,14 +20,15 @@ BoxStimulus::BoxStimulus(const cdh_box_stim &b, const std::vector<int> &cells, h
    list_.upload(cells.data(), cells.size());
 }
 
-void BoxStimulus::stim(double time, double *iStim)
+bool BoxStimulus::stim(double time, double *iStim)
 {
-   if (!(time > b_.t0 && time < b_.tf)) return;
+   if (!(time > b_.t0 && time < b_.tf)) return false;
    const double t = time - std::floor(time / b_.period) * b_.period;
-   if (!(t >= b_.phase && t < b_.phase + b_.duration)) return;
-   if (b_.amplitude == 0.0 || n_ == 0) return;
+   if (!(t >= b_.phase && t < b_.phase + b_.duration)) return false;
+   if (b_.amplitude == 0.0 || n_ == 0) return false;
    // subClassStim assigns the value on its cells (BoxStimulus.cc:61-62)
    check(cdh_set_list(n_, list_.p, b_.amplitude, iStim, stream_));
+   return true;
 }
 
 ActivationSensor::ActivationSensor(int64_t n, double threshold, const double *vrestForApd,
@@ -66,11 +67,14 @@ void ActivationSensor::t90(double *out) const
 void simulationLoop(Simulate &sim, int nsteps)
 {
    const int64_t n = sim.nLocal;
-   // iStim = 0 (simulationLoop.cc:186); each step's end leaves it so
-   if (nsteps > 0) check(cdh_fill(n, 0.0, sim.iStim.p, sim.stream));
+   // whether iStim may hold anything but zeros: whatever the caller left there,
+   // then what the last step's stimuli assigned
+   bool assigned = true;
    for (int step = 0; step < nsteps; step++) {
-      // every stimulus (:187-193)
-      for (auto &s : sim.stimulus) s->stim(sim.time, sim.iStim.p);
+      // iStim = 0, then every stimulus (simulationLoop.cc:186-193)
+      if (assigned) check(cdh_fill(n, 0.0, sim.iStim.p, sim.stream));
+      assigned = false;
+      for (auto &s : sim.stimulus) assigned |= s->stim(sim.time, sim.iStim.p);
       // reaction (:195-200)
       sim.reaction->calc(sim.dt, sim.Vm.p, sim.iStim.p, sim.dVmReaction.p);
       // diffusion (:203-210); one rank, so no remote cells arrive

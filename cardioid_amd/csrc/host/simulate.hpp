@@ -26,7 +26,8 @@ namespace host {
 class BoxStimulus {
  public:
    BoxStimulus(const cdh_box_stim &b, const std::vector<int> &cells, hipStream_t stream);
-   void stim(double time, double *iStim);
+   // whether it assigned anything: on at `time`, and not empty
+   bool stim(double time, double *iStim);
 
  private:
    cdh_box_stim b_;

@@ -238,7 +238,7 @@ __global__ void k_sensor_f64(SensorArgs a, const double *Vm, const double *vrest
 __global__ void k_sensor4_f64(SensorArgs a, const double *Vm, const double *vrest);
 template <bool CHECK>
 __global__ void k_step_end_f64(int n, double dt, double *Vm, const double *dVmR,
-                               const double *dVmD, double *iStim, double vmin, double vmax,
+                               const double *dVmD, const double *iStim, double vmin, double vmax,
                                int loop, RangeRec *r);
 
 }  // namespace cdh

@@ -400,17 +400,18 @@ __global__ __launch_bounds__(256) void k_sensor4_f64(SensorArgs a, const double 
 }
 
 // The end of a step of the host's loop in one pass: Simulate::checkRanges on
-// Vm before the integrator (elec/simulationLoop.cc:214-217; CHECK), the
-// integrator (:221-227), and iStim zeroed for the next step's stimuli (:186).
-// Bound by its 48 bytes a cell.  Three passes of their own read 16 bytes a cell
-// more and launched twice more: 1.06 million cells
-// 157 -> 152 us a step of the loop.
+// Vm before the integrator (elec/simulationLoop.cc:214-217; CHECK), and the
+// integrator (:221-227).  Bound by its 40 bytes a cell; passes of their own
+// read 16 bytes a cell more and launched once more.  With iStim's zeroing only
+// after a step that had a stimulus on, 1.06 million cells take 157 -> 151 us a
+// step of the loop.
 template <bool CHECK>
 __global__ __launch_bounds__(256) void k_step_end_f64(int n, double dt, double *__restrict__ Vm,
                                                       const double *__restrict__ dVmR,
                                                       const double *__restrict__ dVmD,
-                                                      double *__restrict__ iStim, double vmin,
-                                                      double vmax, int loop, RangeRec *r)
+                                                      const double *__restrict__ iStim,
+                                                      double vmin, double vmax, int loop,
+                                                      RangeRec *r)
 {
    const int i = blockIdx.x * blockDim.x + threadIdx.x;
    const bool in = i < n;
@@ -420,7 +421,6 @@ __global__ __launch_bounds__(256) void k_step_end_f64(int n, double dt, double *
       dR = dVmR[i];
       dD = dVmD[i];
       Vm[i] = v + dt * (dR + dD + iStim[i]);
-      iStim[i] = 0.0;
    }
    if constexpr (CHECK) {
       const uint64_t m = __ballot(in && (v > vmax || v < vmin));
@@ -429,10 +429,10 @@ __global__ __launch_bounds__(256) void k_step_end_f64(int n, double dt, double *
 }
 
 template __global__ void k_step_end_f64<false>(int, double, double *, const double *,
-                                               const double *, double *, double, double, int,
+                                               const double *, const double *, double, double, int,
                                                RangeRec *);
 template __global__ void k_step_end_f64<true>(int, double, double *, const double *,
-                                              const double *, double *, double, double, int,
+                                              const double *, const double *, double, double, int,
                                               RangeRec *);
 
 }  // namespace cdh

@@ -1,0 +1,90 @@
+// shim.hip -- the library's C++ parts that no C entry point shows, for the
+// tests (native.py).
+#include <hip/hip_runtime.h>
+
+#include <memory>
+#include <vector>
+
+#include "host/simulate.hpp"
+
+using namespace cdh;
+
+namespace {
+
+// a row of n cells along x with one cell type and no conduction to speak of,
+// stimulated in its first `nstim` cells; the exact functions, so no fits
+std::unique_ptr<host::Simulate> row_simulation(int n, int nstim, const cdh_box_stim &pulse)
+{
+   auto sim = std::make_unique<host::Simulate>(nullptr);
+   sim->dt = 0.02;
+   sim->nLocal = n;
+   for (DevBuf<double> *b : {&sim->Vm, &sim->iStim, &sim->dVmReaction, &sim->dVmDiffusion}) {
+      b->alloc(n);
+      b->zero();
+   }
+   sim->range.alloc(1);
+   sim->range.zero();
+   cdh_tt06_params tp{};
+   tp.dt = sim->dt;
+   tp.mod = 1;
+   if (cdh_celltype_standard("endoCellML", &tp.celltype) != CDH_OK) throw std::runtime_error("cell type");
+   tp.s_kr = tp.s_cal = tp.s_na = 1.0;
+   std::vector<int> cells(n), tissue(n, 1);
+   std::vector<int64_t> gid(n);
+   std::vector<double> sigma(6 * (size_t)n, 0.0);
+   for (int k = 0; k < n; k++) {
+      cells[k] = k;
+      gid[k] = k;
+      sigma[6 * k] = sigma[6 * k + 3] = sigma[6 * k + 5] = 1e-4;
+   }
+   sim->reaction = std::make_unique<host::ReactionManager>();
+   sim->reaction->addReaction(host::reactionFactory("TT06Dev", tp, n, nullptr), cells);
+   sim->reaction->initializeMembraneVoltage(sim->Vm.p);
+   cdh_fgr_params fp{};
+   fp.nx = n;
+   fp.ny = fp.nz = 1;
+   fp.dx = fp.dy = fp.dz = 0.2;
+   fp.diffusionScale = 1.0;
+   fp.nLocal = n;
+   fp.gid = gid.data();
+   fp.cellType = tissue.data();
+   fp.sigma = sigma.data();
+   sim->diffusion = host::diffusionFactory("FGR", fp, nullptr);
+   cells.resize(nstim);
+   sim->stimulus.push_back(std::make_unique<host::BoxStimulus>(pulse, cells, nullptr));
+   return sim;
+}
+
+}  // namespace
+
+extern "C" {
+
+// iStim after each of `ncall` calls of simulationLoop of steps[k] steps, in
+// out[ncall][n]; before each call every cell of it is set to `before`.
+int shim_loop_istim(int n, int nstim, double t0, double duration, double amplitude, int ncall,
+                    const int *steps, double before, double *out)
+{
+   try {
+      cdh_box_stim pulse{};
+      pulse.t0 = -1.0;
+      pulse.tf = 1e9;
+      pulse.period = 1000.0;
+      pulse.phase = t0;
+      pulse.duration = duration;
+      pulse.amplitude = amplitude;
+      auto sim = row_simulation(n, nstim, pulse);
+      const std::vector<double> set(n, before);
+      for (int k = 0; k < ncall; k++) {
+         sim->iStim.upload(set.data(), n);
+         host::simulationLoop(*sim, steps[k]);
+         CDH_HIP(hipDeviceSynchronize());
+         sim->iStim.download(out + (size_t)k * n, n);
+      }
+   } catch (const std::exception &e) {
+      set_last_error(e.what());
+      return 1;
+   }
+   return 0;
+}
+
+}  // extern "C"
