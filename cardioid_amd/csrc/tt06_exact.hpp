@@ -51,7 +51,15 @@ struct ExactMath {
       double r = __builtin_fma(n, E->ex[1], x);
       r = __builtin_fma(n, E->ex[2], r);
       const double q = horner64<3, 13, true>(E->ex, r);
-      return ldexp(__builtin_fma(r, __builtin_fma(r, q, 1.0), 1.0), (int)n);
+      return ldexp(__builtin_fma(r, __builtin_fma(r, q, 1.0), 1.0), exponent(n));
+   }
+   // n as an integer, the nearest one past an int's range (n reaches 6e11) and 0
+   // for NaN, as the instruction converts; the language leaves those undefined
+   __device__ __forceinline__ static int exponent(double n)
+   {
+      int i;
+      asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(n));
+      return i;
    }
    __device__ __forceinline__ static double clamp(double V)
    {
