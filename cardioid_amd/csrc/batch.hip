@@ -250,6 +250,21 @@ int cdh_batch_get_launch(cdh_batch *b, int *waves, int *block, int *occupancy, i
    });
 }
 
+int cdh_batch_set_resident(cdh_batch *b, int on)
+{
+   return guard([&] { engine(b).set_resident(on != 0); });
+}
+
+int cdh_batch_get_resident(cdh_batch *b, int *on, int64_t *steps, int64_t *tiles)
+{
+   return guard([&] {
+      const Engine::ResidentUse u = engine(b).resident_use();
+      if (on) *on = u.on;
+      if (steps) *steps = u.steps;
+      if (tiles) *tiles = u.tiles;
+   });
+}
+
 int cdh_batch_autotune(cdh_batch *b, int steps, double *best_ms, double *table, int max_rows,
                        int *nrows)
 {

@@ -1007,6 +1007,8 @@ int Engine::run_resident(int nsteps)
                          stream_, a, r, (int)slabs_.size());
       CDH_LAUNCH_CHECK();
       epoch_ += (uint32_t)n;
+      resident_steps_ += n;
+      resident_held_ = resident_cap_[which];
       parity_ ^= n & 1;
       for (Slab &s : slabs_)
          if (s.live)

@@ -102,6 +102,17 @@ class Engine {
    void set_launch(const LaunchCfg &c);
    void set_default_launch(const LaunchCfg &c) { cfg_ = c; }   // before any run
    LaunchCfg launch() const { return cfg_; }
+   // the resident form: on unless a launch was chosen since
+   void set_resident(bool on) { resident_ = on; }
+   struct ResidentUse {
+      bool on = false;
+      int64_t steps = 0;           // run resident since creation
+      int64_t tiles = 0;           // what the last resident launch's kernel holds
+   };
+   ResidentUse resident_use() const
+   {
+      return ResidentUse{resident_ && resident_tiles_ > 0, resident_steps_, resident_held_};
+   }
    void set_graph_steps(int k);           // 0: launch each step; else replay k-step graphs
    // times each launch configuration over `steps` steps (after a warm-up
    // step) from the same starting state, keeps the fastest; returns its ms
@@ -229,6 +240,7 @@ class Engine {
    uint32_t epoch_ = 0;
    bool links_dirty_ = true;
    bool resident_ = true;          // off once the caller chooses a launch
+   int64_t resident_steps_ = 0, resident_held_ = 0;   // resident_use()
    std::vector<int64_t> resident_cap_;   // tiles at once, per kernel of resident_kernels()
    int64_t resident_tiles_ = 0;    // the most of them
    uint32_t *failed_ = nullptr;    // host memory the kernel writes

@@ -346,6 +346,26 @@ int cdh_sim_run_timed(cdh_sim *s, int nsteps, double *ms)
    });
 }
 
+int cdh_sim_set_resident(cdh_sim *s, int on)
+{
+   return guard([&] {
+      CDH_REQUIRE(s, "cdh_sim_set_resident: null");
+      if (s->eng) s->eng->set_resident(on != 0);
+      else if (on) throw Error(kErrUnsupported, "cdh_sim_set_resident: fused modes only");
+   });
+}
+
+int cdh_sim_get_resident(cdh_sim *s, int *on, int64_t *steps, int64_t *tiles)
+{
+   return guard([&] {
+      CDH_REQUIRE(s, "cdh_sim_get_resident: null");
+      const Engine::ResidentUse u = s->eng ? s->eng->resident_use() : Engine::ResidentUse{};
+      if (on) *on = u.on;
+      if (steps) *steps = u.steps;
+      if (tiles) *tiles = u.tiles;
+   });
+}
+
 int cdh_sim_get_vm(cdh_sim *s, double *host)
 {
    return guard([&] {

@@ -106,6 +106,8 @@ EXPORTS = [
     "cdh_sim_time", "cdh_sim_loop", "cdh_sim_info",
     "cdh_batch_create", "cdh_batch_destroy", "cdh_slab_extent", "cdh_batch_add",
     "cdh_batch_remove", "cdh_batch_run", "cdh_batch_run_timed", "cdh_batch_sync",
+    "cdh_sim_set_resident", "cdh_sim_get_resident", "cdh_batch_set_resident",
+    "cdh_batch_get_resident",
     "cdh_batch_set_graph", "cdh_batch_set_launch", "cdh_batch_get_launch", "cdh_batch_autotune",
     "cdh_batch_get_vm", "cdh_batch_get_state", "cdh_batch_get_activation", "cdh_batch_get_t90",
     "cdh_batch_range_report", "cdh_batch_slab_info", "cdh_batch_info",
@@ -206,6 +208,9 @@ def lib():
         L.cdh_batch_set_graph.argtypes = [C.c_void_p, C.c_int]
         L.cdh_batch_set_launch.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int]
         L.cdh_batch_get_launch.argtypes = [C.c_void_p, ip, ip, ip, ip]
+        for o in ("sim", "batch"):
+            getattr(L, f"cdh_{o}_set_resident").argtypes = [C.c_void_p, C.c_int]
+            getattr(L, f"cdh_{o}_get_resident").argtypes = [C.c_void_p, ip, i64p, i64p]
         L.cdh_batch_autotune.argtypes = [C.c_void_p, C.c_int, dp, dp, C.c_int, ip]
         L.cdh_batch_get_vm.argtypes = [C.c_void_p, C.c_int, dp]
         L.cdh_batch_get_state.argtypes = [C.c_void_p, C.c_int, dp]
@@ -291,6 +296,12 @@ def read_checkpoint(state_file: str, gid):
     check(lib().cdh_checkpoint_read(state_file.encode(), n, ptr(gid, i64p), ptr(Vm), ptr(state),
                                     C.byref(loop), C.byref(time)), "cdh_checkpoint_read")
     return Vm, state, loop.value, time.value
+
+
+def _resident(call, what):
+    on, steps, tiles = C.c_int(), C.c_int64(), C.c_int64()
+    check(call(C.byref(on), C.byref(steps), C.byref(tiles)), what)
+    return {"on": bool(on.value), "steps": steps.value, "tiles": tiles.value}
 
 
 def _range_report(call, what):
@@ -379,6 +390,15 @@ class Simulation:
 
     def sync(self):
         check(lib().cdh_sim_sync(self.h), "cdh_sim_sync")
+
+    def set_resident(self, on: bool):
+        """The resident form of run(), on or off (cdh_sim_set_resident)."""
+        check(lib().cdh_sim_set_resident(self.h, int(on)), "cdh_sim_set_resident")
+
+    def resident(self):
+        """As Batch.resident()."""
+        return _resident(lambda *a: lib().cdh_sim_get_resident(self.h, *a),
+                         "cdh_sim_get_resident")
 
     def vm(self) -> np.ndarray:
         out = np.zeros(self.ncell)
@@ -610,6 +630,16 @@ class Batch:
         check(lib().cdh_batch_get_launch(self.h, C.byref(w), C.byref(b), C.byref(o), C.byref(x)),
               "cdh_batch_get_launch")
         return w.value, b.value, o.value, x.value
+
+    def set_resident(self, on: bool):
+        """The resident form of run(), on or off (cdh_batch_set_resident)."""
+        check(lib().cdh_batch_set_resident(self.h, int(on)), "cdh_batch_set_resident")
+
+    def resident(self):
+        """{"on", "steps" run resident so far, "tiles" the last such launch's
+        kernel holds} (cdh_batch_get_resident)"""
+        return _resident(lambda *a: lib().cdh_batch_get_resident(self.h, *a),
+                         "cdh_batch_get_resident")
 
     def autotune(self, steps: int = 10):
         """(best ms per step, [(waves, block, occupancy, tile order, ms per

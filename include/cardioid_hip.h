@@ -282,6 +282,11 @@ int cdh_sim_sync(cdh_sim *s);
 /* runs nsteps and returns the GPU time between events recorded on the
  * engine's stream around them, in ms */
 int cdh_sim_run_timed(cdh_sim *s, int nsteps, double *ms);
+/* the fused modes' resident form, as cdh_batch_set_resident and
+ * cdh_batch_get_resident; a nonzero variant creates the engine with it off.
+ * The unfused mode has none (set: an error where `on`; get: 0, 0, 0). */
+int cdh_sim_set_resident(cdh_sim *s, int on);
+int cdh_sim_get_resident(cdh_sim *s, int *on, int64_t *steps, int64_t *tiles);
 int cdh_sim_get_vm(cdh_sim *s, double *host);          /* ncell, input order */
 int cdh_sim_get_state(cdh_sim *s, double *host);       /* [19][ncell], input order */
 int cdh_sim_set_state(cdh_sim *s, const double *state, const double *Vm);
@@ -424,7 +429,10 @@ int cdh_batch_set_sensors(cdh_batch *b, int slab, const double *rows, double tim
  * 390,000 cells, by mode), no halo is linked and no launch was chosen with
  * cdh_batch_set_launch, a run of 8 steps or more keeps the cells resident
  * over many steps of one cooperative launch, with the same results bit for
- * bit.  Such launches of several batches follow one another on the device. */
+ * bit.  Such launches of several batches follow one another on the device,
+ * and one that fills the chip lets other streams' kernels start only at its
+ * end, after 2 to 5 ms, where step kernels let them in between two steps: a
+ * caller who shares the device can turn the form off (cdh_batch_set_resident). */
 int cdh_batch_run(cdh_batch *b, int nsteps);
 int cdh_batch_run_timed(cdh_batch *b, int nsteps, double *ms);
 int cdh_batch_sync(cdh_batch *b);
@@ -437,10 +445,19 @@ int cdh_batch_set_graph(cdh_batch *b, int steps);
  * workgroup) and the order in which tiles meet the 8 XCDs, each with its own
  * L2 (-1: XCD x serves the x-th contiguous eighth of the tiles; k >= 0: runs
  * of 2^k workgroups dealt to the XCDs in turn).  From then on every step is
- * the step kernel's (see cdh_batch_run), until an autotune finds the
- * resident form faster. */
+ * the step kernel's (see cdh_batch_run), until cdh_batch_set_resident turns
+ * the resident form on again or an autotune finds it faster. */
 int cdh_batch_set_launch(cdh_batch *b, int waves, int block, int occupancy, int tile_order);
 int cdh_batch_get_launch(cdh_batch *b, int *waves, int *block, int *occupancy, int *tile_order);
+/* The resident form of cdh_batch_run, on or off: on at creation, off after a
+ * cdh_batch_set_launch.  With it on, runs that do not fit it take the launch
+ * configuration as it is. */
+int cdh_batch_set_resident(cdh_batch *b, int on);
+/* *on: whether runs may be resident (0 as well where the device takes no
+ * cooperative launches or refused one); *steps: the steps run resident since
+ * creation; *tiles: how many tiles the kernel of the last resident launch
+ * holds at once (0: none yet).  Any may be NULL. */
+int cdh_batch_get_resident(cdh_batch *b, int *on, int64_t *steps, int64_t *tiles);
 /* times every launch configuration for `steps` steps from the current state
  * (which is restored afterwards) and keeps the fastest; the table gets
  * (waves, block, occupancy, tile order, ms per step) rows, up to max_rows */
