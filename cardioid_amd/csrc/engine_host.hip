@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "engine_resident.hpp"
+#include "resident_rules.hpp"
 #include "setup.hpp"
 #include "setup_device.hpp"
 
@@ -968,8 +969,9 @@ bool Engine::resident_fits() const
 }
 
 // Up to nsteps of every live slab by the resident kernel, at most
-// kResidentSteps (kResidentStepsFew) in one launch; returns the steps that are left to the step
-// kernels, where the device would not take a cooperative launch.
+// kResidentSteps (kResidentStepsFew) in one launch; returns the steps that are
+// left to the step kernels, where the device turns the cooperative launch down
+// (resident_refused), which resident_use() then shows.
 int Engine::run_resident(int nsteps)
 {
    if (links_dirty_) {
@@ -997,9 +999,13 @@ int Engine::run_resident(int nsteps)
       r.failed = failed_;
       r.tile_ranges = (int)(ranges_.n - (size_t)resident_tiles_);
       void *kargs[2] = {&a, &r};
-      if (hipLaunchCooperativeKernel((const void *)kernel.fn, dim3(8 * a.groups_per_xcd),
-                                     dim3(kernel.threads), kargs, 0, stream_) != hipSuccess) {
+      const hipError_t e =
+          hipLaunchCooperativeKernel((const void *)kernel.fn, dim3(8 * a.groups_per_xcd),
+                                     dim3(kernel.threads), kargs, 0, stream_);
+      if (e != hipSuccess) {
          (void)hipGetLastError();
+         if (!resident_refused(e))
+            throw Error(kErrHip, std::string("engine: resident launch: ") + hipGetErrorString(e));
          resident_ = false;
          return nsteps;
       }

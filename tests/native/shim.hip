@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "host/simulate.hpp"
+#include "resident_rules.hpp"
 
 using namespace cdh;
 
@@ -86,5 +87,7 @@ int shim_loop_istim(int n, int nstim, double t0, double duration, double amplitu
    }
    return 0;
 }
+
+int shim_resident_refused(int error) { return resident_refused((hipError_t)error); }
 
 }  // extern "C"
