@@ -20,6 +20,12 @@ struct cdh_batch {
    std::map<int, std::array<int, 3>> grid;
 };
 
+Engine &cdh::batch_engine(cdh_batch *b)
+{
+   CDH_REQUIRE(b && b->eng, "batch is null");
+   return *b->eng;
+}
+
 namespace {
 
 SlabInput slab_input(const cdh_slab_desc *d, std::vector<CellType> &cts)
@@ -58,11 +64,7 @@ SlabInput slab_input(const cdh_slab_desc *d, std::vector<CellType> &cts)
    return in;
 }
 
-Engine &engine(cdh_batch *b)
-{
-   CDH_REQUIRE(b && b->eng, "batch is null");
-   return *b->eng;
-}
+Engine &engine(cdh_batch *b) { return batch_engine(b); }
 
 // input-order copy of a slab-order array
 void scatter(const Engine::Slab &s, const double *src, double *dst, int nq = 1)

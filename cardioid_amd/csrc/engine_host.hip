@@ -564,7 +564,8 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
       resident_cap_.push_back(coop ? (int64_t)ncu * per_cu : 0);
       resident_tiles_ = std::max(resident_tiles_, resident_cap_.back());
    }
-   track(flags_, (kFlagStride + 6) * (size_t)resident_tiles_);
+   track(flags_, (kFlagStride + 6) * (size_t)resident_tiles_ + kFlagStride);
+   CDH_HIP(hipMemset(resident_failed_word(), 0, sizeof(uint32_t)));
    CDH_HIP(hipMemset(blk_slab_.p, 0xFF, ntile * sizeof(uint16_t)));
    track(slabdev_, cap_slabs);
    slabdev_.zero();
@@ -985,6 +986,7 @@ int Engine::run_resident(int nsteps)
    while (resident_cap_[which] < (nlist_ + 7) / 8 * 8) ++which;     // resident_fits()
    const ResidentKernel kernel = resident_kernels(mode_, exact_ != 0)[which];
    while (nsteps > 0) {
+      check_waits();
       const int n = std::min(nsteps, kernel.threads > kBlk ? kResidentStepsFew : kResidentSteps);
       EngineArgs a = args(parity_);
       a.xcd_chunk_log2 = -1;
@@ -996,7 +998,9 @@ int Engine::run_resident(int nsteps)
       r.nsteps = n;
       r.box[0] = box_[parity_].p;
       r.box[1] = box_[parity_ ^ 1].p;
-      r.failed = failed_;
+      r.failed = resident_failed_word();
+      r.failed_host = failed_;
+      r.wait_ticks = wait_ticks_;
       r.tile_ranges = (int)(ranges_.n - (size_t)resident_tiles_);
       void *kargs[2] = {&a, &r};
       const hipError_t e =
@@ -1067,12 +1071,24 @@ double Engine::run_timed(int nsteps)
    return ms;
 }
 
-void Engine::sync()
+// the word behind the flags and the links, in a line of its own
+uint32_t *Engine::resident_failed_word() const
 {
-   CDH_HIP(hipStreamSynchronize(stream_));
+   return flags_.p + (flags_.n - 1) / kFlagStride * kFlagStride;
+}
+
+// Throws if a resident wait has passed its bound.
+void Engine::check_waits()
+{
    if (failed_ && *(volatile uint32_t *)failed_)
       throw Error(kErrHip, "engine: a resident tile waited past its bound for a neighbour; the "
                            "states are not valid");
+}
+
+void Engine::sync()
+{
+   CDH_HIP(hipStreamSynchronize(stream_));
+   check_waits();
    retire_staging();
 }
 

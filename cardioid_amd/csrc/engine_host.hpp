@@ -19,6 +19,8 @@
 #include "setup_device.hpp"
 #include "slab.hpp"
 
+struct cdh_batch;
+
 namespace cdh {
 
 // first-fit allocator of [0, capacity) ranges
@@ -36,6 +38,9 @@ class RangeAlloc {
    std::map<int64_t, int64_t> taken_;
    int64_t cap_ = 0, used_ = 0;
 };
+
+// the bound of a resident tile's wait (engine_resident.hpp): 20 s of the 100 MHz clock
+constexpr uint64_t kResidentWaitTicks = 2000000000ull;
 
 struct LaunchCfg {
    int waves = 0;     // register target of the kernel instance (waves per SIMD)
@@ -55,6 +60,7 @@ struct RowArgs {
 };
 
 class Engine {
+   friend struct EngineProbe;      // the tests' access
  public:
    struct Slab {
       bool live = false;
@@ -163,6 +169,8 @@ class Engine {
    void read_cols(int id, int ncol, const double *const *arena, double *const *host);
    bool resident_fits() const;
    int run_resident(int nsteps);
+   uint32_t *resident_failed_word() const;
+   void check_waits();
    void launch_step(int parity);
    void upload_halo();
    void rebuild_graph();
@@ -235,7 +243,8 @@ class Engine {
    bool tiles_direct_ = false;     // the live tiles are tile_base_ .. + nlist_ - 1
    int64_t tile_base_ = 0;
    // the resident form (engine_resident.hpp): per tile the steps it has done,
-   // counted in epoch_ over all launches, and behind them its links
+   // counted in epoch_ over all launches, behind them its links, and behind
+   // those the word that a wait past its bound sets
    DevBuf<uint32_t> flags_;
    uint32_t epoch_ = 0;
    bool links_dirty_ = true;
@@ -244,6 +253,7 @@ class Engine {
    std::vector<int64_t> resident_cap_;   // tiles at once, per kernel of resident_kernels()
    int64_t resident_tiles_ = 0;    // the most of them
    uint32_t *failed_ = nullptr;    // host memory the kernel writes
+   uint64_t wait_ticks_ = kResidentWaitTicks;
    // A cooperative launch takes about 24 us more than a plain one; a step
    // then saves 3 to 8 us (see resident_kernels and engine_resident.hpp), so
    // that 4 to 6 steps break even.
@@ -283,5 +293,8 @@ class Engine {
 // holds; -1 is K_i - K0
 int mixed_slot_source(int q);
 constexpr int kMixed32 = 17;
+
+// the engine behind a C handle (batch.hip)
+Engine &batch_engine(::cdh_batch *b);
 
 }  // namespace cdh

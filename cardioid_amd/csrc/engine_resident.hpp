@@ -20,8 +20,10 @@
 //
 // Every tile is resident because the launch is cooperative and the host
 // keeps the grid within the kernel's occupancy, so every wait ends.  All the
-// same each wait is bounded (kResidentWaitTicks): past it the wavefront
-// raises `failed`, which the host reports, and nobody waits any longer.
+// same each wait is bounded (ResidentArgs::wait_ticks): past it the wavefront
+// raises `failed`, which the host reports, and nobody waits any longer: a long
+// wait looks for it, and so does every wavefront of the launches queued behind,
+// before its first step.
 //
 // Vm and the flags are stored and loaded at agent scope (SC1), where the XCDs'
 // caches agree, as relaxed atomics are; a tile's flag is stored after the
@@ -60,7 +62,9 @@ namespace cdh {
 // there: at 2,940 tiles (mixed) a wait took 17,400 cycles of a step, with a
 // line each 4,000.
 constexpr int kFlagStride = 32;
-constexpr uint64_t kResidentWaitTicks = 2000000000ull;   // 20 s of the 100 MHz clock
+// Polls between two looks at the clock and at `failed`: some 50 us.  A look at
+// every poll delays the next one (500 steps of 504 cells 1,504 us, this 1,461).
+constexpr uint32_t kResidentPolls = 64;
 
 struct ResidentArgs {
    // both by the tile's place in the list of live tiles
@@ -70,7 +74,9 @@ struct ResidentArgs {
    uint32_t base;               // every tile's flag at the launch
    int nsteps;
    double *box[2];              // box[k & 1] is read in step k of this launch
-   uint32_t *failed;            // host memory; 1 once a wait has passed its bound
+   uint32_t *failed;            // 1 once a wait has passed its bound; on the device
+   uint32_t *failed_host;       // the same in host memory
+   uint64_t wait_ticks;         // that bound, in ticks of the 100 MHz clock
    int tile_ranges;             // the tiles' range records in EngineArgs::ranges (resident_range)
 };
 
@@ -140,30 +146,47 @@ __device__ __forceinline__ void renew(ModelTables &T)
    asm volatile("" : "+s"(T.K), "+s"(T.E), "+s"(T.coef));
 }
 
+__device__ __forceinline__ bool resident_failed(const ResidentArgs &r)
+{
+   return __builtin_amdgcn_readfirstlane(
+       __hip_atomic_load(r.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// The look of a wait that has polled for a while; whether it is to end, for its
+// own bound or for another wavefront's.
+__device__ __forceinline__ bool resident_give_up(const ResidentArgs &r, int lane, uint64_t &since)
+{
+   const uint64_t now = __builtin_amdgcn_s_memrealtime();
+   if (since == 0) since = now;
+   if (resident_failed(r)) return true;
+   if (now - since <= r.wait_ticks) return false;
+   if (lane == 0) {
+      __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(r.failed_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+   }
+   return true;
+}
+
 // Waits until every tile of the three ranges has done `target` - base steps.
 __device__ __forceinline__ void resident_wait(const ResidentArgs &r, const uint32_t *lk, int lane,
                                               uint32_t target, bool &bail)
 {
    const int n0 = (int)(lk[1] - lk[0]), n1 = (int)(lk[3] - lk[2]), n2 = (int)(lk[5] - lk[4]);
    const int n = n0 + n1 + n2;
-   for (int q = lane; __ballot(q < n); q += kBlk) {
+   for (int q = lane; !bail && __ballot(q < n); q += kBlk) {
       const bool mine = q < n;
       const uint32_t t = !mine ? 0u
                          : q < n0 ? lk[0] + q
                          : q < n0 + n1 ? lk[2] + (q - n0) : lk[4] + (q - n0 - n1);
       uint64_t since = 0;
-      while (!bail) {
+      for (uint32_t polls = 1;; polls++) {
          const uint32_t f = mine ? __hip_atomic_load(r.flags + kFlagStride * t, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT)
                                  : target;
          if (!__ballot((int32_t)(f - target) < 0)) break;
-         const uint64_t now = __builtin_amdgcn_s_memrealtime();
-         if (since == 0) since = now;
-         if (now - since > kResidentWaitTicks) {
-            if (lane == 0) __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_SYSTEM);
-            bail = true;
-         }
+         if (polls % kResidentPolls) continue;
+         bail = __builtin_amdgcn_readfirstlane(resident_give_up(r, lane, since));
+         if (bail) break;
       }
    }
 }
@@ -176,6 +199,7 @@ struct ResidentLinks {
    {
 #pragma unroll
       for (int q = 0; q < 6; q++) lk[q] = __builtin_amdgcn_readfirstlane(r.links[6 * j + q]);
+      bail = resident_failed(r);
    }
    // before the stencil of step k of the launch
    __device__ __forceinline__ void wait(const ResidentArgs &r, const ResidentTile &t, int k)

@@ -5,10 +5,30 @@
 #include <memory>
 #include <vector>
 
+#include "engine_host.hpp"
+#include "engine_resident.hpp"
 #include "host/simulate.hpp"
 #include "resident_rules.hpp"
 
 using namespace cdh;
+
+namespace cdh {
+struct EngineProbe {
+   static void set_wait(Engine &e, double seconds) { e.wait_ticks_ = (uint64_t)(seconds * 1e8); }
+   // Has the first tile wait for one that the engine does not have, whose flag
+   // nobody advances; the kernels' bounded wait then passes its bound.
+   static void wait_for_nobody(Engine &e)
+   {
+      e.sync();
+      CDH_REQUIRE(!e.links_dirty_ && e.nlist_ + 1 < e.resident_tiles_, "no resident run yet");
+      const uint32_t far = (uint32_t)e.resident_tiles_ - 1;
+      const uint32_t link[2] = {far, far + 1};
+      e.flags_.upload(&e.epoch_, 1, kFlagStride * (size_t)far);
+      e.flags_.upload(link, 2, kFlagStride * (size_t)e.resident_tiles_ + 4);
+      CDH_HIP(hipDeviceSynchronize());
+   }
+};
+}  // namespace cdh
 
 namespace {
 
@@ -86,6 +106,15 @@ int shim_loop_istim(int n, int nstim, double t0, double duration, double amplitu
       return 1;
    }
    return 0;
+}
+
+// the batch's resident runs time out after `seconds`, in a wait that nothing ends
+int shim_resident_stuck(cdh_batch *b, double seconds)
+{
+   return guard([&] {
+      EngineProbe::set_wait(batch_engine(b), seconds);
+      EngineProbe::wait_for_nobody(batch_engine(b));
+   });
 }
 
 int shim_resident_refused(int error) { return resident_refused((hipError_t)error); }

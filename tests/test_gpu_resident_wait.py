@@ -1,0 +1,52 @@
+"""A resident tile's wait past its bound: the error, and what follows it.  The
+first tile is made to wait for a flag that nobody advances, so that the
+kernel's own bound ends the wait and every launch exits."""
+import time
+
+import numpy as np
+import pytest
+
+import native_lib
+from cardioid_amd import hip
+from test_gpu_resident import make, results, slab
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+BOUND = 0.25                      # seconds
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    hip.lib()
+    yield
+
+
+def stuck(mode, s):
+    """A batch holding slab s (its id) whose resident runs time out."""
+    b = make([s], mode, False)
+    i = b.add(s)
+    b.run(8)
+    b.sync()
+    assert b.resident()["steps"] == 8
+    native_lib.check(native_lib.shim().shim_resident_stuck(b.h, native_lib.C.c_double(BOUND)))
+    return b, i
+
+
+# few tiles: six wavefronts to a tile, 1,024 steps a launch; many: one, 256 steps
+SIZES = [("mixed_fused", (9, 10, 11), 1024), ("fp64_fma", (5, 6, 70), 1024),
+         ("fp64_fused", (40, 42, 44), 256), ("mixed_fused", (40, 42, 44), 256)]
+
+
+@pytest.mark.parametrize("mode,dims,launch", SIZES)
+def test_later_launches_do_not_wait_again(mode, dims, launch):
+    b, _ = stuck(mode, slab(*dims))
+    print("ten launches, the first of which times out", flush=True)
+    t = time.perf_counter()
+    with pytest.raises(hip.CardioidHipError, match="waited past its bound"):
+        b.run(10 * launch)
+        b.sync()
+    t = time.perf_counter() - t
+    assert BOUND < t < 3 * BOUND, t
+    b.close()
