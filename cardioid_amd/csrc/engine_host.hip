@@ -1066,6 +1066,7 @@ double Engine::run_timed(int nsteps)
    run(nsteps);
    CDH_HIP(hipEventRecord(ev1_, stream_));
    CDH_HIP(hipEventSynchronize(ev1_));
+   check_waits();
    float ms = 0.0f;
    CDH_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
    return ms;

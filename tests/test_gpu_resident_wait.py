@@ -50,3 +50,11 @@ def test_later_launches_do_not_wait_again(mode, dims, launch):
     t = time.perf_counter() - t
     assert BOUND < t < 3 * BOUND, t
     b.close()
+
+
+def test_a_timed_run_is_an_error_too():
+    """It used to return a time for states that are not valid."""
+    b, _ = stuck("mixed_fused", slab(9, 10, 11))
+    with pytest.raises(hip.CardioidHipError, match="waited past its bound"):
+        b.run_timed(40)
+    b.close()
