@@ -672,6 +672,7 @@ int Engine::add(const SlabHost &h)
       Slab &s = slabs_[id];
       s = Slab{};
       s.live = true;
+      s.launch0 = resident_launches_;
       s.tile0 = t0;
       s.ntile = h.ntile;
       s.box0 = b0;
@@ -790,6 +791,7 @@ void Engine::remove(int id)
    tiles_.release(s.tile0, s.ntile);
    boxes_.release(s.box0, s.nbox);
    params_.release(s.param0, s.nparam);
+   nlost_ -= s.lost;
    s = Slab{};
 }
 
@@ -1018,6 +1020,7 @@ int Engine::run_resident(int nsteps)
       CDH_LAUNCH_CHECK();
       epoch_ += (uint32_t)n;
       resident_steps_ += n;
+      ++resident_launches_;
       resident_held_ = resident_cap_[which];
       parity_ ^= n & 1;
       for (Slab &s : slabs_)
@@ -1035,6 +1038,7 @@ void Engine::run(int nsteps)
 {
    CDH_REQUIRE(nsteps >= 0, "engine: negative step count");
    retire_staging();
+   check_waits();
    refresh_tiles();      // before any capture: an upload must not land in a graph
    if (nsteps >= kResidentMin && resident_fits()) nsteps = run_resident(nsteps);
    while (nsteps > 0) {
@@ -1078,12 +1082,25 @@ uint32_t *Engine::resident_failed_word() const
    return flags_.p + (flags_.n - 1) / kFlagStride * kFlagStride;
 }
 
-// Throws if a resident wait has passed its bound.
+// Throws while a slab is live that took part in a run with a resident wait
+// past its bound.  Such a wait ends all others, those of the launches queued
+// behind included, so that every slab of any of them is lost; one that was
+// added since, behind the last launch, is not.
 void Engine::check_waits()
 {
-   if (failed_ && *(volatile uint32_t *)failed_)
+   if (failed_ && *(volatile uint32_t *)failed_) {
+      CDH_HIP(hipStreamSynchronize(stream_));
+      for (Slab &s : slabs_)
+         if (s.live && !s.lost && s.launch0 < resident_launches_) {
+            s.lost = true;
+            ++nlost_;
+         }
+      *(volatile uint32_t *)failed_ = 0;
+      put(resident_failed_word(), std::vector<uint32_t>(1, 0u));
+   }
+   if (nlost_ > 0)
       throw Error(kErrHip, "engine: a resident tile waited past its bound for a neighbour; the "
-                           "states are not valid");
+                           "states of the slabs that ran are not valid until they are removed");
 }
 
 void Engine::sync()

@@ -76,6 +76,8 @@ class Engine {
       std::vector<uint32_t> remote_bi; // box index within the slab's box
       int sensors = 0;
       bool order_up = false;           // the caller's order is on the device
+      int64_t launch0 = 0;             // resident launches queued before it was added
+      bool lost = false;               // took part in a failed one (check_waits)
       double time = 0.0;               // host copy of the slab clock
       int loop = 0;
    };
@@ -250,6 +252,8 @@ class Engine {
    bool links_dirty_ = true;
    bool resident_ = true;          // off once the caller chooses a launch
    int64_t resident_steps_ = 0, resident_held_ = 0;   // resident_use()
+   int64_t resident_launches_ = 0;
+   int nlost_ = 0;                 // live slabs that are lost
    std::vector<int64_t> resident_cap_;   // tiles at once, per kernel of resident_kernels()
    int64_t resident_tiles_ = 0;    // the most of them
    uint32_t *failed_ = nullptr;    // host memory the kernel writes

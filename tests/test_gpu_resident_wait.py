@@ -58,3 +58,49 @@ def test_a_timed_run_is_an_error_too():
     with pytest.raises(hip.CardioidHipError, match="waited past its bound"):
         b.run_timed(40)
     b.close()
+
+
+@pytest.mark.parametrize("mode,dims", [("mixed_fused", (9, 10, 11)), ("fp64_fma", (40, 42, 44))])
+def test_the_engine_goes_on_once_the_slab_is_replaced(mode, dims):
+    """The failure belongs to the slabs that took part: they stay an error
+    until they leave, and what is added after runs as in a fresh engine."""
+    s, t = slab(*dims, phi=-30.0), slab(*dims, phi=15.0)
+    b, i = stuck(mode, s)
+    b.run(40)
+    for call in (b.sync, lambda: b.vm(i), lambda: b.state(i), lambda: b.run(40),
+                 lambda: b.run_timed(40), b.sync):
+        with pytest.raises(hip.CardioidHipError, match="waited past its bound"):
+            call()
+    b.remove(i)
+    b.sync()
+    i = b.add(t)
+    steps = b.resident()["steps"]
+    b.run(300)
+    got = results(b, [i])
+    assert b.resident()["steps"] == steps + 300
+    b.close()
+    fresh = make([t], mode, False)
+    j = fresh.add(t)
+    fresh.run(300)
+    for a, r in zip(got, results(fresh, [j])):
+        assert np.array_equal(a, r)
+    fresh.close()
+
+
+def test_a_slab_added_behind_the_failing_run_is_not_lost():
+    """Replaced without a sync in between: the new slab took no part."""
+    s, t = slab(9, 10, 11), slab(6, 7, 8, phi=15.0)
+    b, i = stuck("mixed_fused", s)
+    b.run(40)
+    time.sleep(2 * BOUND)              # the launch has failed by now
+    b.remove(i)
+    i = b.add(t)
+    b.run(100)
+    got = results(b, [i])
+    b.close()
+    fresh = make([t], "mixed_fused", False)
+    j = fresh.add(t)
+    fresh.run(100)
+    for a, r in zip(got, results(fresh, [j])):
+        assert np.array_equal(a, r)
+    fresh.close()
