@@ -1002,7 +1002,7 @@ int Engine::run_resident(int nsteps)
       r.box[1] = box_[parity_ ^ 1].p;
       r.failed = resident_failed_word();
       r.failed_host = failed_;
-      r.wait_ticks = wait_ticks_;
+      r.max_polls = max_polls_;
       r.tile_ranges = (int)(ranges_.n - (size_t)resident_tiles_);
       void *kargs[2] = {&a, &r};
       const hipError_t e =

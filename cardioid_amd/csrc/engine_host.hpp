@@ -39,8 +39,9 @@ class RangeAlloc {
    int64_t cap_ = 0, used_ = 0;
 };
 
-// the bound of a resident tile's wait (engine_resident.hpp): 20 s of the 100 MHz clock
-constexpr uint64_t kResidentWaitTicks = 2000000000ull;
+// the bound of a resident tile's wait (engine_resident.hpp), in polls of some
+// 0.16 us: 20 s of polling
+constexpr uint32_t kResidentPollsMost = 1u << 27;
 
 struct LaunchCfg {
    int waves = 0;     // register target of the kernel instance (waves per SIMD)
@@ -257,7 +258,7 @@ class Engine {
    std::vector<int64_t> resident_cap_;   // tiles at once, per kernel of resident_kernels()
    int64_t resident_tiles_ = 0;    // the most of them
    uint32_t *failed_ = nullptr;    // host memory the kernel writes
-   uint64_t wait_ticks_ = kResidentWaitTicks;
+   uint32_t max_polls_ = kResidentPollsMost;
    // A cooperative launch takes about 24 us more than a plain one; a step
    // then saves 3 to 8 us (see resident_kernels and engine_resident.hpp), so
    // that 4 to 6 steps break even.

@@ -20,7 +20,7 @@
 //
 // Every tile is resident because the launch is cooperative and the host
 // keeps the grid within the kernel's occupancy, so every wait ends.  All the
-// same each wait is bounded (ResidentArgs::wait_ticks): past it the wavefront
+// same each wait is bounded (ResidentArgs::max_polls): past it the wavefront
 // raises `failed`, which the host reports, and nobody waits any longer: a long
 // wait looks for it, and so does every wavefront of the launches queued behind,
 // before its first step.
@@ -62,8 +62,8 @@ namespace cdh {
 // there: at 2,940 tiles (mixed) a wait took 17,400 cycles of a step, with a
 // line each 4,000.
 constexpr int kFlagStride = 32;
-// Polls between two looks at the clock and at `failed`: some 50 us.  A look at
-// every poll delays the next one (500 steps of 504 cells 1,504 us, this 1,461).
+// Polls between two looks at the bound and at `failed`: 10 us.  A look at every poll
+// delays the next one (500 steps of 504 cells 1,504 us, this 1,461).
 constexpr uint32_t kResidentPolls = 64;
 
 struct ResidentArgs {
@@ -76,7 +76,7 @@ struct ResidentArgs {
    double *box[2];              // box[k & 1] is read in step k of this launch
    uint32_t *failed;            // 1 once a wait has passed its bound; on the device
    uint32_t *failed_host;       // the same in host memory
-   uint64_t wait_ticks;         // that bound, in ticks of the 100 MHz clock
+   uint32_t max_polls;          // that bound
    int tile_ranges;             // the tiles' range records in EngineArgs::ranges (resident_range)
 };
 
@@ -153,13 +153,13 @@ __device__ __forceinline__ bool resident_failed(const ResidentArgs &r)
 }
 
 // The look of a wait that has polled for a while; whether it is to end, for its
-// own bound or for another wavefront's.
-__device__ __forceinline__ bool resident_give_up(const ResidentArgs &r, int lane, uint64_t &since)
+// own bound or for another wavefront's.  The bound counts polls and no time: a
+// wavefront that is held off the chip, as all of a process's are while another
+// process has its turn, does not poll, and whom it waits for is held off too.
+__device__ __forceinline__ bool resident_give_up(const ResidentArgs &r, int lane, uint32_t polls)
 {
-   const uint64_t now = __builtin_amdgcn_s_memrealtime();
-   if (since == 0) since = now;
    if (resident_failed(r)) return true;
-   if (now - since <= r.wait_ticks) return false;
+   if (polls <= r.max_polls) return false;
    if (lane == 0) {
       __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(r.failed_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -178,14 +178,13 @@ __device__ __forceinline__ void resident_wait(const ResidentArgs &r, const uint3
       const uint32_t t = !mine ? 0u
                          : q < n0 ? lk[0] + q
                          : q < n0 + n1 ? lk[2] + (q - n0) : lk[4] + (q - n0 - n1);
-      uint64_t since = 0;
       for (uint32_t polls = 1;; polls++) {
          const uint32_t f = mine ? __hip_atomic_load(r.flags + kFlagStride * t, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT)
                                  : target;
          if (!__ballot((int32_t)(f - target) < 0)) break;
          if (polls % kResidentPolls) continue;
-         bail = __builtin_amdgcn_readfirstlane(resident_give_up(r, lane, since));
+         bail = __builtin_amdgcn_readfirstlane(resident_give_up(r, lane, polls));
          if (bail) break;
       }
    }

@@ -432,7 +432,11 @@ int cdh_batch_set_sensors(cdh_batch *b, int slab, const double *rows, double tim
  * bit.  Such launches of several batches follow one another on the device,
  * and one that fills the chip lets other streams' kernels start only at its
  * end, after 2 to 5 ms, where step kernels let them in between two steps: a
- * caller who shares the device can turn the form off (cdh_batch_set_resident). */
+ * caller who shares the device can turn the form off (cdh_batch_set_resident).
+ * Inside a launch a tile waits for its neighbours' tiles; should such a wait
+ * poll for some 20 s (time that the process is held off the device does not
+ * count), this and every later call on the batch that needs its states returns
+ * CDH_ERR_HIP until the slabs that ran have been removed. */
 int cdh_batch_run(cdh_batch *b, int nsteps);
 int cdh_batch_run_timed(cdh_batch *b, int nsteps, double *ms);
 int cdh_batch_sync(cdh_batch *b);

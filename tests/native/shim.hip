@@ -14,7 +14,7 @@ using namespace cdh;
 
 namespace cdh {
 struct EngineProbe {
-   static void set_wait(Engine &e, double seconds) { e.wait_ticks_ = (uint64_t)(seconds * 1e8); }
+   static void set_wait(Engine &e, uint32_t polls) { e.max_polls_ = polls; }
    // Has the first tile wait for one that the engine does not have, whose flag
    // nobody advances; the kernels' bounded wait then passes its bound.
    static void wait_for_nobody(Engine &e)
@@ -108,11 +108,11 @@ int shim_loop_istim(int n, int nstim, double t0, double duration, double amplitu
    return 0;
 }
 
-// the batch's resident runs time out after `seconds`, in a wait that nothing ends
-int shim_resident_stuck(cdh_batch *b, double seconds)
+// the batch's resident runs time out after `polls`, in a wait that nothing ends
+int shim_resident_stuck(cdh_batch *b, unsigned polls)
 {
    return guard([&] {
-      EngineProbe::set_wait(batch_engine(b), seconds);
+      EngineProbe::set_wait(batch_engine(b), polls);
       EngineProbe::wait_for_nobody(batch_engine(b));
    });
 }
