@@ -1142,6 +1142,7 @@ double Engine::autotune(int steps, std::vector<std::pair<LaunchCfg, double>> *ta
    const int par0 = parity_;
    std::vector<Slab> host0 = slabs_;
    const LaunchCfg keep = cfg_;
+   const bool was_resident = resident_;
    const int gsteps = graph_steps_;
    graph_steps_ = 0;
    // two interleaved rounds, each candidate's faster time kept: the
@@ -1170,11 +1171,13 @@ double Engine::autotune(int steps, std::vector<std::pair<LaunchCfg, double>> *ta
       }
    }
    // the resident form in the same way, over enough steps that its launch
-   // weighs as it does in a run
+   // weighs as it does in a run; where the tiles do not fit it stays as it was
    set_launch(bestc);
    resident_ = true;
    refresh_tiles();
-   if (resident_fits()) {
+   if (!resident_fits()) {
+      resident_ = was_resident;
+   } else {
       const int n = std::max(steps, kResidentSteps);
       const double t = run_timed(n) / n;
       resident_ = t < best;
