@@ -464,7 +464,10 @@ int cdh_batch_set_resident(cdh_batch *b, int on);
 int cdh_batch_get_resident(cdh_batch *b, int *on, int64_t *steps, int64_t *tiles);
 /* times every launch configuration for `steps` steps from the current state
  * (which is restored afterwards) and keeps the fastest; the table gets
- * (waves, block, occupancy, tile order, ms per step) rows, up to max_rows */
+ * (waves, block, occupancy, tile order, ms per step) rows, up to max_rows.
+ * Where the live slabs fit the resident form it is timed as well and turned on
+ * or off by what comes out, whatever it was before (else it stays as it was);
+ * where it is the fastest, *best_ms is its time and stands in no row. */
 int cdh_batch_autotune(cdh_batch *b, int steps, double *best_ms, double *table, int max_rows,
                        int *nrows);
 /* per-slab results, in the slab's input cell order */

@@ -32,3 +32,17 @@ def test_a_batch_too_large_leaves_the_form_as_it_was(chosen):
     b.run(16)
     assert b.resident()["steps"] == (0 if chosen else 16)
     b.close()
+
+
+def test_the_resident_form_is_timed_like_the_launches():
+    """Warmed up and the better of two timings, as each launch; where it is the
+    fastest, best_ms is its time and no row's."""
+    s = slab(9, 10, 11)
+    b = make([s], "mixed_fused", True)
+    i = b.add(s)
+    vm = b.vm(i)
+    best, rows = b.autotune(5)
+    assert b.resident() == {"on": True, "steps": 2 * (8 + 256), "tiles": 1024}
+    assert best < min(r[4] for r in rows)
+    assert np.array_equal(b.vm(i), vm) and b.slab_info(i)["loop"] == 0
+    b.close()
