@@ -85,11 +85,8 @@ __global__ __launch_bounds__(256) void k_halo(int64_t n, const uint32_t *pairs, 
 }
 
 // The tiles that can hold neighbours of a tile's cells, for the resident
-// kernels: three ranges (the planes one step back in x, level, and one step
-// on), each {first, last + 1}.  A slab's cells are in box order, so the tiles
-// with cells in a range of box points are a range too, found by the tiles'
-// first box points; a range may hold a tile too many at its start.  Flags of
-// the live tiles start at `base`.
+// kernels: three ranges (tile_range), each {first, last + 1} by the tiles' places
+// in the list.  Flags of the live tiles start at `base`.
 __global__ __launch_bounds__(64) void k_tile_links(EngineArgs a, uint32_t *links, uint32_t *flags,
                                                    uint32_t base)
 {
@@ -106,26 +103,15 @@ __global__ __launch_bounds__(64) void k_tile_links(EngineArgs a, uint32_t *links
       while (last > 0 && (a.meta[(int64_t)blk * kBlk + last] & kMetaPad)) --last;
       const int64_t plane = (int64_t)(S.soff[3] / 8) - kBoxShift;    // x + 1
       const int64_t row = (int64_t)(S.soff[4] / 8) - kBoxShift;      // y + 1
-      const int64_t reach = part == 1 ? row + 1 : row;
-      const int64_t from = (int64_t)a.bi[(int64_t)blk * kBlk] + (part - 1) * plane - reach;
-      const int64_t to = (int64_t)a.bi[(int64_t)blk * kBlk + last] + (part - 1) * plane + reach;
-      // the number of the slab's tiles whose first box point is at most x
-      auto upto = [&](int64_t x) {
-         int n0 = 0, n1 = S.ntile;
-         while (n0 < n1) {
-            const int m = (n0 + n1) / 2;
-            if ((int64_t)a.bi[((int64_t)S.first_blk + m) * kBlk] <= x) n0 = m + 1;
-            else n1 = m;
-         }
-         return n0;
-      };
-      const int e = upto(to);
-      const int f = upto(from);
-      if (e > 0) {
+      const uint32_t *bi = a.bi + (int64_t)blk * kBlk;
+      const TileRange t = tile_range(part, bi[0], bi[last], plane, row, S.ntile, [&](int m) {
+         return (int64_t)a.bi[((int64_t)S.first_blk + m) * kBlk];
+      });
+      if (t.end > 0) {
          // a slab's tiles stand together in the list
          const int j0 = j - (blk - S.first_blk);
-         lo = (uint32_t)(j0 + (f > 0 ? f - 1 : 0));
-         hi = (uint32_t)(j0 + e);
+         lo = (uint32_t)(j0 + t.begin);
+         hi = (uint32_t)(j0 + t.end);
       }
    }
    links[6 * j + 2 * part] = lo;

@@ -2,6 +2,7 @@
 // tests (native.py).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <memory>
 #include <vector>
 
@@ -115,6 +116,21 @@ int shim_resident_stuck(cdh_batch *b, unsigned polls)
       EngineProbe::set_wait(batch_engine(b), polls);
       EngineProbe::wait_for_nobody(batch_engine(b));
    });
+}
+
+// the three ranges of each tile of a slab with cells at box points bi[ncell],
+// out[tiles][3][2]
+void shim_tile_ranges(int64_t ncell, const int64_t *bi, int64_t plane, int64_t row, int *out)
+{
+   const int ntile = (int)((ncell + kBlk - 1) / kBlk);
+   for (int64_t t = 0; t < ntile; t++)
+      for (int part = 0; part < 3; part++) {
+         const TileRange r =
+             tile_range(part, bi[kBlk * t], bi[std::min<int64_t>(kBlk * t + kBlk, ncell) - 1], plane,
+                        row, ntile, [&](int m) { return bi[(int64_t)kBlk * m]; });
+         out[6 * t + 2 * part] = r.begin;
+         out[6 * t + 2 * part + 1] = r.end;
+      }
 }
 
 int shim_resident_refused(int error) { return resident_refused((hipError_t)error); }
