@@ -5,6 +5,9 @@
 
 #include <algorithm>
 #include <cstring>
+#include <map>
+#include <mutex>
+#include <tuple>
 
 #include "engine_resident.hpp"
 #include "resident_rules.hpp"
@@ -178,6 +181,45 @@ std::vector<ResidentKernel> resident_kernels(int mode, bool exact)
               {k_resident_f64<kFitsFma, 4>, kBlk}};
    return {{k_resident_split_f64<kFits, 6>, split}, {k_resident_split_f64<kFits, 8>, split}, {k_resident_f64<kFits, 3>, kBlk},
            {k_resident_f64<kFits, 4>, kBlk}};
+}
+
+// Tiles that each of resident_kernels() holds on a device at once.  Asked for
+// once per device and mode: the answers do not change, and the calls for them
+// took some 15 us of a small engine's 480.
+std::vector<int64_t> resident_capacity(int dev, int mode, bool exact)
+{
+   static std::mutex lock;
+   static std::map<std::tuple<int, int, bool>, std::vector<int64_t>> known;
+   std::lock_guard<std::mutex> hold(lock);
+   std::vector<int64_t> &cap = known[{dev, mode, exact}];
+   if (!cap.empty()) return cap;
+   int ncu = 0, coop = 0;
+   CDH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+   CDH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+   std::vector<int64_t> c;
+   for (const ResidentKernel &k : resident_kernels(mode, exact)) {
+      int per_cu = 0;
+      CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, k.threads, 0));
+      // The call counts wavefronts per CU, as if a workgroup's could stand on
+      // any SIMD: it gives 4 workgroups of 6 wavefronts at 80 registers where
+      // 3 run at once (seen on the device).  A workgroup of several takes
+      // ceil(w / 4) places of the SIMD that has most of it, of the 512 / (its
+      // registers, by eights) that a SIMD has, at most 8.
+      // It rounds LDS up by less than the 1,280 bytes it is allocated in, too
+      // (of 160 KB to a CU): it counts 28 workgroups of 5,376 bytes where 25
+      // find room.
+      hipFuncAttributes fa{};
+      CDH_HIP(hipFuncGetAttributes(&fa, (const void *)k.fn));
+      if (fa.sharedSizeBytes > 0)
+         per_cu = std::min(per_cu, 128 / (int)((fa.sharedSizeBytes + 1279) / 1280));
+      if (k.threads > kBlk) {
+         const int places = std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
+         per_cu = std::min(per_cu, places / ((k.threads / kBlk + 3) / 4));
+      }
+      c.push_back(coop ? (int64_t)ncu * per_cu : 0);
+   }
+   cap = c;
+   return cap;
 }
 
 using KernelFn = void (*)(EngineArgs);
@@ -525,31 +567,8 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
    track(tile_list_, ntile);
    CDH_HIP(hipHostMalloc((void **)&failed_, sizeof(uint32_t), hipHostMallocDefault));
    *failed_ = 0;
-   int ncu = 0, coop = 0;
-   CDH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-   CDH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-   for (const ResidentKernel &k : resident_kernels(mode, exact_ != 0)) {
-      int per_cu = 0;
-      CDH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, k.threads, 0));
-      // The call counts wavefronts per CU, as if a workgroup's could stand on
-      // any SIMD: it gives 4 workgroups of 6 wavefronts at 80 registers where
-      // 3 run at once (seen on the device).  A workgroup of several takes
-      // ceil(w / 4) places of the SIMD that has most of it, of the 512 / (its
-      // registers, by eights) that a SIMD has, at most 8.
-      // It rounds LDS up by less than the 1,280 bytes it is allocated in, too
-      // (of 160 KB to a CU): it counts 28 workgroups of 5,376 bytes where 25
-      // find room.
-      hipFuncAttributes fa{};
-      CDH_HIP(hipFuncGetAttributes(&fa, (const void *)k.fn));
-      if (fa.sharedSizeBytes > 0)
-         per_cu = std::min(per_cu, 128 / (int)((fa.sharedSizeBytes + 1279) / 1280));
-      if (k.threads > kBlk) {
-         const int places = std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
-         per_cu = std::min(per_cu, places / ((k.threads / kBlk + 3) / 4));
-      }
-      resident_cap_.push_back(coop ? (int64_t)ncu * per_cu : 0);
-      resident_tiles_ = std::max(resident_tiles_, resident_cap_.back());
-   }
+   resident_cap_ = resident_capacity(dev, mode, exact_ != 0);
+   for (int64_t c : resident_cap_) resident_tiles_ = std::max(resident_tiles_, c);
    track(flags_, (kFlagStride + 6) * (size_t)resident_tiles_ + kFlagStride);
    CDH_HIP(hipMemset(resident_failed_word(), 0, sizeof(uint32_t)));
    CDH_HIP(hipMemset(blk_slab_.p, 0xFF, ntile * sizeof(uint16_t)));
