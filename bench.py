@@ -340,6 +340,7 @@ def serving(hip, W, nreq, rate, hbm_gb, graph, max_active_cells=None):
     cells, box = serve.arena_for_budget(int(hbm_gb * 2 ** 30))
     b = hip.Batch(DT, cells, box, slab_capacity=1024, mode="mixed_fused", sensors=3)
     b.set_launch(3, 64, 0, -1)
+    b.set_resident(True)       # for the chunks with few cells in flight
     b.set_graph(graph)
     st = serve.Server(b, chunk=100, max_active_cells=max_active_cells).serve(reqs)
     b.close()
