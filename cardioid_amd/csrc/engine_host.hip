@@ -565,8 +565,6 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
    track(bi_, 2 * S);             // and the cells' places in the caller's order
    track(blk_slab_, ntile);
    track(tile_list_, ntile);
-   CDH_HIP(hipHostMalloc((void **)&failed_, sizeof(uint32_t), hipHostMallocDefault));
-   *failed_ = 0;
    resident_cap_ = resident_capacity(dev, mode, exact_ != 0);
    for (int64_t c : resident_cap_) resident_tiles_ = std::max(resident_tiles_, c);
    track(flags_, (kFlagStride + 6) * (size_t)resident_tiles_ + kFlagStride);
@@ -602,6 +600,9 @@ Engine::Engine(int mode, double dt, const int *fit_l, const int *fit_m, const do
       track(t90_, S);
    }
    CDH_HIP(hipDeviceSynchronize());
+   // last: an arena too large for the device throws above
+   CDH_HIP(hipHostMalloc((void **)&failed_, sizeof(uint32_t), hipHostMallocDefault));
+   *failed_ = 0;
 }
 
 Engine::~Engine()
