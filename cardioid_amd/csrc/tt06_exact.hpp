@@ -28,9 +28,9 @@ namespace cdh {
 // by two FMAs (Cody and Waite), exp(r) = 1 + r (1 + r q(r)) with q of degree
 // 10 (its interpolation at the Chebyshev nodes of [-ln 2 / 2, ln 2 / 2];
 // 3e-19 relative), and the scaling by 2^n, which gives infinity or 0 past the
-// range.  Against 64-bit values it is off by 0.257 ulp in the mean and 0.82 at
-// most over [-30, 30], the library's by 0.258 and 0.85.
-// The library's takes some 25, six of them to catch arguments past the range
+// range.  Against quadruple precision it is off by 0.257 ulp in the mean and
+// 0.856 at most (20 million arguments drawn from [-30, 30]); the device
+// library's mean is 0.258.  The library's takes some 25, six of them to catch arguments past the range
 // one by one.  Here the voltage is clamped once per cell instead, to +-1e7,
 // where every one of the functions below has long reached the value it has at
 // infinity; NaN stays NaN.

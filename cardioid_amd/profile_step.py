@@ -3,7 +3,7 @@ workload (or the 64 batched slabs) for a few steps, preceded by a plain
 512 MiB device-to-device copy whose known byte count calibrates rocprofv3's
 FETCH_SIZE / WRITE_SIZE.
 
-    python -m cardioid_amd.profile_step MODE STEPS WAVES BLOCK OCC [shell|batch]
+    python -m cardioid_amd.profile_step MODE STEPS WAVES BLOCK OCC [shell|batch|NX,NY,NZ]
 
 MODE is fp64_fused, fp64_fma or mixed_fused (the fused engine; WAVES/BLOCK/OCC
 the launch configuration: register target, workgroup size, occupancy cap), or
@@ -11,7 +11,8 @@ fp64_unfused (the reference loop over the drop-in objects: reaction, scatter,
 FGR stencil, integrator and sensor kernels; WAVES/BLOCK/OCC ignored), or
 fp64_unfused_exact (the same loop with the reaction factory's default deck,
 TT06Dev tolerance 0: the exact functions), or fp64_fused_exact (that deck in
-the fused FP64 engine).  Meant
+the fused FP64 engine).  NX,NY,NZ is a fibre slab of that size; WAVES 0 leaves
+the launch to the engine, which keeps a slab that fits the chip resident.  Meant
 to run under rocprofv3 (kernel trace, or one --pmc counter per run).
 """
 from __future__ import annotations
@@ -50,6 +51,10 @@ def main(argv):
         anat, depth = W.ellipsoid_shell(256, 256, 512, seed=0)
         stims = W.endocardial_point_stimuli(anat, depth, 8, seed=0)
         slabs = [hip.Slab(anat, W.CELLTYPES_EMI, W.DIFFUSION_SCALE, stims)]
+    elif work != "batch":
+        nx, ny, nz = (int(v) for v in work.split(","))
+        slabs = [hip.Slab(W.fibre_slab(nx, ny, nz, 20.0), ["midCellML"], W.DIFFUSION_SCALE,
+                          [W.box_stimulus(xMax=3, nx=nx, ny=ny, nz=nz)])]
     else:
         slabs = [hip.Slab(c.anatomy, ["endoCellML"], W.DIFFUSION_SCALE, c.stimuli, scales=c.scales)
                  for c in W.batched_slabs()]
@@ -60,12 +65,13 @@ def main(argv):
                   jhTauSmooth=1 if exact else 0)
     for s in slabs:
         b.add(s)
-    b.set_launch(waves, block, occ)
+    if waves:
+        b.set_launch(waves, block, occ)
     b.run(steps)
     b.sync()
     ncell = sum(s.ncell for s in slabs)
     print(f"profile_step: {mode} {work} launch ({waves}, {block}, {occ}), {steps} steps on "
-          f"{ncell} cells",
+          f"{ncell} cells, {b.resident()['steps']} of them resident",
           flush=True)
 
 
