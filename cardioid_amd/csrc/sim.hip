@@ -351,7 +351,8 @@ int cdh_sim_set_resident(cdh_sim *s, int on)
    return guard([&] {
       CDH_REQUIRE(s, "cdh_sim_set_resident: null");
       if (s->eng) s->eng->set_resident(on != 0);
-      else if (on) throw Error(kErrUnsupported, "cdh_sim_set_resident: fused modes only");
+      else if (on && s->mode == CDH_MODE_FP64_UNFUSED)
+         throw Error(kErrUnsupported, "cdh_sim_set_resident: fused modes only");
    });
 }
 
