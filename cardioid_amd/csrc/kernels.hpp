@@ -16,6 +16,10 @@ struct ParamSet;
 constexpr int kMaxStim = 8;
 
 // Reaction over n cells of one reaction group (drop-in object).
+// What a reaction launch updates: the 12 gates (a bit each) and the other
+// states with dVm.
+constexpr uint32_t kMaskGates = 0xFFFu, kMaskNonGate = 1u << 12;
+
 struct ReactionArgs {
    // the constants in device memory rather than a kernel argument: the
    // kernel would otherwise load all of them into SGPRs at entry and spill
@@ -30,7 +34,7 @@ struct ReactionArgs {
    const double *Vm;
    double *dVm;
    double dt;
-   uint32_t gate_mask;          // bits 0..12 set; see gates64 and k_tt06_calc_f64
+   uint32_t gate_mask;          // kMaskGates, kMaskNonGate; see gates64 and k_tt06_calc_f64
    const TT06ExactConst *E;     // configuration A (exact functions) constants, or null
 };
 

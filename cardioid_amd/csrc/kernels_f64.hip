@@ -42,9 +42,15 @@ namespace cdh {
 //
 // EXACT: configuration A, the non-gate update with the exact fv0..fv6, then
 // the generic gate update with the exact steady states and rates, at the
-// step's Vm.  Gate flags bit 0 holds every gate of a cell (the pdr loop's
-// updateNonGate); the generic loop has no v2 loop bounds, so otherwise every
-// cell's gates advance.
+// step's Vm.  Gate flags bit 0 holds every gate of a cell; the generic loop has
+// no v2 loop bounds, so otherwise every cell's gates advance.
+//
+// Without kMaskGates (the pdr loop's updateNonGate) the gates are read and not
+// stored: 208 bytes a cell instead of 304.  Exact functions, us a call, in
+// workgroups of four with the gates stored, as this with them stored, and this:
+// 500,000 cells 27.7, 27.7 and 21.3, 1 million 49.5, 53.2 and 38.5, 1.3 million
+// 63, 69 and 49; the fits, persistent, as this with them stored, and this: 1
+// million 59.5, 53.2 and 37.4.
 //
 // The body takes its arrays as restrict-qualified arguments: the stores then
 // provably leave the constants and fit coefficients alone, and their reads
@@ -75,16 +81,20 @@ __device__ __forceinline__ void calc_tile(const TT06Const *__restrict__ K,
    const ParamSet P = params[0];
    double dVR = 0.0;
    if constexpr (EXACT) {
-      if (gate_mask & (1u << 12))
+      if (gate_mask & kMaskNonGate)
          dVR = nongate_core64(*K, P, exact_voltage_fns(E, K), dt, V, st);
       if (!(fl & kFlagGatesFixed)) gates_exact64(*E, P.s_switch, dt, V, st, gate_mask);
    } else {
-      if (gate_mask & (1u << 12)) dVR = nongate64(*K, P, coef, dt, V, st);
+      if (gate_mask & kMaskNonGate) dVR = nongate64(*K, P, coef, dt, V, st);
       gates64(coef, K->exp_coef, P.s_switch, fl, V, st, gate_mask);
    }
    if (!live) return;
 #pragma unroll
-   for (int s = 0; s < N_STATE; s++) __builtin_nontemporal_store(st[s], sp + kBlk * s);
+   for (int s = 0; s < S_M; s++) __builtin_nontemporal_store(st[s], sp + kBlk * s);
+   if (gate_mask & kMaskGates) {
+#pragma unroll
+      for (int s = S_M; s < N_STATE; s++) __builtin_nontemporal_store(st[s], sp + kBlk * s);
+   }
    dVm[e] = dVR;
 }
 
@@ -133,7 +143,7 @@ __device__ __forceinline__ void calc_split_gates(const ReactionArgs &a, int i, b
       gates64(constant_ptr(a.coef), constant_ptr(a.K)->exp_coef, s_switch, fl, V, st, mask);
    }
    __syncthreads();
-   if (!live) return;
+   if (!live || !mask) return;
 #pragma unroll
    for (int q = S_M; q < N_STATE; q++)
       if ((GATES >> (q - S_M)) & 1) sp[kBlk * q] = st[q];

@@ -40,7 +40,6 @@ struct TT06Reaction {
    DevBuf<ParamSet> params;
    DevBuf<uint8_t> flags;
    DevBuf<double> state;
-   DevBuf<uint8_t> flagsAllFixed;   // gates skipped (updateNonGate-only launches)
 };
 
 }  // namespace cdh
@@ -89,7 +88,7 @@ ReactionArgs reaction_args(cdh_tt06 *r, double dt, const int *index, int n, cons
    a.Vm = Vm;
    a.dVm = dVm;
    a.dt = dt;
-   a.gate_mask = 0x1FFFu;
+   a.gate_mask = kMaskGates | kMaskNonGate;
    a.E = r->exact ? r->Ed.p : nullptr;
    return a;
 }
@@ -194,12 +193,10 @@ int cdh_tt06_create(const cdh_tt06_params *p, int numPoints, cdh_tt06 **out)
       // configuration B reproduces the v2 loops' per-group bounds and f-gate
       // rounding per cell; the generic gate loop of configuration A visits
       // every cell alike
-      std::vector<uint8_t> fl(r->stride, kFlagGatesFixed), fixed(r->stride, kFlagGatesFixed);
+      std::vector<uint8_t> fl(r->stride, kFlagGatesFixed);
       for (int i = 0; i < numPoints; i++) fl[i] = exact ? 0 : gate_flags(i, numPoints);
       r->flags.alloc(r->stride);
       r->flags.upload(fl.data(), fl.size());
-      r->flagsAllFixed.alloc(r->stride);
-      r->flagsAllFixed.upload(fixed.data(), fixed.size());
       // states in 64-cell tiles (state s of cell i at blk_index(s, i, 19)): a
       // wavefront's 19 rows are one contiguous 9.5 KB run
       const std::vector<double> st = rest_state_soa(r->ct, numPoints, r->stride, r->K.c9);
@@ -236,9 +233,10 @@ int cdh_tt06_update_nongate(cdh_tt06 *r, double dt, const int *indexArray, int n
    return guard([&] {
       CDH_REQUIRE(r && Vm && dVR && n == r->n, "cdh_tt06_update_nongate: bad arguments");
       if (n == 0) return;
-      // the calc kernel with every gate held fixed is the non-gate update
-      launch_calc(r, reaction_args(r, dt, indexArray, n, Vm, dVR, r->flagsAllFixed.p),
-                  S(stream));
+      // the calc kernel without its gates is the non-gate update
+      ReactionArgs a = reaction_args(r, dt, indexArray, n, Vm, dVR, r->flags.p);
+      a.gate_mask = kMaskNonGate;
+      launch_calc(r, a, S(stream));
    });
 }
 
